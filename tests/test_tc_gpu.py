@@ -43,3 +43,21 @@ def test_tc_rejects_directed():
     with pytest.raises(gpu.GpuError) as e:
         gpu.tc(gpu.DeviceGraph(g))
     assert e.value.code == -95
+
+
+@pytest.mark.parametrize("lo", [98304 - 40, 98304, 131072 - 20, 262144])
+def test_tc_high_ids(lo):
+    # Long lists whose ids straddle the start of the shared (aliased) bits:
+    # a clique on [lo, lo + 80), and 40 vertices 32768 higher, each joined to
+    # the clique's upper half and to a neighbour, so probes hit aliases of
+    # staged entries that are not neighbours.
+    print(f"[tc] ids from {lo}", flush=True)
+    iu, iv = np.triu_indices(80, 1)
+    far = np.arange(40) + lo + 32768
+    u = np.concatenate([iu + lo, np.repeat(far, 40), far[:-1]])
+    v = np.concatenate([iv + lo, np.tile(np.arange(40, 80) + lo, 40), far[1:]])
+    g = Graph.from_edges(u, v)
+    # clique; far vertex + clique pair; far pair + clique vertex
+    want = math.comb(80, 3) + 40 * math.comb(40, 2) + 39 * 40
+    assert oracle.ordered_count(g)[0] == want
+    assert gpu.OrderedCount(gpu.DeviceGraph(g)) == want
