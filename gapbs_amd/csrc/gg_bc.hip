@@ -23,11 +23,10 @@
 //   * the sigma pull runs one thread per vertex; vertices with >= 256
 //     in-edges are cut into chunks summed by whole blocks and combined with
 //     one double atomic per chunk;
-//   * delta runs one thread per vertex below 64 edges and one wavefront per
-//     vertex above: the wavefront computes 64 successor terms at a time and
-//     folds them into the accumulator in successor order (ballot, then one
-//     lane after another), so every vertex's delta is rounded exactly as the
-//     reference rounds it;
+//   * delta runs one thread per vertex below 64 edges and one wavefront or
+//     block per vertex above: 64 successor terms are computed at a time and
+//     folded into the accumulator as if in successor order (FoldTerms), so
+//     every vertex's delta is rounded exactly as the reference rounds it;
 //   * GG_BC_FP32: the reference's float arithmetic throughout (its verifier
 //     allows only FLT_EPSILON); GG_BC_FP32_KAHAN: float dependencies and
 //     scores, each per-vertex dependency sum and each score sum over roots
@@ -44,7 +43,8 @@ constexpr int kQueueCap = 2048;
 constexpr int kStripes = 64;
 constexpr int64_t kHubEdges = 256;   // sigma pull: vertices with this many in-edges use chunks
 constexpr int64_t kWaveEdges = 64;   // delta: vertices with this many edges use a wavefront
-constexpr int64_t kBcHubEdges = 16384;  // ... and with this many, a block (BcDeltaHub)
+constexpr int kBcWaveUnroll = 4;     // 64-edge runs per wavefront step
+constexpr int64_t kBcHubEdges = 4096;  // ... and with this many, a block (BcDeltaHub)
 constexpr int kBcHubProducers = 15;
 constexpr int kBcHubUnroll = 2;  // 64-edge runs per producer wavefront and round
 constexpr int kBcHubGrid = 2;    // BcDeltaHub blocks per CU
@@ -253,6 +253,78 @@ struct AccFor<float, true> {
   using Type = KahanAcc;
 };
 
+// Inclusive scan within the wavefront by data-parallel moves (no LDS).
+__device__ __forceinline__ int WaveScanDpp(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
+  return v;
+}
+
+__device__ __forceinline__ double ReadLane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Adds the terms of the lanes in m (wave-uniform) to acc (wave-uniform) in
+// lane order, one after another.
+template <class Acc>
+__device__ __forceinline__ void FoldTerms(Acc& acc, double term, uint64_t m) {
+  while (m) {
+    const int j = __builtin_ctzll(m);
+    acc.Add(ReadLane(term, j));
+    m &= m - 1;
+  }
+}
+
+// The same sum, bit for bit, without the chain of widen / add / round per
+// term.  While the total stays in one binade [2^E, 2^(E+1)) every rounding
+// is to the same grid g = 2^(E-23), on which the total already lies, so
+// adding t moves it by t rounded to the grid, whatever the total: the terms
+// become whole numbers of grid steps and add up in any order.  That fails
+// only for a term within 2^-30 g of a grid midpoint (there the rounding to
+// double before the one to float, or the tie rule, decides) or once the
+// binade is left, so a lane takes part when its term is at least 2^-28 g
+// from a midpoint and every lane before it (inclusive scan) stays below
+// 2^24 steps; the first lane that does not is added the reference's way and
+// the rest tried again with the new binade.  Terms are not negative; NaN and
+// infinities compare false and go the reference's way.  A hub's total
+// crosses a binade only as often as it doubles.  Measured on Kronecker 22,
+// 4 roots: the wavefront kernel 8.7 to 3.9 ms,
+// the hub kernel 10.5 to 6.5 ms with hubs from 4096 instead of 16384
+// successors.
+template <>
+__device__ __forceinline__ void FoldTerms(RefAcc<float>& acc, double term, uint64_t m) {
+  const int lane = LaneId();
+  constexpr int kSteps = 1 << 24;
+  while (m) {
+    const uint32_t bits = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(__float_as_int(acc.v)));
+    const uint32_t e = bits >> 23;  // the sign is 0
+    if (e != 0 && e < 255) {
+      const double x = term * __hiloint2double(static_cast<int>(1023 + 150 - e) << 20, 0);  // exact: / g
+      const double r = rint(x);
+      const bool whole = fabs(x - r) < 0.5 - 0x1p-28 && r < 0x1p24;
+      const bool in = (m >> lane) & 1;
+      const int sum = WaveScanDpp(in ? (whole ? static_cast<int>(r) : kSteps) : 0);
+      const int start = static_cast<int>((bits & 0x7FFFFF) | 0x800000);
+      const uint64_t past = __ballot(in && start + sum >= kSteps);
+      const uint64_t take = past ? m & ((past & -past) - 1) : m;
+      if (take) {
+        const int last = 63 - __builtin_clzll(take);
+        const uint32_t steps = static_cast<uint32_t>(start + __builtin_amdgcn_readlane(sum, last));
+        acc.v = __uint_as_float((e << 23) | (steps & 0x7FFFFF));
+        m &= ~take;
+      }
+      if (!m) break;
+    }
+    acc.Add(ReadLane(term, __builtin_ctzll(m)));
+    m &= m - 1;
+  }
+}
+
 // score += delta: plain, or with a Kahan compensation term (float only).
 template <bool kKahan>
 __device__ __forceinline__ void AddScore(float* score, float* comp, int32_t u, float d) {
@@ -335,23 +407,22 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
     const int64_t b = off[u], e = off[u + 1];
     const double su = sigma[u];
     typename AccFor<T, kKahan>::Type acc = AccFor<T, kKahan>::Type::Zero();
-    for (int64_t base = b; base < e; base += kWave) {
-      const int64_t k = base + lane;
-      double term = 0.0;
-      bool has = false;
-      if (k < e) {
-        const int32_t v = dst[k];
-        if (depth[v] == level + 1) {
-          term = DeltaTerm(su, sigma[v], delta[v]);
-          has = true;
-        }
-      }
-      uint64_t m = __ballot(has);
-      if (lane == 0) mat += static_cast<unsigned long long>(__popcll(m));
-      while (m) {
-        const int j = __ffsll(static_cast<unsigned long long>(m)) - 1;
-        acc.Add(__shfl(term, j));
-        m &= m - 1;
+    for (int64_t base = b; base < e; base += kWave * kBcWaveUnroll) {
+      // kBcWaveUnroll runs of 64 edges, their loads issued together.
+      int32_t v[kBcWaveUnroll];
+      bool has[kBcWaveUnroll];
+      double term[kBcWaveUnroll];
+#pragma unroll
+      for (int r = 0; r < kBcWaveUnroll; r++) v[r] = base + r * kWave + lane < e ? dst[base + r * kWave + lane] : -1;
+#pragma unroll
+      for (int r = 0; r < kBcWaveUnroll; r++) has[r] = v[r] >= 0 && depth[v[r]] == level + 1;
+#pragma unroll
+      for (int r = 0; r < kBcWaveUnroll; r++) term[r] = has[r] ? DeltaTerm(su, sigma[v[r]], delta[v[r]]) : 0.0;
+#pragma unroll
+      for (int r = 0; r < kBcWaveUnroll; r++) {
+        const uint64_t m = __ballot(has[r]);
+        if (lane == 0) mat += static_cast<unsigned long long>(__popcll(m));
+        FoldTerms(acc, term[r], m);
       }
     }
     if (lane == 0) {
@@ -369,14 +440,10 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
 // consecutive edges (from b + 64 kBcHubUnroll (round kBcHubProducers + p))
 // and packs the matched ones, in edge order, into one half of an LDS double
 // buffer; the last wavefront folds the previous round's terms in edge
-// order.  Same terms, same order, same arithmetic as BcDeltaWave; only the
-// loads and divisions run in parallel.  The fold (widen, add in double,
-// round to float per term, as the reference's float `+=` of a double term)
-// is a chain of three dependent double-precision operations per matched
-// edge, so the largest hubs set the kernel's time.  Blocks take hubs from
-// a counter, so a block held by a large hub takes no others meanwhile (the
-// list follows the level's queue, which on a degree-ordered layout runs
-// roughly from the largest hub down).
+// order (FoldTerms).  Same terms, same order, same arithmetic as
+// BcDeltaWave.  Blocks take hubs from a counter, so a block held by a large
+// hub takes no others meanwhile (the list follows the level's queue, which
+// on a degree-ordered layout runs roughly from the largest hub down).
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict__ off,
                                                        const int32_t* __restrict__ dst,
@@ -436,15 +503,10 @@ __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict
         const int h = (k - 1) & 1;
         for (int p = 0; p < kBcHubProducers; p++) {
           const int cnt = counts[h][p];
-          int j = 0;
-          for (; j + 8 <= cnt; j += 8) {  // eight LDS reads in flight, then the ordered fold
-            double t[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) t[q] = terms[h][p][j + q];
-#pragma unroll
-            for (int q = 0; q < 8; q++) acc.Add(t[q]);
+          for (int j = 0; j < cnt; j += kWave) {
+            const double t = j + lane < cnt ? terms[h][p][j + lane] : 0.0;
+            FoldTerms(acc, t, cnt - j >= kWave ? ~uint64_t(0) : (uint64_t(1) << (cnt - j)) - 1);
           }
-          for (; j < cnt; j++) acc.Add(terms[h][p][j]);
         }
       }
       __syncthreads();

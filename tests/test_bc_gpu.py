@@ -109,3 +109,26 @@ def test_bc_deep_graph_uses_level_by_level_discovery():
     dg = gpu.DeviceGraph(g)
     roots = np.array([0, 2500, 4999], dtype=np.int32)
     assert np.array_equal(gpu.bc(dg, roots).scores, oracle.brandes(g, roots))
+
+
+@pytest.mark.parametrize("leaves", [70, 2500, 9000])
+def test_bc_folds_ties_and_binades(leaves):
+    # One vertex whose total passes many powers of two through terms of 1
+    # and 2 (its leaves, some with a child of their own) interleaved with
+    # terms of exactly 2^-10, which fall on rounding ties once the total is
+    # 2^13: the fold must round each as the reference's one-by-one sum does,
+    # on the thread, wavefront and block paths.
+    print(f"[bc] ties, {leaves} leaves", flush=True)
+    mids, apex = 1024, 200
+    ids = np.random.default_rng(leaves).permutation(np.arange(1 + mids, 1 + mids + leaves + apex))
+    leaf, top = ids[:leaves], ids[leaves:]
+    child = np.arange(leaves // 2) + ids.max() + 1
+    u = np.concatenate([np.zeros(mids, int), np.ones(leaves, int), np.repeat(np.arange(1, 1 + mids), apex),
+                        leaf[:leaves // 2]])
+    v = np.concatenate([np.arange(1, 1 + mids), leaf, np.tile(top, mids), child])
+    g = Graph.from_edges(u, v)
+    roots = np.array([0, 2, int(leaf[0])], dtype=np.int32)
+    want = oracle.brandes(g, roots)
+    dg = gpu.DeviceGraph(g)
+    assert np.array_equal(gpu.bc(dg, roots).scores, want)
+    assert np.array_equal(gpu.bc_batch(dg, roots).scores, want)
