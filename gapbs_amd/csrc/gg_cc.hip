@@ -8,7 +8,9 @@
 //     ends labelled with its smallest vertex id -- the result is exactly the
 //     reference's, not just the same partition;
 //   * neighbor_rounds sampled rounds (default 2): each vertex links to its
-//     r-th neighbour, then Compress (cc.cc:104-117);
+//     r-th neighbour, then Compress (cc.cc:104-117); round 0 hooks vertices
+//     whose first neighbour is smaller as it initialises the labels, and
+//     leaves the other first neighbours to the next round's links;
 //   * the most frequent label among 1024 samples drawn with a default-seeded
 //     std::mt19937 and std::uniform_int_distribution over [0, N-1]
 //     (cc.cc:69-92) names the component whose vertices skip the final link;
@@ -95,12 +97,37 @@ __global__ __launch_bounds__(kBS) void CcInit(int32_t* __restrict__ comp, int64_
     comp[i] = static_cast<int32_t>(i);
 }
 
-// Sampled round r: link u with its r-th out-neighbour, if it has one.
+// Labels before any link: a vertex whose first out-neighbour is smaller starts
+// hooked under it (labels only ever point to smaller ids of the same
+// component, so any such start is as good as the identity).  Round 0's Link
+// calls would do the same through compare-and-swaps and retries on labels
+// that the whole chip was rewriting: 717 us on Kronecker 22 against 24 us.
+__global__ __launch_bounds__(kBS) void CcHook(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
+                                              int32_t* __restrict__ comp, int64_t n) {
+  for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBS) {
+    const int32_t u = static_cast<int32_t>(i);
+    const int64_t b = off[i];
+    const int32_t v = off[i + 1] > b ? dst[b] : u;
+    comp[i] = v < u ? v : u;
+  }
+}
+
+// Sampled round r: link u with its r-th out-neighbour, if it has one; with
+// `first`, also with its first where CcHook did not hook it.  Two launches:
+// the first takes one wavefront's vertices in kLinkSample (`sample`), the
+// second the others.  The trees that most vertices belong to are then merged
+// by few threads, and the rest find their labels joined instead of queueing
+// compare-and-swaps on the same roots (Kronecker 22: 325 us in one launch,
+// 156 us in two).
+constexpr int kLinkSample = 64;
 __global__ __launch_bounds__(kBS) void CcLinkRound(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
-                                                   int32_t* comp, int64_t n, int r) {
-  for (int64_t u = blockIdx.x * int64_t(kBS) + threadIdx.x; u < n; u += int64_t(gridDim.x) * kBS) {
-    const int64_t b = off[u];
-    if (off[u + 1] - b > r) Link(static_cast<int32_t>(u), dst[b + r], comp);
+                                                   int32_t* comp, int64_t n, int r, bool first, bool sample) {
+  for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBS) {
+    if ((i / kWave % kLinkSample == 0) != sample) continue;  // wavefront-uniform
+    const int32_t u = static_cast<int32_t>(i);
+    const int64_t b = off[i], e = off[i + 1];
+    if (first && e > b && dst[b] > u) Link(u, dst[b], comp);
+    if (r > 0 && e - b > r) Link(u, dst[b + r], comp);
   }
 }
 
@@ -275,14 +302,29 @@ int64_t RunAfforest(gg_graph* g, int neighbor_rounds, const CcBuffers& b, int32_
   const double N = static_cast<double>(n);
   int64_t launches = 0;
   hipLaunchKernelGGL(CcClear, dim3(1), dim3(64), 0, st, b.examined, b.nchunks);
-  Run(g, "cc_init", 4 * N, CcInit, grid_n, blk, b.comp, n);
-  launches += 2;
-  for (int r = 0; r < neighbor_rounds; r++) {
-    // offsets 16 B (both ends), the r-th neighbour, comp read/write.
-    Run(g, "cc_link_round", 16 * N + 4 * N + 8 * N, CcLinkRound, grid_n, blk,
-        static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), b.comp, n, r);
+  auto compress = [&] {
     Run(g, "cc_compress", 8 * N, CcCompress, grid_n, blk, b.comp, n);
-    launches += 2;
+    launches++;
+  };
+  launches += 2;
+  if (neighbor_rounds == 0) {
+    Run(g, "cc_init", 4 * N, CcInit, grid_n, blk, b.comp, n);
+  } else {
+    // Round 0 is CcHook; the first neighbours it left are linked with the
+    // next round's, once the labels are compressed.  Offsets, the first
+    // neighbour, comp.
+    Run(g, "cc_hook", 16 * N, CcHook, grid_n, blk, static_cast<const int64_t*>(g->out_off),
+        static_cast<const int32_t*>(g->out_dst), b.comp, n);
+    compress();
+    for (int r = neighbor_rounds == 1 ? 0 : 1; r < neighbor_rounds; r++) {
+      // offsets 16 B (both ends), the r-th neighbour, comp read/write.
+      for (const bool sample : {true, false})
+        Run(g, "cc_link_round", sample ? 0 : 16 * N + 4 * N + 8 * N, CcLinkRound, grid_n, blk,
+            static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), b.comp, n, r, r <= 1,
+            sample);
+      launches += 2;
+      compress();
+    }
   }
   CcGather<<<dim3(kSamples / kBS), blk, 0, st>>>(b.comp, b.sample_idx, b.sample_val, kSamples);
   GG_HIP(hipMemcpyAsync(h_samples, b.sample_val, sizeof(int32_t) * kSamples, hipMemcpyDeviceToHost, st));
@@ -303,8 +345,7 @@ int64_t RunAfforest(gg_graph* g, int neighbor_rounds, const CcBuffers& b, int32_
   };
   final_link(g->out_off, g->out_dst, neighbor_rounds);
   if (g->directed) final_link(g->in_off, g->in_dst, 0);
-  Run(g, "cc_compress", 8 * N, CcCompress, grid_n, blk, b.comp, n);
-  launches++;
+  compress();
   GG_HIP(hipGetLastError());
   return launches;
 }

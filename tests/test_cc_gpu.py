@@ -88,3 +88,21 @@ def test_sv_directed_grid_hub_and_ordered():
     assert np.array_equal(gpu.cc_sv(gpu.DeviceGraph(h)).comp, oracle.cc_min_labels(h))
     k = cached_graph("g16", lambda: Graph.kronecker(16))
     assert np.array_equal(gpu.cc_sv(gpu.DeviceGraph(k, order_by_degree=True)).comp, oracle.cc_min_labels(k))
+
+
+@pytest.mark.parametrize("rounds", [0, 1, 2, 3])
+@pytest.mark.parametrize("directed", [False, True])
+def test_cc_rounds_and_first_neighbours(rounds, directed):
+    # First neighbours that are larger (local minima, linked after the first
+    # labels), smaller (hooked at once) and missing; chains in both id
+    # directions; a last wavefront that is not full.
+    print(f"[cc] rounds {rounds} directed {directed}", flush=True)
+    rng = np.random.default_rng(rounds)
+    n = 64 * 300 + 17
+    u, v = rng.integers(0, n // 2, 9000), rng.integers(0, n // 2, 9000)
+    chain = np.arange(n // 2, n - 200)
+    u = np.concatenate([u, chain[:3000], chain[3001:6000], [n - 1]])
+    v = np.concatenate([v, chain[1:3001], chain[3000:5999], [n - 1]])
+    g = Graph.from_edges(u, v, symmetrize=not directed)
+    want = oracle.cc_min_labels(g)
+    assert np.array_equal(gpu.cc(gpu.DeviceGraph(g), neighbor_rounds=rounds).comp, want)
