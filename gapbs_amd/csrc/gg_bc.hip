@@ -91,22 +91,26 @@ struct DiscoverVisit {
   LdsQueue<kQueueCap>* lq;
   int32_t* queue;
   int32_t* tail;
-  __device__ __forceinline__ void operator()(int32_t, int32_t, int64_t e, bool valid) {
-    bool won = false;
-    int32_t v = 0;
-    if (valid) {
-      v = dst[e];
-      won = Load(&depth[v]) == -1 && atomicCAS(&depth[v], -1, next_depth) == -1;
-    }
-    LdsQueuePush(*lq, won, v, queue, tail);
+  __device__ __forceinline__ void Visit(const int32_t (&)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t v[kExpandEdges];
+    bool won[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) v[k] = dst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) won[k] = Load(&depth[v[k]]) == -1;
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++)
+      won[k] = valid[k] && won[k] && atomicCAS(&depth[v[k]], -1, next_depth) == -1;
+    LdsQueuePushMany(*lq, won, v, queue, tail);
   }
+  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, queue, tail); }
 };
 
 // Claims the next level's vertices and appends them to the queue.
 __global__ __launch_bounds__(kBS) void BcDiscover(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
                                                   int32_t* depth, int32_t* queue, int32_t qb, int32_t qn,
-                                                  int32_t next_depth, BcCounters* c, EdgeChunk* chunks,
-                                                  int64_t chunk_min) {
+                                                  int32_t next_depth, BcCounters* c, EdgeChunk* chunks) {
   __shared__ ExpandShared sh;
   __shared__ LdsQueue<kQueueCap> lq;
   __shared__ unsigned long long s_red[kBS / kWave];
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(kBS) void BcDiscover(const int64_t* __restrict__ of
       end = off[u + 1];
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile(sh, 0, 0, beg, end, visit, chunks, &c->nchunks, chunk_min);
+    ExpandTile<FrontierCut>(sh, 0, 0, beg, end, visit, chunks, &c->nchunks);
   }
   LdsQueueFlush(lq, queue, &c->tail);
   ex = BlockSum<kBS>(ex, s_red);
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(kBS) void BcDiscoverChunks(const int32_t* __restric
   __shared__ LdsQueue<kQueueCap> lq;
   LdsQueueInit(lq);
   DiscoverVisit visit{dst, depth, next_depth, &lq, queue, &c->tail};
-  ExpandChunks(chunks, c->nchunks, visit);
+  ExpandChunks<FrontierCut>(chunks, c->nchunks, visit);
   LdsQueueFlush(lq, queue, &c->tail);
 }
 
@@ -680,8 +684,8 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   int32_t* lvl_cursor = g->Scratch<int32_t>("bc.level_cursor", kBucketLevels);
   std::vector<int32_t> h_counts(kBucketLevels);
   const int64_t entries = g->out_entries > g->in_entries ? g->out_entries : g->in_entries;
-  EdgeChunk* chunks = g->Scratch<EdgeChunk>("bc.chunks", MaxChunks(n, entries));
-  EdgeChunk* rchunks = g->Scratch<EdgeChunk>("bc.rchunks", MaxChunks(n, entries));
+  EdgeChunk* chunks = g->Scratch<EdgeChunk>("bc.chunks", FrontierCut::Bound(n, entries));
+  EdgeChunk* rchunks = g->Scratch<EdgeChunk>("bc.rchunks", entries / kChunkEdges + entries / kHubEdges + 2);
   const bool hubs = g->max_degree >= kHubEdges;
   const dim3 blk(kBS);
   const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
@@ -752,11 +756,10 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     }
     while (!bucketed) {
       const int32_t qb = bounds[bounds.size() - 2], qn = bounds.back() - qb;
-      const int64_t chunk_min = qn <= 4096 ? kExpandBS : kChunkEdges;
       const int idx = Run(g, "bc_discover", 8.0 * qn, BcDiscover, dim3(GridFor(qn, kBS, g->cu_count * 8)), blk,
                           static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst),
                           depth, queue, qb, qn, level + 1, dc,
-                          hubs ? chunks : static_cast<EdgeChunk*>(nullptr), chunk_min);
+                          hubs ? chunks : static_cast<EdgeChunk*>(nullptr));
       launches++;
       if (hubs) {
         Run(g, "bc_discover_chunks", 0, BcDiscoverChunks, grid_c, blk, static_cast<const int32_t*>(g->out_dst),

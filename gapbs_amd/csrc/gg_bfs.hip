@@ -15,9 +15,9 @@
 //   * the final fix-up parent < -1 -> -1 (bfs.cc:174-177).
 // What is GPU-specific:
 //   * top-down expands 256-vertex tiles of the frontier with gg_expand.h
-//     (hubs cut into chunks spread over the grid; when the frontier is small
-//     every vertex with >= 256 edges is chunked); discovered vertices are
-//     staged in an LDS queue and flushed with one atomic per block;
+//     (vertices with many edges cut into chunks spread over the grid);
+//     discovered vertices are staged in an LDS queue and flushed with one
+//     atomic per block;
 //   * bottom-up gives each wavefront 64 consecutive vertices, so the next
 //     frontier word is one ballot, written without atomics; a visited bitmap
 //     (with vertices that have no in-neighbours pre-set) lets whole words be
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kBS) void BfsInit(const int64_t* __restrict__ off,
   }
 }
 
-// One frontier edge u -> dst[e] (valid lanes only act; all lanes of a
+// Frontier edges u[k] -> dst[e[k]] (valid ones only act; all lanes of a
 // wavefront call together).  Winners of the parent CAS join the next queue.
 struct TdVisit {
   const int32_t* dst;
@@ -147,23 +147,29 @@ struct TdVisit {
   int32_t level;
   unsigned long long scout = 0, reach = 0;
 
-  __device__ __forceinline__ void operator()(int32_t u, int32_t, int64_t e, bool valid) {
-    bool won = false;
-    int32_t cur = 0, v = 0;
-    if (valid) {
-      v = dst[e];
-      cur = parent[v];
-      if (cur < 0) won = atomicCAS(&parent[v], cur, u) == cur;
-    }
-    if (won) {
-      if (depth) depth[v] = level;
-      scout += static_cast<unsigned long long>(-static_cast<int64_t>(cur));
+  __device__ __forceinline__ void Visit(const int32_t (&u)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t v[kExpandEdges], cur[kExpandEdges];
+    bool won[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) v[k] = dst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) cur[k] = parent[v[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++)
+      won[k] = valid[k] && cur[k] < 0 && atomicCAS(&parent[v[k]], cur[k], u[k]) == cur[k];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      if (!won[k]) continue;
+      if (depth) depth[v[k]] = level;
+      scout += static_cast<unsigned long long>(-static_cast<int64_t>(cur[k]));
       // -1 encodes both degree 0 and degree 1; read the degree for those.
-      reach += cur < -1 ? static_cast<unsigned long long>(-static_cast<int64_t>(cur))
-                        : static_cast<unsigned long long>(off[v + 1] - off[v]);
+      reach += cur[k] < -1 ? static_cast<unsigned long long>(-static_cast<int64_t>(cur[k]))
+                           : static_cast<unsigned long long>(off[v[k] + 1] - off[v[k]]);
     }
-    LdsQueuePush(*lq, won, v, qout, qtail);
+    LdsQueuePushMany(*lq, won, v, qout, qtail);
   }
+  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, qout, qtail); }
 };
 
 __device__ __forceinline__ void FlushTdCounters(const TdVisit& visit, unsigned long long examined,
@@ -184,7 +190,7 @@ __global__ __launch_bounds__(kBS) void BfsTopDown(const int64_t* __restrict__ of
                                                   int32_t* __restrict__ parent, int32_t* __restrict__ depth,
                                                   const int32_t* __restrict__ qin, int32_t qn,
                                                   int32_t* __restrict__ qout, BfsCounters* c, int32_t level,
-                                                  EdgeChunk* chunks, int64_t chunk_min) {
+                                                  EdgeChunk* chunks) {
   __shared__ ExpandShared sh;
   __shared__ LdsQueue<kQueueCap> lq;
   __shared__ unsigned long long s_red[kBS / kWave];
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(kBS) void BfsTopDown(const int64_t* __restrict__ of
       end = off[u + 1];
       examined += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile(sh, u, 0, beg, end, visit, chunks, &c->nchunks, chunk_min);
+    ExpandTile<FrontierCut>(sh, u, 0, beg, end, visit, chunks, &c->nchunks);
   }
   LdsQueueFlush(lq, qout, &c->qtail);
   FlushTdCounters(visit, examined, c, s_red);
@@ -218,7 +224,7 @@ __global__ __launch_bounds__(kBS) void BfsTopDownChunks(const int64_t* __restric
   __shared__ unsigned long long s_red[kBS / kWave];
   LdsQueueInit(lq);
   TdVisit visit{dst, parent, depth, off, &lq, qout, &c->qtail, level};
-  ExpandChunks(chunks, c->nchunks, visit);
+  ExpandChunks<FrontierCut>(chunks, c->nchunks, visit);
   LdsQueueFlush(lq, qout, &c->qtail);
   FlushTdCounters(visit, 0, c, s_red);
 }
@@ -417,9 +423,9 @@ BfsRun RunDobfs(gg_graph* g, int32_t source, int alpha, int beta, int32_t* depth
   uint64_t* next = g->Scratch<uint64_t>("bfs.next", nwords);
   uint64_t* visited = g->Scratch<uint64_t>("bfs.visited", nwords);
   BfsCounters* dc = g->Scratch<BfsCounters>("bfs.ctr", 1);
-  const bool use_chunks = g->max_degree >= kExpandBS;
+  const bool use_chunks = g->max_degree >= FrontierCut::kMin;
   EdgeChunk* chunks =
-      use_chunks ? g->Scratch<EdgeChunk>("bfs.chunks", MaxChunks(n, g->out_entries)) : nullptr;
+      use_chunks ? g->Scratch<EdgeChunk>("bfs.chunks", FrontierCut::Bound(n, g->out_entries)) : nullptr;
 
   const dim3 blk(kBS);
   const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
@@ -492,17 +498,14 @@ BfsRun RunDobfs(gg_graph* g, int32_t source, int alpha, int beta, int32_t* depth
       scout = 1;
     } else {
       edges_to_check -= scout;
-      const bool hubs = use_chunks && frontier_deg >= kExpandBS;
-      // A small frontier gets every vertex with >= 256 edges chunked across
-      // the grid; a large one only the real hubs.
-      const int64_t chunk_min = qsize <= 4096 ? kExpandBS : kChunkEdges;
+      const bool hubs = use_chunks && frontier_deg >= FrontierCut::kMin;
       const int idx = Run(g, "bfs_top_down", 16.0 * qsize, BfsTopDown,
                           dim3(GridFor(qsize, kBS, g->cu_count * 8)), blk, g->out_off, g->out_dst,
                           parent, depth, qin, static_cast<int32_t>(qsize), qout, dc, level,
-                          hubs ? chunks : static_cast<EdgeChunk*>(nullptr), chunk_min);
+                          hubs ? chunks : static_cast<EdgeChunk*>(nullptr));
       launches++;
       if (hubs) {
-        const dim3 grid_c(GridFor(frontier_deg / kExpandBS + kChunkSlices, 1, g->cu_count * 8));
+        const dim3 grid_c(GridFor(frontier_deg / FrontierCut::kMin + 1, 1, g->cu_count * 8));
         Run(g, "bfs_top_down_chunks", 0, BfsTopDownChunks, grid_c, blk, g->out_off, g->out_dst,
             parent, depth, qout, dc, level, static_cast<const EdgeChunk*>(chunks));
         launches++;

@@ -152,9 +152,16 @@ __global__ __launch_bounds__(kBS) void CcGather(const int32_t* __restrict__ comp
 struct LinkVisit {
   const int32_t* dst;
   int32_t* comp;
-  __device__ __forceinline__ void operator()(int32_t u, int32_t, int64_t e, bool valid) {
-    if (valid) Link(u, dst[e], comp);
+  __device__ __forceinline__ void Visit(const int32_t (&u)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t v[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) v[k] = dst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++)
+      if (valid[k]) Link(u[k], v[k], comp);
   }
+  __device__ __forceinline__ void StepEnd() {}
 };
 
 // Final link: every vertex outside the skipped component links with its
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(kBS) void CcFinalLink(const int64_t* __restrict__ o
       beg = off[u] + start < end ? off[u] + start : end;
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, kChunkEdges);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks);
   }
   ex = BlockSum<kBS>(ex, s_red);
   if (threadIdx.x == 0 && ex) atomicAdd(&examined[blockIdx.x & 63], ex);
@@ -184,10 +191,10 @@ __global__ __launch_bounds__(kBS) void CcFinalLink(const int64_t* __restrict__ o
 __global__ __launch_bounds__(kBS) void CcFinalLinkChunks(const int32_t* __restrict__ dst, int32_t* comp,
                                                          const EdgeChunk* chunks, const int32_t* nchunks) {
   LinkVisit visit{dst, comp};
-  ExpandChunks(chunks, *nchunks, visit);
+  ExpandChunks<WholeCut>(chunks, *nchunks, visit);
 }
 
-// Shiloach-Vishkin's hook (src/cc_sv.cc:58-71): over edge (u, v), the higher
+// Shiloach-Vishkin's hook (src/cc_sv.cc:58-71): over each edge (u, v), the higher
 // of the two labels, while it is still a root, takes the lower one -- the
 // min-max swap that makes lower labels win whatever the edge's direction.
 // An agent-scope store where the reference has a plain one (see Load);
@@ -196,17 +203,28 @@ struct HookVisit {
   const int32_t* dst;
   int32_t* comp;
   bool* hooked;
-  __device__ __forceinline__ void operator()(int32_t u, int32_t, int64_t e, bool valid) {
-    if (!valid) return;
-    const int32_t cu = Load(&comp[u]), cv = Load(&comp[dst[e]]);
-    if (cu == cv) return;
-    const int32_t high = cu > cv ? cu : cv;
-    const int32_t low = cu + (cv - high);
-    if (Load(&comp[high]) == high) {
-      Store(&comp[high], low);
-      *hooked = true;
+  __device__ __forceinline__ void Visit(const int32_t (&u)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t v[kExpandEdges], cu[kExpandEdges], cv[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) v[k] = dst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      cv[k] = Load(&comp[v[k]]);
+      cu[k] = valid[k] ? Load(&comp[u[k]]) : cv[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      if (cu[k] == cv[k]) continue;
+      const int32_t high = cu[k] > cv[k] ? cu[k] : cv[k];
+      const int32_t low = cu[k] + (cv[k] - high);
+      if (Load(&comp[high]) == high) {
+        Store(&comp[high], low);
+        *hooked = true;
+      }
     }
   }
+  __device__ __forceinline__ void StepEnd() {}
 };
 
 // One wavefront store per wavefront that hooked.
@@ -223,7 +241,7 @@ __global__ __launch_bounds__(kBS) void SvHook(const int64_t* __restrict__ off, c
   for (int64_t tile = int64_t(blockIdx.x) * kBS; tile < n; tile += int64_t(gridDim.x) * kBS) {
     const int64_t u = tile + threadIdx.x;
     const int64_t beg = u < n ? off[u] : 0, end = u < n ? off[u + 1] : 0;
-    ExpandTile(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, kChunkEdges);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks);
   }
   NoteChange(hooked, change);
 }
@@ -232,7 +250,7 @@ __global__ __launch_bounds__(kBS) void SvHookChunks(const int32_t* __restrict__ 
                                                     const EdgeChunk* chunks, const int32_t* nchunks, int* change) {
   bool hooked = false;
   HookVisit visit{dst, comp, &hooked};
-  ExpandChunks(chunks, *nchunks, visit);
+  ExpandChunks<WholeCut>(chunks, *nchunks, visit);
   NoteChange(hooked, change);
 }
 
@@ -288,7 +306,7 @@ struct CcBuffers {
   int32_t* sample_val;           // kSamples
   unsigned long long* examined;  // 64 striped counters
   int32_t* nchunks;              // 1
-  EdgeChunk* chunks;             // MaxChunks(n, entries), or null when no vertex reaches kChunkEdges
+  EdgeChunk* chunks;             // WholeCut::Bound(n, entries), or null when no vertex reaches WholeCut::kMin
 };
 
 // Afforest (cc.cc:95-151) on g->stream into b.comp, inside the caller's
@@ -377,7 +395,7 @@ extern "C" int gg_cc(gg_graph* g, int neighbor_rounds, int32_t* comp_out, gg_sta
     b.sample_val = g->Scratch<int32_t>("cc.sample_val", kSamples);
     b.examined = g->Scratch<unsigned long long>("cc.examined", 64);
     b.nchunks = g->Scratch<int32_t>("cc.nchunks", 2);
-    b.chunks = g->max_degree >= kChunkEdges ? g->Scratch<EdgeChunk>("cc.chunks", MaxChunks(n, CcEntries(g)))
+    b.chunks = g->max_degree >= WholeCut::kMin ? g->Scratch<EdgeChunk>("cc.chunks", WholeCut::Bound(n, CcEntries(g)))
                                             : nullptr;
     int32_t* h_samples = g->Pinned<int32_t>(kSamples);
     if (g->cc_samples_n != n) {  // sample positions depend only on n
@@ -422,7 +440,7 @@ extern "C" int gg_cc_noalloc(gg_graph* g, int neighbor_rounds, int32_t* comp_out
     }
     GG_REQUIRE(base != nullptr, GG_ENODEV, "gg_init has not been called for this graph's device");
     const int64_t n = g->n;
-    const bool use_chunks = g->max_degree >= kChunkEdges;
+    const bool use_chunks = g->max_degree >= WholeCut::kMin;
     size_t used = 0;
     auto carve = [&](size_t bytes) {
       const size_t at = used;
@@ -434,7 +452,9 @@ extern "C" int gg_cc_noalloc(gg_graph* g, int neighbor_rounds, int32_t* comp_out
     const size_t at_val = carve(sizeof(int32_t) * kSamples);
     const size_t at_ex = carve(sizeof(unsigned long long) * 64);
     const size_t at_nc = carve(sizeof(int32_t) * 2);
-    const size_t at_chunks = use_chunks ? carve(sizeof(EdgeChunk) * MaxChunks(n, CcEntries(g))) : 0;
+    // (room for more chunks than WholeCut makes: which graphs fit the scratch
+    // array is not to change with the cut)
+    const size_t at_chunks = use_chunks ? carve(sizeof(EdgeChunk) * ChunkCut<256, 4096>::Bound(n, CcEntries(g))) : 0;
     const size_t at_least = g->new_id ? carve(sizeof(int32_t) * n) : 0;
     const size_t at_out = g->new_id ? carve(sizeof(int32_t) * n) : 0;
     GG_REQUIRE(used <= kNoAllocBytes, GG_EINVAL,
@@ -491,8 +511,8 @@ extern "C" int gg_cc_sv(gg_graph* g, int32_t* comp_out, gg_stats* stats) {
     int32_t* comp = g->Scratch<int32_t>("cc.comp", n);
     int32_t* nchunks = g->Scratch<int32_t>("cc.nchunks", 2);
     int* change = g->Scratch<int>("sv.change", 1);
-    const bool use_chunks = g->max_degree >= kChunkEdges;
-    EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("cc.chunks", MaxChunks(n, g->out_entries)) : nullptr;
+    const bool use_chunks = g->max_degree >= WholeCut::kMin;
+    EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("cc.chunks", WholeCut::Bound(n, g->out_entries)) : nullptr;
     int* h_change = g->Pinned<int>(1);
     int64_t iterations = 0, launches = 0;
     BeginTiming(g);

@@ -310,21 +310,27 @@ struct TdVisit {
   LdsQueue<kQueueCap>* lq;
   int32_t* touched;
   int32_t* touched_tail;
-  __device__ __forceinline__ void operator()(int32_t v, int32_t, int64_t e, bool valid) {
-    bool first = false;
-    int32_t w = 0;
-    if (valid) {
-      w = dst[e];
-      const uint64_t bits = frontier[v] & ~seen[w];
+  __device__ __forceinline__ void Visit(const int32_t (&v)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t w[kExpandEdges];
+    uint64_t bits[kExpandEdges], have[kExpandEdges];
+    bool first[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) w[k] = dst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      bits[k] = (valid[k] ? frontier[v[k]] : 0) & ~seen[w[k]];
       // acc[w] only gains bits during the level, so a plain (possibly
       // stale) read that already holds them makes the atomic redundant.
-      if (bits && (bits & ~acc[w])) {
-        const uint64_t old = atomicOr(reinterpret_cast<unsigned long long*>(&acc[w]), bits);
-        first = old == 0;
-      }
+      have[k] = acc[w[k]];
     }
-    LdsQueuePush(*lq, first, w, touched, touched_tail);
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++)
+      first[k] = (bits[k] & ~have[k]) &&
+                 atomicOr(reinterpret_cast<unsigned long long*>(&acc[w[k]]), bits[k]) == 0;
+    LdsQueuePushMany(*lq, first, w, touched, touched_tail);
   }
+  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, touched, touched_tail); }
 };
 
 __global__ __launch_bounds__(kBS) void MsTopDown(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
@@ -334,9 +340,6 @@ __global__ __launch_bounds__(kBS) void MsTopDown(const int64_t* __restrict__ off
                                                  int32_t* touched, MsCounters* c, EdgeChunk* chunks) {
   if (L->done || L->bottom_up) return;
   const int64_t na = L->na;
-  // A small frontier gets every vertex with >= kExpandBS edges chunked
-  // across the grid; a large one only the real hubs.
-  const int64_t chunk_min = na <= 4096 ? kExpandBS : kChunkEdges;
   __shared__ ExpandShared sh;
   __shared__ LdsQueue<kQueueCap> lq;
   __shared__ unsigned long long s_red[kBS / kWave];
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(kBS) void MsTopDown(const int64_t* __restrict__ off
       end = off[v + 1];
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile(sh, v, 0, beg, end, visit, chunks, &c->nchunks, chunk_min);
+    ExpandTile<FrontierCut>(sh, v, 0, beg, end, visit, chunks, &c->nchunks);
   }
   LdsQueueFlush(lq, touched, &c->touched_tail);
   ex = BlockSum<kBS>(ex, s_red);
@@ -369,7 +372,7 @@ __global__ __launch_bounds__(kBS) void MsTopDownChunks(const int32_t* __restrict
   __shared__ LdsQueue<kQueueCap> lq;
   LdsQueueInit(lq);
   TdVisit visit{dst, frontier, seen, acc, &lq, touched, &c->touched_tail};
-  ExpandChunks(chunks, c->nchunks, visit);
+  ExpandChunks<FrontierCut>(chunks, c->nchunks, visit);
   LdsQueueFlush(lq, touched, &c->touched_tail);
 }
 
@@ -882,7 +885,7 @@ struct MsBuffers {
   uint64_t* seen;
   uint64_t* acc;
   int32_t* touched;
-  EdgeChunk* chunks;  // null: no chunking (no vertex reaches kExpandBS edges)
+  EdgeChunk* chunks;  // null: no chunking (no vertex reaches FrontierCut::kMin edges)
   uint16_t* depth16;
   uint64_t full;
   // Propagation blocks for the densest bottom-up level (pb null when the
@@ -1053,8 +1056,8 @@ inline MsTraversal MsTraverse(gg_graph* g, const int32_t* droots, const int32_t*
   int32_t* act_a = g->Scratch<int32_t>("ms.act_a", n + 64);
   int32_t* act_b = g->Scratch<int32_t>("ms.act_b", n + 64);
   int32_t* touched = g->Scratch<int32_t>("ms.touched", n + 64);
-  const bool use_chunks = g->max_degree >= kExpandBS;
-  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("ms.chunks", MaxChunks(n, g->out_entries)) : nullptr;
+  const bool use_chunks = g->max_degree >= FrontierCut::kMin;
+  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("ms.chunks", FrontierCut::Bound(n, g->out_entries)) : nullptr;
   // Propagation blocks (the layout FP32 Jacobi PageRank runs through, built
   // on first use) for the first bottom-up level after a top-down one while
   // more than bfs_blocks_pct percent (default 50) of the in-edges are

@@ -69,12 +69,29 @@ struct RlCopy {
   const int64_t* new_off;
   const int32_t* new_id;
   int32_t* new_dst;
-  __device__ __forceinline__ void operator()(int32_t u, int32_t, int64_t e, bool valid) {
-    if (!valid) return;
-    const int64_t to = new_off[new_id[u]] + (e - old_off[u]);
-    new_dst[W * to] = new_id[old_dst[W * e]];
-    if (W == 2) new_dst[W * to + 1] = old_dst[W * e + 1];
+  __device__ __forceinline__ void Visit(const int32_t (&u)[kExpandEdges], const int32_t (&)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int32_t v[kExpandEdges], w[kExpandEdges];
+    int64_t to[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      v[k] = old_dst[W * e[k]];
+      w[k] = W == 2 ? old_dst[W * e[k] + 1] : 0;
+      to[k] = valid[k] ? e[k] - old_off[u[k]] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      v[k] = new_id[v[k]];
+      to[k] += valid[k] ? new_off[new_id[u[k]]] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      if (!valid[k]) continue;
+      new_dst[W * to[k]] = v[k];
+      if (W == 2) new_dst[W * to[k] + 1] = w[k];
+    }
   }
+  __device__ __forceinline__ void StepEnd() {}
 };
 
 template <int W>
@@ -92,7 +109,7 @@ __global__ __launch_bounds__(kBS) void RlCopyRows(const int64_t* __restrict__ ol
       b = old_off[u];
       e = old_off[u + 1];
     }
-    ExpandTile(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks, kChunkEdges);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks);
   }
 }
 
@@ -103,7 +120,7 @@ __global__ __launch_bounds__(kBS) void RlCopyChunks(const int64_t* __restrict__ 
                                                     const int32_t* __restrict__ new_id, int32_t* new_dst,
                                                     const EdgeChunk* chunks, const int32_t* nchunks) {
   RlCopy<W> op{old_off, old_dst, new_off, new_id, new_dst};
-  ExpandChunks(chunks, *nchunks, op);
+  ExpandChunks<WholeCut>(chunks, *nchunks, op);
 }
 
 // bounds[0] = first row with <= kMediumRow entries, bounds[1] = first row
@@ -218,8 +235,8 @@ void CopyLists(gg_graph* g, const int64_t* new_off, const int32_t* new_id, int32
   const int64_t n = g->n, entries = g->out_entries;
   const dim3 blk(kBS);
   int32_t* nchunks = g->Scratch<int32_t>("rl.nchunks", 1);
-  const bool use_chunks = g->max_degree >= kExpandBS;
-  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("rl.chunks", MaxChunks(n, entries)) : nullptr;
+  const bool use_chunks = g->max_degree >= WholeCut::kMin;
+  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("rl.chunks", WholeCut::Bound(n, entries)) : nullptr;
   Run(g, "relabel_clear", 0, RlZero, dim3(1), dim3(64), nchunks);
   Run(g, "relabel_copy", 8.0 * n + (8.0 * W + 4.0) * entries, RlCopyRows<W>, dim3(GridFor(n, kBS, g->cu_count * 8)),
       blk, static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), new_off, new_id,

@@ -33,7 +33,7 @@ namespace gg {
 namespace {
 
 constexpr int kBS = 256;
-constexpr int kQueueCap = 1024;
+constexpr int kQueueCap = 2048;
 constexpr int32_t kDistInf = INT32_MAX / 2;
 constexpr int kStripes = 64;
 constexpr int64_t kWindow = 8;  // buckets per mid window
@@ -119,7 +119,8 @@ __global__ __launch_bounds__(kBS) void SsspPublish(SsspCounters* c, int mode, un
   }
 }
 
-// Relaxes edge e of u (payload = dist[u] when u was loaded).
+// Relaxes edges e[k] of frontier vertices (payload = the vertex's distance when
+// it was loaded).
 struct RelaxVisit {
   const int2* wdst;
   int32_t* dist;
@@ -134,28 +135,42 @@ struct RelaxVisit {
   SsspCounters* c;
   unsigned long long relaxed = 0, improved = 0;
 
-  __device__ __forceinline__ void operator()(int32_t, int32_t du, int64_t e, bool valid) {
-    bool to_near = false, to_fresh = false;
-    int32_t v = 0;
-    if (valid) {
-      const int2 vw = wdst[e];
-      v = vw.x;
-      const int64_t nd = static_cast<int64_t>(du) + vw.y;
-      relaxed++;
-      if (nd < kDistInf && nd < dist[v]) {
-        const int32_t d = static_cast<int32_t>(nd);
-        const int32_t old = atomicMin(&dist[v], d);
-        if (d < old) {
-          improved++;
-          if (d < bucket_end)
-            to_near = atomicExch(&stamp[v], near_tag) != near_tag;
-          else
-            to_fresh = atomicExch(&freshstamp[v], fresh_tag) != fresh_tag;
-        }
-      }
+  __device__ __forceinline__ void Visit(const int32_t (&)[kExpandEdges], const int32_t (&du)[kExpandEdges],
+                                        const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
+    int2 vw[kExpandEdges];
+    int32_t v[kExpandEdges], old[kExpandEdges];
+    int64_t nd[kExpandEdges];
+    bool to_near[kExpandEdges], to_fresh[kExpandEdges], better[kExpandEdges];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) vw[k] = wdst[e[k]];
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      v[k] = vw[k].x;
+      nd[k] = static_cast<int64_t>(du[k]) + vw[k].y;
+      old[k] = dist[v[k]];
+      relaxed += valid[k];
     }
-    LdsQueuePush(*lnear, to_near, v, near, &c->near_tail);
-    LdsQueuePush(*lfresh, to_fresh, v, fresh, &c->fresh_tail);
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      better[k] = valid[k] && nd[k] < kDistInf && nd[k] < old[k];
+      if (better[k]) old[k] = atomicMin(&dist[v[k]], static_cast<int32_t>(nd[k]));
+    }
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) {
+      better[k] = better[k] && nd[k] < old[k];
+      improved += better[k];
+      const bool here = nd[k] < bucket_end;
+      const int32_t tag = here ? near_tag : fresh_tag;
+      const bool first = better[k] && atomicExch(here ? &stamp[v[k]] : &freshstamp[v[k]], tag) != tag;
+      to_near[k] = first && here;
+      to_fresh[k] = first && !here;
+    }
+    LdsQueuePushMany(*lnear, to_near, v, near, &c->near_tail);
+    LdsQueuePushMany(*lfresh, to_fresh, v, fresh, &c->fresh_tail);
+  }
+  __device__ __forceinline__ void StepEnd() {
+    LdsQueueMakeRoom(*lnear, near, &c->near_tail);
+    LdsQueueMakeRoom(*lfresh, fresh, &c->fresh_tail);
   }
 };
 
@@ -177,7 +192,7 @@ __global__ __launch_bounds__(kBS) void SsspRelax(const int64_t* __restrict__ off
                                                  const int32_t* __restrict__ frontier, int32_t fn,
                                                  int32_t bucket_end, int32_t near_tag, int32_t fresh_tag,
                                                  int32_t* __restrict__ near, int32_t* __restrict__ fresh,
-                                                 SsspCounters* c, EdgeChunk* chunks, int64_t chunk_min) {
+                                                 SsspCounters* c, EdgeChunk* chunks) {
   __shared__ ExpandShared sh;
   __shared__ LdsQueue<kQueueCap> lnear, lfresh;
   __shared__ unsigned long long s_red[kBS / kWave];
@@ -194,7 +209,7 @@ __global__ __launch_bounds__(kBS) void SsspRelax(const int64_t* __restrict__ off
       beg = off[u];
       end = off[u + 1];
     }
-    ExpandTile(sh, u, du, beg, end, rv, chunks, &c->nchunks, chunk_min);
+    ExpandTile<FrontierCut>(sh, u, du, beg, end, rv, chunks, &c->nchunks);
   }
   FlushRelax(rv, c, s_red);
 }
@@ -210,7 +225,7 @@ __global__ __launch_bounds__(kBS) void SsspRelaxChunks(const int2* __restrict__ 
   LdsQueueInit(lnear);
   LdsQueueInit(lfresh);
   RelaxVisit rv{wdst, dist, stamp, freshstamp, bucket_end, near_tag, fresh_tag, &lnear, &lfresh, near, fresh, c};
-  ExpandChunks(chunks, c->nchunks, rv);
+  ExpandChunks<FrontierCut>(chunks, c->nchunks, rv);
   FlushRelax(rv, c, s_red);
 }
 
@@ -331,9 +346,9 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
     int32_t* far = g->Scratch<int32_t>("sssp.far", 2 * n + 64);
     int32_t* far2 = g->Scratch<int32_t>("sssp.far2", 2 * n + 64);
     SsspCounters* dc = g->Scratch<SsspCounters>("sssp.ctr", 1);
-    const bool use_chunks = g->max_degree >= kExpandBS;
+    const bool use_chunks = g->max_degree >= FrontierCut::kMin;
     EdgeChunk* chunks =
-        use_chunks ? g->Scratch<EdgeChunk>("sssp.chunks", MaxChunks(n, g->out_entries)) : nullptr;
+        use_chunks ? g->Scratch<EdgeChunk>("sssp.chunks", FrontierCut::Bound(n, g->out_entries)) : nullptr;
 
     const dim3 blk(kBS);
     const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
@@ -381,12 +396,11 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
         GG_REQUIRE(relax_launches < max_launches, GG_EHIP, "SSSP did not converge");
         const int32_t near_tag = ++tag;
         const int32_t end32 = clamp(bucket_end);
-        const int64_t chunk_min = fsize <= 4096 ? kExpandBS : kChunkEdges;
         const int idx = Run(g, "sssp_relax", 12.0 * fsize, SsspRelax,
                             dim3(GridFor(fsize, kBS, g->cu_count * kBucketBlocksPerCu)), blk, g->out_off, wdst, dist,
                             stamp, freshstamp, static_cast<const int32_t*>(fq),
                             static_cast<int32_t>(fsize), end32, near_tag, fresh_tag, nq, fresh, dc,
-                            use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), chunk_min);
+                            use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr));
         launches++;
         if (use_chunks) {
           Run(g, "sssp_relax_chunks", 0, SsspRelaxChunks, dim3(g->cu_count * kBucketBlocksPerCu), blk, wdst, dist,

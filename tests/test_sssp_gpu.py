@@ -99,3 +99,21 @@ def test_sssp_errors():
     with pytest.raises(gpu.GpuError) as e:
         gpu.sssp(ug, 0, 2)
     assert e.value.code == -95
+
+
+@pytest.mark.parametrize("delta", [1, 64, 1024])
+def test_sssp_and_bfs_list_lengths(delta):
+    # Frontier vertices whose lists end around a step, a slice and a chunk of
+    # the tile expansion, with empty and one-entry lists between them.
+    print(f"[sssp] list lengths, delta {delta}", flush=True)
+    rng = np.random.default_rng(9)
+    lens = [0, 1, 2, 255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 5121, 8192, 8193] + [1, 3, 0] * 300
+    first = 1 + len(lens)
+    n = first + 9000
+    u = np.concatenate([np.zeros(len(lens), int), np.repeat(np.arange(1, first), lens)])
+    v = np.concatenate([np.arange(1, first)] + [rng.choice(np.arange(first, n), d, replace=False) for d in lens])
+    w = rng.integers(1, 256, len(u))
+    g = Graph.from_edges(u, v, w, symmetrize=False)
+    assert np.array_equal(gpu.sssp(gpu.DeviceGraph(g), 0, delta).dist, oracle.dijkstra(g, 0))
+    plain = g.strip_weights()
+    assert np.array_equal(gpu.bfs(gpu.DeviceGraph(plain), 0, alpha=1).depth, oracle.bfs_depth(plain, 0))
