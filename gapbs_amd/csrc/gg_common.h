@@ -342,6 +342,12 @@ __global__ __attribute__((unused)) void WorkClear(unsigned long long* work, int 
 // Sums the counters of `kinds` consecutive kinds: {entries, matched} each.
 std::vector<unsigned long long> ReadWork(gg_graph* g, const unsigned long long* work, int kinds);
 
+// Blocks per CU of the kernels that sum reached vertices and edges for the
+// statistics: each block ends with an atomic per total on one address, which
+// the chip takes one after another (8192 blocks spent 201 us on Kronecker 22's
+// 4.2 M vertices; 512 blocks 28 us).
+constexpr unsigned kReachBlocksPerCu = 2;
+
 inline unsigned GridFor(int64_t items, int block, unsigned cap = 1u << 20) {
   int64_t b = (items + block - 1) / block;
   if (b < 1) b = 1;

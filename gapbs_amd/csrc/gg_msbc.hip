@@ -651,7 +651,7 @@ void RunBatchBrandes(gg_graph* g, const int32_t* droots, int k, float* scores, g
     const std::vector<unsigned long long> w = ReadWork(g, ctr, kWKinds);
     unsigned long long* sums = g->Scratch<unsigned long long>("ms.reach", 2);
     MsZero2<<<1, 64, 0, st>>>(sums);
-    MsReach<<<grid_n, dim3(kBS), 0, st>>>(t.seen, g->out_off, n, sums);
+    MsReach<<<dim3(GridFor(n, kBS, g->cu_count * kReachBlocksPerCu)), dim3(kBS), 0, st>>>(t.seen, g->out_off, n, sums);
     unsigned long long reach[2];
     GG_HIP(hipMemcpyAsync(reach, sums, sizeof(reach), hipMemcpyDeviceToHost, st));
     GG_HIP(hipStreamSynchronize(st));

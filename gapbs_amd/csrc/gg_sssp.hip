@@ -465,7 +465,7 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
     if (stats) {
       unsigned long long* acc = g->Scratch<unsigned long long>("sssp.reach", 2);
       GG_HIP(hipMemsetAsync(acc, 0, 2 * sizeof(unsigned long long), st));
-      SsspReach<<<grid_n, blk, 0, st>>>(dist, g->out_off, n, acc);
+      SsspReach<<<dim3(GridFor(n, kBS, g->cu_count * kReachBlocksPerCu)), blk, 0, st>>>(dist, g->out_off, n, acc);
       unsigned long long h[2];
       GG_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, st));
       GG_HIP(hipStreamSynchronize(st));

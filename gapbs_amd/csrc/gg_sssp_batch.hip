@@ -804,7 +804,7 @@ extern "C" int gg_sssp_batch(gg_graph* g, const int32_t* roots, int k, int32_t d
     if (stats) {
       unsigned long long* acc = g->Scratch<unsigned long long>("sb.reach", 2);
       SbZero2<<<1, 64, 0, st>>>(acc);
-      SbReach<<<dim3(GridFor(n, kBS, g->cu_count * 16)), blk, 0, st>>>(b.dist, g->out_off, n, k, lg, acc);
+      SbReach<<<dim3(GridFor(n, kBS, g->cu_count * kReachBlocksPerCu)), blk, 0, st>>>(b.dist, g->out_off, n, k, lg, acc);
       unsigned long long h[2];
       GG_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, st));
       GG_HIP(hipStreamSynchronize(st));

@@ -289,3 +289,15 @@ def test_batch_blocks_pass_in_bc_and_default_off():
     assert e.value.code == -22
     plain.free()
     blk.free()
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 63, 64])
+def test_batch_read_out_groups(k, ordered):
+    # Depths are read out eight roots at a time: full, partial and single groups.
+    print(f"[msbfs] {k} roots, ordered {ordered}", flush=True)
+    g = cached_graph("g10", lambda: Graph.kronecker(10))
+    roots = g.pick_sources(64)[:k]
+    res = gpu.bfs_batch(gpu.DeviceGraph(g, order_by_degree=ordered), roots)
+    for i, r in enumerate(roots):
+        assert np.array_equal(res.depths[i], oracle.bfs_depth(g, int(r)))
