@@ -20,9 +20,13 @@
 //   * sigma is pulled: each newly discovered vertex sums sigma over its
 //     in-neighbours at the previous level (no floating-point atomics; the
 //     sums are exact integers below 2^53, so the order does not matter);
-//   * the sigma pull runs one thread per vertex; vertices with >= 256
-//     in-edges are cut into chunks summed by whole blocks and combined with
-//     one double atomic per chunk;
+//   * the sigma pull runs one thread per vertex below 64 in-edges; longer
+//     lists are cut into chunks of 1024, a wavefront each, whose sums are
+//     combined with one double atomic per chunk;
+//   * whether a neighbour lies on the next (or previous) level is one bit of
+//     that level's bitmap, which stays in L2, rather than its depth; a
+//     vertex's path count and dependency share a 16-byte record, one
+//     transaction per successor;
 //   * delta runs one thread per vertex below 64 edges and one wavefront or
 //     block per vertex above: 64 successor terms are computed at a time and
 //     folded into the accumulator as if in successor order (FoldTerms), so
@@ -32,6 +36,8 @@
 //     scores, each per-vertex dependency sum and each score sum over roots
 //     carrying a float compensation term; GG_BC_FP64: double dependencies
 //     and scores.
+#include <algorithm>
+
 #include "gg_common.h"
 #include "gg_expand.h"
 
@@ -41,14 +47,33 @@ namespace {
 constexpr int kBS = 256;
 constexpr int kQueueCap = 2048;
 constexpr int kStripes = 64;
-constexpr int64_t kHubEdges = 256;   // sigma pull: vertices with this many in-edges use chunks
-constexpr int64_t kWaveEdges = 64;   // delta: vertices with this many edges use a wavefront
+constexpr int64_t kWaveEdges = 64;   // vertices with this many edges use a wavefront ...
+constexpr int64_t kSigmaChunk = 1024;  // ... per this many (sigma pull)
+constexpr int kThreadUnroll = 4;     // edges in flight per thread below that
 constexpr int kBcWaveUnroll = 4;     // 64-edge runs per wavefront step
 constexpr int64_t kBcHubEdges = 4096;  // ... and with this many, a block (BcDeltaHub)
 constexpr int kBcHubProducers = 15;
 constexpr int kBcHubUnroll = 2;  // 64-edge runs per producer wavefront and round
 constexpr int kBcHubGrid = 2;    // BcDeltaHub blocks per CU
 constexpr int kBcHubBS = (kBcHubProducers + 1) * kWave;
+
+// A vertex's path count and dependency, read together by its predecessors.
+template <class T>
+struct alignas(16) BcNode {
+  double sigma;
+  T delta;
+};
+
+// Tells whether a vertex lies on one level: its bit in the level's bitmap,
+// or, without bitmaps (deep traversals), its depth.
+struct OnLevel {
+  const uint32_t* bits;
+  const int32_t* depth;
+  int32_t level;
+  __device__ __forceinline__ bool operator()(int32_t v) const {
+    return bits ? (bits[v >> 5] >> (v & 31)) & 1 : depth[v] == level;
+  }
+};
 
 struct BcCounters {
   int32_t tail;     // queue length (all levels so far)
@@ -64,15 +89,16 @@ __device__ __forceinline__ int32_t Load(const int32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <class T>
 __global__ __launch_bounds__(kBS) void BcResetSource(int32_t* __restrict__ depth, int64_t n, int32_t src,
-                                                     double* __restrict__ sigma, int32_t* __restrict__ queue,
+                                                     BcNode<T>* __restrict__ node, int32_t* __restrict__ queue,
                                                      BcCounters* c) {
   for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBS)
     depth[i] = i == src ? 0 : -1;
   if (blockIdx.x == 0) {
     if (threadIdx.x < kStripes) c->examined[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
-      sigma[src] = 1.0;
+      node[src].sigma = 1.0;
       queue[0] = src;
       c->tail = 1;
       c->nchunks = 0;
@@ -143,69 +169,102 @@ __global__ __launch_bounds__(kBS) void BcDiscoverChunks(const int32_t* __restric
   LdsQueueFlush(lq, queue, &c->tail);
 }
 
-// Appends the chunks of a hub vertex (>= kHubEdges edges) for a reduction.
-__device__ __forceinline__ void EmitReduceChunks(int32_t u, int64_t beg, int64_t end, EdgeChunk* chunks,
-                                                 int32_t* nchunks) {
-  const int nc = static_cast<int>((end - beg + kChunkEdges - 1) / kChunkEdges);
-  const int base = atomicAdd(nchunks, nc);
-  for (int k = 0; k < nc; k++) {
-    const int64_t cb = beg + k * kChunkEdges;
-    chunks[base + k] = EdgeChunk{cb, cb + kChunkEdges < end ? cb + kChunkEdges : end, u, k == 0};
-  }
-}
-
 // sigma[v] for the new level: sum of sigma over in-neighbours one level up.
-// Hubs get sigma = 0 here and their chunks summed by BcSigmaChunks.
+// Vertices with kWaveEdges in-edges or more are listed in chunks of
+// kSigmaChunk edges (one reservation per wavefront) and summed by
+// BcSigmaChunks; those of several chunks start from sigma = 0 here.
+template <class T>
 __global__ __launch_bounds__(kBS) void BcSigma(const int64_t* __restrict__ in_off, const int32_t* __restrict__ in_dst,
-                                               const int32_t* __restrict__ depth, double* __restrict__ sigma,
-                                               const int32_t* __restrict__ queue, int32_t qb, int32_t qn,
-                                               int32_t prev_depth, EdgeChunk* chunks, BcCounters* c,
+                                               OnLevel prev, BcNode<T>* node, const int32_t* __restrict__ queue,
+                                               int32_t qb, int32_t qn, EdgeChunk* __restrict__ chunks, BcCounters* c,
                                                unsigned long long* work) {
   __shared__ unsigned long long s_red[kBS / kWave];
   unsigned long long ent = 0, mat = 0;
-  for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < qn; i += int64_t(gridDim.x) * kBS) {
-    const int32_t v = queue[qb + i];
-    const int64_t b = in_off[v], e = in_off[v + 1];
-    if (e - b >= kHubEdges) {
-      sigma[v] = 0.0;
-      EmitReduceChunks(v, b, e, chunks, &c->nred);
-      continue;
+  for (int64_t base = int64_t(blockIdx.x) * kBS; base < qn; base += int64_t(gridDim.x) * kBS) {
+    const int64_t i = base + threadIdx.x;
+    int32_t v = 0;
+    int64_t b = 0, e = 0;
+    if (i < qn) {
+      v = queue[qb + i];
+      b = in_off[v];
+      e = in_off[v + 1];
     }
+    const int nc = e - b >= kWaveEdges ? static_cast<int>((e - b + kSigmaChunk - 1) / kSigmaChunk) : 0;
+    const int upto = WaveInclusiveScan(nc);
+    const int total = __builtin_amdgcn_readlane(upto, kWave - 1);
+    if (total) {
+      int at = 0;
+      if (LaneId() == 0) at = atomicAdd(&c->nred, total);
+      at = __builtin_amdgcn_readfirstlane(at) + upto - nc;
+      for (int k = 0; k < nc; k++) {
+        const int64_t cb = b + k * kSigmaChunk;
+        // payload: whether the chunk is the whole list (its sum is stored)
+        chunks[at + k] = EdgeChunk{cb, cb + kSigmaChunk < e ? cb + kSigmaChunk : e, v, nc == 1};
+      }
+      if (nc > 1) node[v].sigma = 0.0;
+    }
+    if (nc || i >= qn) continue;
     double s = 0.0;
-    for (int64_t k = b; k < e; k++) {
-      const int32_t u = in_dst[k];
-      if (depth[u] == prev_depth) {
-        s += sigma[u];
-        mat++;
+    for (int64_t k = b; k < e; k += kThreadUnroll) {
+      int32_t u[kThreadUnroll];
+      bool has[kThreadUnroll];
+      double x[kThreadUnroll];
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) u[j] = in_dst[k + j < e ? k + j : k];
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) has[j] = prev(u[j]) && k + j < e;
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) x[j] = has[j] ? node[u[j]].sigma : 0.0;
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) {
+        s += x[j];
+        mat += has[j];
       }
     }
     ent += static_cast<unsigned long long>(e - b);
-    sigma[v] = s;
+    node[v].sigma = s;
   }
   WorkAdd(work, BlockSum<kBS>(ent, s_red), BlockSum<kBS>(mat, s_red));
 }
 
-__global__ __launch_bounds__(kBS) void BcSigmaChunks(const int32_t* __restrict__ in_dst,
-                                                     const int32_t* __restrict__ depth, double* sigma,
-                                                     int32_t prev_depth, const EdgeChunk* chunks,
+// One wavefront per chunk.
+template <class T>
+__global__ __launch_bounds__(kBS) void BcSigmaChunks(const int32_t* __restrict__ in_dst, OnLevel prev,
+                                                     BcNode<T>* node, const EdgeChunk* __restrict__ chunks,
                                                      const BcCounters* c, unsigned long long* work) {
-  __shared__ double s_red[kBS / kWave];
   __shared__ unsigned long long s_cnt[kBS / kWave];
+  const int lane = LaneId();
   const int32_t nc = c->nred;
+  const int32_t wave = blockIdx.x * (kBS / kWave) + threadIdx.x / kWave;
+  const int32_t nwaves = gridDim.x * (kBS / kWave);
   unsigned long long ent = 0, mat = 0;
-  for (int32_t ci = blockIdx.x; ci < nc; ci += gridDim.x) {
+  for (int32_t ci = wave; ci < nc; ci += nwaves) {
     const EdgeChunk ch = chunks[ci];
     double s = 0.0;
-    for (int64_t k = ch.beg + threadIdx.x; k < ch.end; k += kBS) {
-      const int32_t u = in_dst[k];
-      ent++;
-      if (depth[u] == prev_depth) {
-        s += sigma[u];
-        mat++;
+    for (int64_t k = ch.beg + lane; k - lane < ch.end; k += kWave * kThreadUnroll) {
+      int32_t u[kThreadUnroll];
+      bool has[kThreadUnroll];
+      double x[kThreadUnroll];
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) u[j] = in_dst[k + j * kWave < ch.end ? k + j * kWave : ch.beg];
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) has[j] = prev(u[j]) && k + j * kWave < ch.end;
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) x[j] = has[j] ? node[u[j]].sigma : 0.0;
+#pragma unroll
+      for (int j = 0; j < kThreadUnroll; j++) {
+        s += x[j];
+        mat += has[j];
       }
     }
-    s = BlockSum<kBS>(s, s_red);
-    if (threadIdx.x == 0 && s != 0.0) atomicAdd(&sigma[ch.u], s);
+    s = WaveSum(s);
+    if (lane == 0) {
+      ent += static_cast<unsigned long long>(ch.end - ch.beg);
+      if (ch.payload)
+        node[ch.u].sigma = s;
+      else if (s != 0.0)
+        atomicAdd(&node[ch.u].sigma, s);
+    }
   }
   WorkAdd(work, BlockSum<kBS>(ent, s_cnt), BlockSum<kBS>(mat, s_cnt));
 }
@@ -351,11 +410,9 @@ __device__ __forceinline__ void AddScore(double* score, double*, int32_t u, doub
 // BcDeltaWave, and those with kBcHubEdges or more for BcDeltaHub.
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBS) void BcDelta(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
-                                               const int32_t* __restrict__ depth,
-                                               const double* __restrict__ sigma, T* __restrict__ delta,
-                                               T* __restrict__ score, T* __restrict__ comp,
-                                               const int32_t* __restrict__ queue, int32_t qb, int32_t qn,
-                                               int32_t level, int32_t* __restrict__ wave_list,
+                                               OnLevel next, BcNode<T>* node, T* __restrict__ score,
+                                               T* __restrict__ comp, const int32_t* __restrict__ queue, int32_t qb,
+                                               int32_t qn, int32_t* __restrict__ wave_list,
                                                int32_t* __restrict__ hub_list, BcCounters* c,
                                                unsigned long long* work) {
   __shared__ unsigned long long s_red[kBS / kWave];
@@ -370,18 +427,28 @@ __global__ __launch_bounds__(kBS) void BcDelta(const int64_t* __restrict__ off, 
       big = e - b >= kWaveEdges;
       hub = e - b >= kBcHubEdges;
       if (!big) {
-        const double su = sigma[u];
+        const double su = node[u].sigma;
         typename AccFor<T, kKahan>::Type acc = AccFor<T, kKahan>::Type::Zero();
-        for (int64_t k = b; k < e; k++) {
-          const int32_t v = dst[k];
-          if (depth[v] == level + 1) {
-            acc.Add(DeltaTerm(su, sigma[v], delta[v]));
+        for (int64_t k = b; k < e; k += kThreadUnroll) {
+          int32_t v[kThreadUnroll];
+          bool has[kThreadUnroll];
+          BcNode<T> x[kThreadUnroll];
+#pragma unroll
+          for (int j = 0; j < kThreadUnroll; j++) v[j] = dst[k + j < e ? k + j : k];
+#pragma unroll
+          for (int j = 0; j < kThreadUnroll; j++) has[j] = next(v[j]) && k + j < e;
+#pragma unroll
+          for (int j = 0; j < kThreadUnroll; j++) x[j] = node[has[j] ? v[j] : u];
+#pragma unroll
+          for (int j = 0; j < kThreadUnroll; j++) {
+            if (!has[j]) continue;
+            acc.Add(DeltaTerm(su, x[j].sigma, x[j].delta));
             mat++;
           }
         }
         ent += static_cast<unsigned long long>(e - b);
         const T d = acc.Value();
-        delta[u] = d;
+        node[u].delta = d;
         AddScore<kKahan>(score, comp, u, d);
       }
     }
@@ -395,10 +462,8 @@ __global__ __launch_bounds__(kBS) void BcDelta(const int64_t* __restrict__ off, 
 // folded into the accumulator in edge order.
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
-                                                   const int32_t* __restrict__ depth,
-                                                   const double* __restrict__ sigma, T* __restrict__ delta,
-                                                   T* __restrict__ score, T* __restrict__ comp,
-                                                   const int32_t* __restrict__ wave_list, int32_t level,
+                                                   OnLevel next, BcNode<T>* node, T* __restrict__ score,
+                                                   T* __restrict__ comp, const int32_t* __restrict__ wave_list,
                                                    const BcCounters* c, unsigned long long* work) {
   __shared__ unsigned long long s_red[kBS / kWave];
   const int lane = LaneId();
@@ -409,19 +474,24 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
   for (int64_t i = wave; i < nw; i += nwaves) {
     const int32_t u = wave_list[i];
     const int64_t b = off[u], e = off[u + 1];
-    const double su = sigma[u];
+    const double su = node[u].sigma;
     typename AccFor<T, kKahan>::Type acc = AccFor<T, kKahan>::Type::Zero();
     for (int64_t base = b; base < e; base += kWave * kBcWaveUnroll) {
       // kBcWaveUnroll runs of 64 edges, their loads issued together.
       int32_t v[kBcWaveUnroll];
       bool has[kBcWaveUnroll];
+      BcNode<T> x[kBcWaveUnroll];
       double term[kBcWaveUnroll];
+      const int64_t k = base + lane;
 #pragma unroll
-      for (int r = 0; r < kBcWaveUnroll; r++) v[r] = base + r * kWave + lane < e ? dst[base + r * kWave + lane] : -1;
+      for (int r = 0; r < kBcWaveUnroll; r++) v[r] = dst[k + r * kWave < e ? k + r * kWave : b];
 #pragma unroll
-      for (int r = 0; r < kBcWaveUnroll; r++) has[r] = v[r] >= 0 && depth[v[r]] == level + 1;
+      for (int r = 0; r < kBcWaveUnroll; r++) has[r] = next(v[r]) && k + r * kWave < e;
+      // (a lane without a successor reads the vertex's own record)
 #pragma unroll
-      for (int r = 0; r < kBcWaveUnroll; r++) term[r] = has[r] ? DeltaTerm(su, sigma[v[r]], delta[v[r]]) : 0.0;
+      for (int r = 0; r < kBcWaveUnroll; r++) x[r] = node[has[r] ? v[r] : u];
+#pragma unroll
+      for (int r = 0; r < kBcWaveUnroll; r++) term[r] = DeltaTerm(su, x[r].sigma, x[r].delta);
 #pragma unroll
       for (int r = 0; r < kBcWaveUnroll; r++) {
         const uint64_t m = __ballot(has[r]);
@@ -432,7 +502,7 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
     if (lane == 0) {
       ent += static_cast<unsigned long long>(e - b);
       const T d = acc.Value();
-      delta[u] = d;
+      node[u].delta = d;
       AddScore<kKahan>(score, comp, u, d);
     }
   }
@@ -451,10 +521,8 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict__ off,
                                                        const int32_t* __restrict__ dst,
-                                                       const int32_t* __restrict__ depth,
-                                                       const double* __restrict__ sigma, T* __restrict__ delta,
-                                                       T* __restrict__ score, T* __restrict__ comp,
-                                                       const int32_t* __restrict__ hub_list, int32_t level,
+                                                       OnLevel next, BcNode<T>* node, T* __restrict__ score,
+                                                       T* __restrict__ comp, const int32_t* __restrict__ hub_list,
                                                        BcCounters* c, unsigned long long* work) {
   __shared__ double terms[2][kBcHubProducers][kWave * kBcHubUnroll];
   __shared__ int counts[2][kBcHubProducers];
@@ -472,23 +540,38 @@ __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict
     if (i >= nh) break;
     const int32_t u = hub_list[i];
     const int64_t b = off[u], e = off[u + 1];
-    const double su = sigma[u];
+    const double su = node[u].sigma;
     typename AccFor<T, kKahan>::Type acc = AccFor<T, kKahan>::Type::Zero();
     const int64_t rounds = (e - b + kRound - 1) / kRound;
+    // kBcHubUnroll consecutive runs of 64 edges per producer and round; the
+    // successor ids of the next round are loaded while this one's records
+    // are on their way.
+    const int64_t mine = b + int64_t(wid) * (kWave * kBcHubUnroll) + lane;
+    auto id_at = [&](int64_t round, int r) {
+      const int64_t at = mine + round * kRound + r * kWave;
+      return dst[at < e ? at : b];
+    };
+    int32_t v[kBcHubUnroll];
+    if (wid < kBcHubProducers) {
+#pragma unroll
+      for (int r = 0; r < kBcHubUnroll; r++) v[r] = id_at(0, r);
+    }
     for (int64_t k = 0; k <= rounds; k++) {
       if (wid < kBcHubProducers) {
         if (k < rounds) {
-          // kBcHubUnroll consecutive runs of 64 edges, their loads issued together.
-          const int64_t k0 = b + k * kRound + int64_t(wid) * (kWave * kBcHubUnroll) + lane;
-          int32_t v[kBcHubUnroll];
+          const int64_t k0 = mine + k * kRound;
           bool has[kBcHubUnroll];
+          BcNode<T> x[kBcHubUnroll];
 #pragma unroll
-          for (int r = 0; r < kBcHubUnroll; r++) v[r] = k0 + r * kWave < e ? dst[k0 + r * kWave] : -1;
+          for (int r = 0; r < kBcHubUnroll; r++) has[r] = next(v[r]) && k0 + r * kWave < e;
+          // (a lane without a successor reads the hub's own record)
 #pragma unroll
-          for (int r = 0; r < kBcHubUnroll; r++) has[r] = v[r] >= 0 && depth[v[r]] == level + 1;
+          for (int r = 0; r < kBcHubUnroll; r++) x[r] = node[has[r] ? v[r] : u];
+#pragma unroll
+          for (int r = 0; r < kBcHubUnroll; r++) v[r] = id_at(k + 1, r);
           double term[kBcHubUnroll];
 #pragma unroll
-          for (int r = 0; r < kBcHubUnroll; r++) term[r] = has[r] ? DeltaTerm(su, sigma[v[r]], delta[v[r]]) : 0.0;
+          for (int r = 0; r < kBcHubUnroll; r++) term[r] = DeltaTerm(su, x[r].sigma, x[r].delta);
           int pos = 0;
 #pragma unroll
           for (int r = 0; r < kBcHubUnroll; r++) {
@@ -517,7 +600,7 @@ __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict
     }
     if (wid == kBcHubProducers && lane == 0) {
       const T d = acc.Value();
-      delta[u] = d;
+      node[u].delta = d;
       AddScore<kKahan>(score, comp, u, d);
     }
   }
@@ -533,45 +616,82 @@ __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict
 // dependency passes read (level d at queue[bounds[d], bounds[d + 1]); the
 // order inside a level does not affect any result).
 constexpr int kBucketLevels = 4096;  // deeper traversals use the top-down discovery
-constexpr int64_t kBucketChunk = 65536;
+constexpr int kBitLevels = 32;       // up to this many levels also get bitmaps (n / 8 bytes each)
+// Vertices per block of the bucketing: enough blocks to fill the chip, few
+// enough that their reservations on a level's one cursor stay cheap.
+inline int64_t BucketChunk(int64_t n) { return std::max<int64_t>(4096, ((n >> 11) + 255) / 256 * 256); }
 
+// For each level d present among the wavefront's 64 depths: op(d, its lanes).
+template <class Op>
+__device__ __forceinline__ void ForLevels(int32_t d, int nlev, Op op) {
+  uint64_t left = __ballot(d >= 0 && d < nlev);
+  while (left) {
+    const int32_t ld = __builtin_amdgcn_readlane(d, __builtin_ctzll(left));
+    const uint64_t m = __ballot(d == ld);
+    op(ld, m);
+    left &= ~m;
+  }
+}
+
+// Vertices per level, and (bits non-null, zeroed before) each level's bitmap
+// of nwords words.  A wavefront takes 64 consecutive vertices and counts a
+// level's by ballot: an LDS atomic per vertex put most of a wavefront on one
+// address (76 us on Kronecker 22 against 30 us, with the bitmaps).
 __global__ __launch_bounds__(kBS) void BcLevelCount(const int32_t* __restrict__ depth, int64_t n, int nlev,
-                                                    int32_t* counts) {
+                                                    int32_t* counts, uint64_t* __restrict__ bits) {
   __shared__ int32_t h[kBucketLevels];
   for (int i = threadIdx.x; i < nlev; i += kBS) h[i] = 0;
   __syncthreads();
-  const int64_t lo = int64_t(blockIdx.x) * kBucketChunk;
-  const int64_t hi = lo + kBucketChunk < n ? lo + kBucketChunk : n;
-  for (int64_t v = lo + threadIdx.x; v < hi; v += kBS) {
-    const int32_t d = depth[v];
-    if (d >= 0 && d < nlev) atomicAdd(&h[d], 1);
+  const int lane = LaneId();
+  const int64_t nwords = (n + 63) >> 6;
+  for (int64_t w = (int64_t(blockIdx.x) * kBS + threadIdx.x) / kWave; w < nwords;
+       w += int64_t(gridDim.x) * (kBS / kWave)) {
+    const int64_t v = w * 64 + lane;
+    ForLevels(v < n ? depth[v] : -1, nlev, [&](int32_t d, uint64_t m) {
+      if (lane != 0) return;
+      atomicAdd(&h[d], __popcll(m));
+      if (bits) bits[d * nwords + w] = m;
+    });
   }
   __syncthreads();
   for (int i = threadIdx.x; i < nlev; i += kBS)
     if (h[i]) atomicAdd(&counts[i], h[i]);
 }
 
-// cursor[d] starts at bounds[d]; each block reserves its ranges with one
-// atomic per level it holds.
-__global__ __launch_bounds__(kBS) void BcLevelScatter(const int32_t* __restrict__ depth, int64_t n, int nlev,
-                                                      int32_t* cursor, int32_t* __restrict__ queue) {
+// cursor[d] starts at bounds[d]; each block (`chunk` vertices) reserves its
+// ranges with one atomic per level it holds.  Kronecker 22: 113 us with 64
+// blocks of 65536 vertices, 28 us with 2048.
+__global__ __launch_bounds__(kBS) void BcLevelScatter(const int32_t* __restrict__ depth, int64_t n, int64_t chunk,
+                                                      int nlev, int32_t* cursor, int32_t* __restrict__ queue) {
   __shared__ int32_t h[kBucketLevels];
   for (int i = threadIdx.x; i < nlev; i += kBS) h[i] = 0;
   __syncthreads();
-  const int64_t lo = int64_t(blockIdx.x) * kBucketChunk;
-  const int64_t hi = lo + kBucketChunk < n ? lo + kBucketChunk : n;
-  for (int64_t v = lo + threadIdx.x; v < hi; v += kBS) {
-    const int32_t d = depth[v];
-    if (d >= 0 && d < nlev) atomicAdd(&h[d], 1);
-  }
+  const int lane = LaneId();
+  const int64_t lo = int64_t(blockIdx.x) * chunk;
+  const int64_t hi = lo + chunk < n ? lo + chunk : n;
+  for (int64_t b = lo + (threadIdx.x - lane); b < hi; b += kBS)
+    ForLevels(b + lane < hi ? depth[b + lane] : -1, nlev, [&](int32_t d, uint64_t m) {
+      if (lane == 0) atomicAdd(&h[d], __popcll(m));
+    });
   __syncthreads();
   for (int i = threadIdx.x; i < nlev; i += kBS)
     if (h[i]) h[i] = atomicAdd(&cursor[i], h[i]);
   __syncthreads();
-  for (int64_t v = lo + threadIdx.x; v < hi; v += kBS) {
-    const int32_t d = depth[v];
-    if (d >= 0 && d < nlev) queue[atomicAdd(&h[d], 1)] = static_cast<int32_t>(v);
-  }
+  for (int64_t b = lo + (threadIdx.x - lane); b < hi; b += kBS)
+    ForLevels(b + lane < hi ? depth[b + lane] : -1, nlev, [&](int32_t d, uint64_t m) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&h[d], __popcll(m));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if ((m >> lane) & 1) queue[at + __popcll(LanesBelow(m))] = static_cast<int32_t>(b + lane);
+    });
+}
+
+// Zeroes the level counts and bitmap words.
+__global__ __launch_bounds__(kBS) void BcLevelClear(int32_t* __restrict__ counts, int nlev,
+                                                    uint64_t* __restrict__ bits, int64_t words) {
+  const int64_t i0 = blockIdx.x * int64_t(kBS) + threadIdx.x;
+  if (i0 < nlev) counts[i0] = 0;
+  for (int64_t i = i0; i < words; i += int64_t(gridDim.x) * kBS) bits[i] = 0;
 }
 
 __global__ __launch_bounds__(kBS) void BcClearReduce(BcCounters* c) {
@@ -660,9 +780,8 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   hipStream_t st = g->stream;
   const char* tag = sizeof(T) == 4 ? "32" : "64";
   int32_t* depth = g->Scratch<int32_t>("bc.depth", n);
-  double* sigma = g->Scratch<double>("bc.sigma", n);
+  BcNode<T>* node = g->Scratch<BcNode<T>>((std::string("bc.node") + tag).c_str(), n);
   int32_t* queue = g->Scratch<int32_t>("bc.queue", n + 64);
-  T* delta = g->Scratch<T>((std::string("bc.delta") + tag).c_str(), n);
   T* score = g->Scratch<T>((std::string("bc.score") + tag).c_str(), n);
   T* comp = sizeof(T) == 4 ? g->Scratch<T>("bc.comp32", n) : nullptr;  // zero unless kKahan
   int32_t* wave_list = g->Scratch<int32_t>("bc.wave_list", n + 64);
@@ -685,8 +804,12 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   std::vector<int32_t> h_counts(kBucketLevels);
   const int64_t entries = g->out_entries > g->in_entries ? g->out_entries : g->in_entries;
   EdgeChunk* chunks = g->Scratch<EdgeChunk>("bc.chunks", FrontierCut::Bound(n, entries));
-  EdgeChunk* rchunks = g->Scratch<EdgeChunk>("bc.rchunks", entries / kChunkEdges + entries / kHubEdges + 2);
-  const bool hubs = g->max_degree >= kHubEdges;
+  const bool hubs = g->max_degree >= FrontierCut::kMin, longs = g->max_degree >= kWaveEdges;
+  // Sigma chunks: sum of ceil(d / kSigmaChunk) over the vertices of kWaveEdges or more.
+  EdgeChunk* rchunks =
+      longs ? g->Scratch<EdgeChunk>("bc.rchunks", entries / kSigmaChunk + std::min(n, entries / kWaveEdges) + 2)
+            : nullptr;
+  const int64_t nwords = (n + 63) / 64;
   const dim3 blk(kBS);
   const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
   const dim3 grid_c(g->cu_count * 4);
@@ -703,7 +826,7 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   launches += 2;
   std::vector<int32_t> bounds;
   for (int r = 0; r < k; r++) {
-    Run(g, "bc_reset_source", 4 * N, BcResetSource, grid_n, blk, depth, n, roots[r], sigma, queue, dc);
+    Run(g, "bc_reset_source", 4 * N, BcResetSource<T>, grid_n, blk, depth, n, roots[r], node, queue, dc);
     launches++;
     bounds.assign(1, 0);
     bounds.push_back(1);
@@ -714,11 +837,33 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     examined_total += br.examined;
     const int nlev = static_cast<int>(br.td + br.bu + 1);
     bool bucketed = false;
+    uint64_t* bits = nullptr;
+    auto on_level = [&](int32_t d) {
+      return OnLevel{bits ? reinterpret_cast<const uint32_t*>(bits + d * nwords) : nullptr, depth, d};
+    };
+    // Path counts of level d, queue[nb, nb + nn).
+    auto pull_sigma = [&](int32_t d, int32_t nb, int32_t nn) {
+      note(kWSigma, Run(g, "bc_sigma", 20.0 * nn, BcSigma<T>, dim3(GridFor(nn, kBS, g->cu_count * 16)), blk,
+                        static_cast<const int64_t*>(g->in_off), static_cast<const int32_t*>(g->in_dst),
+                        on_level(d - 1), node, static_cast<const int32_t*>(queue), nb, nn, rchunks, dc, wk(kWSigma)));
+      launches++;
+      if (longs) {
+        note(kWSigmaChunks,
+             Run(g, "bc_sigma_chunks", 0, BcSigmaChunks<T>, dim3(g->cu_count * 8), blk,
+                 static_cast<const int32_t*>(g->in_dst), on_level(d - 1), node,
+                 static_cast<const EdgeChunk*>(rchunks), static_cast<const BcCounters*>(dc), wk(kWSigmaChunks)));
+        Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
+        launches += 2;
+      }
+    };
     if (nlev <= kBucketLevels) {
-      GG_HIP(hipMemsetAsync(lvl_counts, 0, sizeof(int32_t) * nlev, st));
-      const dim3 grid_b(GridFor(n, static_cast<int>(kBucketChunk), 1u << 20));
-      Run(g, "bc_level_count", 4 * N, BcLevelCount, grid_b, blk, static_cast<const int32_t*>(depth), n, nlev,
-          lvl_counts);
+      if (nlev <= kBitLevels) bits = g->Scratch<uint64_t>("bc.level_bits", kBitLevels * nwords);
+      const int64_t chunk = BucketChunk(n);
+      const dim3 grid_b(GridFor(n, static_cast<int>(chunk)));
+      Run(g, "bc_level_count", 0, BcLevelClear, grid_n, blk, lvl_counts, nlev, bits, bits ? nlev * nwords : 0);
+      Run(g, "bc_level_count", 4 * N, BcLevelCount, dim3(GridFor(nwords, kBS / kWave, g->cu_count * 8)), blk,
+          static_cast<const int32_t*>(depth), n, nlev, lvl_counts, bits);
+      launches++;
       GG_HIP(hipMemcpyAsync(h_counts.data(), lvl_counts, sizeof(int32_t) * nlev, hipMemcpyDeviceToHost, st));
       GG_HIP(hipStreamSynchronize(st));
       int last = 0;
@@ -727,31 +872,16 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
       bounds.assign(1, 0);
       for (int d = 0; d <= last; d++) bounds.push_back(bounds.back() + h_counts[d]);
       GG_HIP(hipMemcpyAsync(lvl_cursor, bounds.data(), sizeof(int32_t) * (last + 1), hipMemcpyHostToDevice, st));
-      Run(g, "bc_level_scatter", 8 * N, BcLevelScatter, grid_b, blk, static_cast<const int32_t*>(depth), n, last + 1,
+      Run(g, "bc_level_scatter", 8 * N, BcLevelScatter, grid_b, blk, static_cast<const int32_t*>(depth), n, chunk, last + 1,
           lvl_cursor, queue);
       launches += 2;
-      for (int32_t d = 1; d <= last; d++) {
-        const int32_t nb = bounds[d], nn = bounds[d + 1] - bounds[d];
-        note(kWSigma, Run(g, "bc_sigma", 20.0 * nn, BcSigma, dim3(GridFor(nn, kBS, g->cu_count * 16)), blk,
-                          static_cast<const int64_t*>(g->in_off), static_cast<const int32_t*>(g->in_dst),
-                          static_cast<const int32_t*>(depth), sigma, static_cast<const int32_t*>(queue), nb, nn,
-                          d - 1, rchunks, dc, wk(kWSigma)));
-        launches++;
-        if (hubs) {
-          note(kWSigmaChunks,
-               Run(g, "bc_sigma_chunks", 0, BcSigmaChunks, grid_c, blk, static_cast<const int32_t*>(g->in_dst),
-                   static_cast<const int32_t*>(depth), sigma, d - 1, static_cast<const EdgeChunk*>(rchunks),
-                   static_cast<const BcCounters*>(dc), wk(kWSigmaChunks)));
-          Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
-          launches += 2;
-        }
-      }
+      for (int32_t d = 1; d <= last; d++) pull_sigma(d, bounds[d], bounds[d + 1] - bounds[d]);
       level = last;
       bucketed = true;
     } else {
       // Too deep for the buckets: the top-down discovery, level by level
       // (the BFS above only cost its own time; reset its outputs).
-      Run(g, "bc_reset_source", 4 * N, BcResetSource, grid_n, blk, depth, n, roots[r], sigma, queue, dc);
+      Run(g, "bc_reset_source", 4 * N, BcResetSource<T>, grid_n, blk, depth, n, roots[r], node, queue, dc);
       launches++;
     }
     while (!bucketed) {
@@ -776,19 +906,7 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
       if (tail == bounds.back()) break;
       const int32_t nb = bounds.back(), nn = tail - nb;
       bounds.push_back(tail);
-      note(kWSigma, Run(g, "bc_sigma", 20.0 * nn, BcSigma, dim3(GridFor(nn, kBS, g->cu_count * 16)), blk,
-                        static_cast<const int64_t*>(g->in_off), static_cast<const int32_t*>(g->in_dst),
-                        static_cast<const int32_t*>(depth), sigma, static_cast<const int32_t*>(queue), nb, nn,
-                        level, rchunks, dc, wk(kWSigma)));
-      launches++;
-      if (hubs) {
-        note(kWSigmaChunks,
-             Run(g, "bc_sigma_chunks", 0, BcSigmaChunks, grid_c, blk, static_cast<const int32_t*>(g->in_dst),
-                 static_cast<const int32_t*>(depth), sigma, level, static_cast<const EdgeChunk*>(rchunks),
-                 static_cast<const BcCounters*>(dc), wk(kWSigmaChunks)));
-        Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
-        launches += 2;
-      }
+      pull_sigma(level + 1, nb, nn);
       level++;
     }
     reached_total += bounds.back();
@@ -796,11 +914,12 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     // Backward: deepest level first; delta of level d reads level d + 1.
     for (int32_t d = level; d >= 0; d--) {
       const int32_t qb = bounds[d], qn = bounds[d + 1] - bounds[d];
+      // (below the deepest level nothing is marked: no bitmap, no depth)
+      const OnLevel next = d < level ? on_level(d + 1) : OnLevel{nullptr, depth, d + 1};
       note(kWDelta, Run(g, "bc_delta", (16.0 + 2 * sizeof(T) + 8.0) * qn, BcDelta<T, kKahan>,
                         dim3(GridFor(qn, kBS, g->cu_count * 16)), blk, static_cast<const int64_t*>(g->out_off),
-                        fold_dst, static_cast<const int32_t*>(depth), static_cast<const double*>(sigma), delta,
-                        score, comp, static_cast<const int32_t*>(queue), qb, qn, d, wave_list, hub_list, dc,
-                        wk(kWDelta)));
+                        fold_dst, next, node, score, comp, static_cast<const int32_t*>(queue), qb, qn, wave_list,
+                        hub_list, dc, wk(kWDelta)));
       launches++;
       if (g->max_degree >= kWaveEdges) {
         // Hubs fold on the side stream beside the wavefront kernel (disjoint
@@ -813,17 +932,15 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
           GG_HIP(hipStreamWaitEvent(g->side, g->ev_fork, 0));
           note(kWDeltaHub,
                RunOn(g, g->side, "bc_delta_hub", 0, BcDeltaHub<T, kKahan>, dim3(g->cu_count * kBcHubGrid), dim3(kBcHubBS),
-                     static_cast<const int64_t*>(g->out_off), fold_dst, static_cast<const int32_t*>(depth),
-                     static_cast<const double*>(sigma), delta, score, comp, static_cast<const int32_t*>(hub_list),
-                     d, dc, wk(kWDeltaHub)));
+                     static_cast<const int64_t*>(g->out_off), fold_dst, next, node, score, comp,
+                     static_cast<const int32_t*>(hub_list), dc, wk(kWDeltaHub)));
           GG_HIP(hipEventRecord(g->ev_join, g->side));
           launches++;
         }
         note(kWDeltaWave,
              Run(g, "bc_delta_wave", 0, BcDeltaWave<T, kKahan>, dim3(GridFor(qn, kBS / kWave, g->cu_count * 8)),
-                 blk, static_cast<const int64_t*>(g->out_off), fold_dst, static_cast<const int32_t*>(depth),
-                 static_cast<const double*>(sigma), delta, score, comp, static_cast<const int32_t*>(wave_list), d,
-                 static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
+                 blk, static_cast<const int64_t*>(g->out_off), fold_dst, next, node, score, comp,
+                 static_cast<const int32_t*>(wave_list), static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
         if (hubs) GG_HIP(hipStreamWaitEvent(st, g->ev_join, 0));
         Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
         launches += 2;
@@ -839,8 +956,9 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   GG_HIP(hipGetLastError());
   if (g->profile) {
     // Bytes beyond the per-vertex parts credited at launch: per list entry
-    // its id and the neighbour's depth (8 B); per matched in-neighbour its
-    // sigma (8 B); per successor its sigma and delta (8 + sizeof(T) B).
+    // its id and the neighbour's depth (8 B; its level bit comes from cache);
+    // per matched in-neighbour its sigma (8 B); per successor its sigma and
+    // delta (8 + sizeof(T) B).
     const std::vector<unsigned long long> w = ReadWork(g, work, kWKinds);
     for (int kind = 0; kind < kWKinds; kind++) {
       const double per_match = kind <= kWSigmaChunks ? 8.0 : 8.0 + sizeof(T);

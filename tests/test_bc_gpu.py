@@ -132,3 +132,24 @@ def test_bc_folds_ties_and_binades(leaves):
     dg = gpu.DeviceGraph(g)
     assert np.array_equal(gpu.bc(dg, roots).scores, want)
     assert np.array_equal(gpu.bc_batch(dg, roots).scores, want)
+
+
+@pytest.mark.parametrize("n", [2, 31, 32, 33, 34, 65, 4097])
+def test_bc_level_bitmaps_and_depths(n):
+    # Paths of as many levels as the level bitmaps hold, and one more or less
+    # (deeper traversals test depths), with lists around a wavefront's length
+    # hanging off the middle.
+    print(f"[bc] path of {n}", flush=True)
+    u, v = list(range(n - 1)), list(range(1, n))
+    at = n
+    for d in (63, 64, 65, 1023, 1024, 1025):
+        u += [min(d % 7, n - 1)] * d
+        v += list(range(at, at + d))
+        at += d
+    g = Graph.from_edges(np.array(u), np.array(v))
+    roots = np.array([0, n - 1, at - 1], dtype=np.int32)
+    for order in (False, True):
+        dg = gpu.DeviceGraph(g, order_by_degree=order)
+        if not order:
+            assert np.array_equal(gpu.bc(dg, roots).scores, oracle.brandes(g, roots))
+        assert np.abs(gpu.bc(dg, roots, fp64=True).scores - oracle.brandes(g, roots, fp64=True)).max() < 1e-7
