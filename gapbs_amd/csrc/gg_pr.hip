@@ -1003,11 +1003,18 @@ __device__ __forceinline__ double PbFinish(const PbArgs<T>& a, int64_t u, T sum)
   return fabs(static_cast<double>(now) - static_cast<double>(old));
 }
 
-template <class T>
+// kLog: the LDS is sized for widths up to 2^kLog.  Both phases are streams
+// with a few dependent loads each, so the bytes in flight set their rate and
+// two 1024-thread blocks per CU beat one; up to kPbSmallLog two always fit
+// (64 KB of 8-byte words each).  Kronecker 24, FP32,
+// 2^12: the sum phase takes 752 us a launch, and 855 with the LDS of 2^14.
+constexpr int kPbSmallLog = 13;
+
+template <class T, int kLog>
 __global__ __launch_bounds__(kPbWriteBS) void PbWrite(PbArgs<T> a, const PbChunk* __restrict__ chunks) {
   using S = PbWriteShape<T>;
   constexpr int E = S::kEntries, U = S::kItems;
-  __shared__ T slice[1 << kPbMaxLog];
+  __shared__ T slice[1 << kLog];
   const PbChunk c = chunks[blockIdx.x];
   const int64_t base = int64_t(c.part) << a.lg;
   const int64_t cnt = min(int64_t(1) << a.lg, a.n - base);
@@ -1035,10 +1042,10 @@ __global__ __launch_bounds__(kPbWriteBS) void PbWrite(PbArgs<T> a, const PbChunk
   }
 }
 
-template <class T>
+template <class T, int kLog>
 __global__ __launch_bounds__(kPbSumBS) void PbSum(PbArgs<T> a, const PbChunk* __restrict__ chunks) {
   using Word = typename PbAcc<T>::Word;
-  __shared__ Word s_acc[1 << kPbMaxLog];
+  __shared__ Word s_acc[1 << kLog];
   __shared__ double s_red[kPbSumBS / kWave];
   const PbChunk c = chunks[blockIdx.x];
   const int w = 1 << a.lg;
@@ -1254,19 +1261,31 @@ __global__ __launch_bounds__(kPbBuildBS) void PbOctIndex(int64_t k, const uint32
 }
 
 // The width the Jacobi run of this precision uses (0: no blocks).  By
-// default about 4096 tiles: 2^(ceil(log2 n) - 12) vertices, from 2^10 to
-// 2^14 (measured on Kronecker graphs of 2^20 to 2^26 vertices: the
-// narrowest width with few enough tiles to keep the padding and the build
-// tables small, since narrower blocks give more bins, so fewer bins summed
-// in several chunks, and smaller LDS footprints).
+// default the narrowest of 2^10 to 2^14 with at least `want` in-entries per
+// (tile, bin) block on average: a block is padded to whole octets, so blocks
+// of a few entries are mostly padding, while narrower bins mean smaller LDS
+// footprints and fewer bins summed in several chunks.  Where degrees are
+// skewed most entries sit in few blocks and a lower average is enough.
+// Measured (FP32 / FP64 ms of a run, by width): Kronecker 22 as uploaded 2^10
+// 6.18 / 7.61 (padding 1.46), 2^11 3.20 / 5.08, 2^12 3.06 / 5.05, 2^14 3.36 /
+// 5.11; degree-ordered 2^10 3.22 / 4.83, 2^11 3.12 / 4.78, 2^12 3.37 / 5.11,
+// 2^14 4.36 / 5.83; Kronecker 20 ordered 2^10 1.10 / 1.83, 2^11 1.21 / 1.93;
+// uniform, 3 M vertices, degree 32, FP64 2^10 4.44 (padding 1.31), 2^12 3.39.
+constexpr int64_t kPbSkew = 32;  // max over average degree from which a graph counts as skewed
+constexpr int64_t kPbBlockEntries = 96, kPbBlockEntriesSkewed = 24;
 int BlockWidth(const gg_graph* g, bool fp64) {
   const int knob = g->tune.pr_blocks_log2;
   if (knob > 0) return knob;
   if (knob < 0 || g->tune.pr_segment_log2[fp64 ? 1 : 0] != 0) return 0;
   const int64_t n = g->n;
   if (n < (int64_t(1) << 20) || n > (int64_t(1) << 27)) return 0;
-  const int ceil_log2 = 64 - __builtin_clzll(static_cast<unsigned long long>(n - 1));
-  return std::min(kPbMaxLog, std::max(10, ceil_log2 - 12));
+  const int64_t want = g->max_degree * n >= kPbSkew * g->in_entries ? kPbBlockEntriesSkewed : kPbBlockEntries;
+  int lg = 10;
+  for (; lg < kPbMaxLog; lg++) {
+    const int64_t k = (n + (int64_t(1) << lg) - 1) >> lg;
+    if (k <= kPbMaxTiles && g->in_entries >= want * k * k) break;
+  }
+  return lg;
 }
 
 // The propagation-block layout, built on first use (and again when the
@@ -1478,11 +1497,12 @@ void RunPageRank(gg_graph* g, int max_iters, double epsilon, bool in_place, floa
                 residual, n, pb->lg};
     const double ent = 8.0 * pb->octets, vs = sizeof(T), ps = sizeof(Word);
     if (pb->n_write)
-      Run(g, fp64 ? "pr_blocks_write_fp64" : "pr_blocks_write", ent * (2 + vs) + vs * N, PbWrite<T>,
+      Run(g, fp64 ? "pr_blocks_write_fp64" : "pr_blocks_write", ent * (2 + vs) + vs * N, pb->lg <= kPbSmallLog ? PbWrite<T, kPbSmallLog> : PbWrite<T, kPbMaxLog>,
           dim3(static_cast<unsigned>(pb->n_write)), dim3(kPbWriteBS), a,
           static_cast<const PbChunk*>(g->ws.Get("pr.pb.wchunks", 0)));
     Run(g, fp64 ? "pr_blocks_sum_fp64" : "pr_blocks_sum",
-        ent * (2 + vs) + 0.5 * ent + N * (8 + 3 * vs) + ps * double(pb->slots << pb->lg), PbSum<T>,
+        ent * (2 + vs) + 0.5 * ent + N * (8 + 3 * vs) + ps * double(pb->slots << pb->lg),
+          pb->lg <= kPbSmallLog ? PbSum<T, kPbSmallLog> : PbSum<T, kPbMaxLog>,
         dim3(static_cast<unsigned>(pb->n_sum)), dim3(kPbSumBS), a, static_cast<const PbChunk*>(g->ws.Get("pr.pb.schunks", 0)));
     launches += pb->n_write ? 2 : 1;
     if (pb->n_multi) {
