@@ -41,15 +41,21 @@ constexpr int kDeltaLoads = 8;   // (sigma, delta) row pairs in flight per wavef
 // successors each per round into an LDS double buffer, one wavefront folds
 // them in list order.  Most hubs go to small blocks (two producers, three
 // wavefronts, 16 KB of LDS, at least seven wavefronts per SIMD: nine hubs on
-// a CU at once); hubs of at least kHubWide successors, whose fold would
-// otherwise outlast the rest of the level, go to wide blocks (fifteen
-// producers, 120 successors per round).
+// a CU at once); the largest (HubWide), whose fold would otherwise outlast
+// the rest of the level, go to wide blocks (fifteen producers, 120 successors
+// per round).
 constexpr int64_t kHubFold = 2048;
-constexpr int64_t kHubWide = 65536;
 constexpr int kHubEdges = 8;
 constexpr int kHubSmall = 2;
 constexpr int kHubLarge = 15;
 constexpr int kHubSmallBlocksPerCu = 8;
+// The cut-off for wide blocks, on a graph of m list entries: a small block
+// folds about 16 successors per microsecond, and the largest hub left to one
+// should not outlast the level's other work, which grows with m.  Measured
+// for 64 roots with cut-offs of 4096 / 16384 / 65536: Kronecker 19 8.05 /
+// 8.25 / 11.32 ms, Kronecker 22 50.8 / 48.6 / 49.9 ms; Kronecker 26 0.684 s
+// at 65536, 0.706 s at 16384.
+inline int64_t HubWide(int64_t m) { return std::min<int64_t>(65536, std::max<int64_t>(2 * kHubFold, m >> 13)); }
 
 __global__ void MbRootSigma(const int32_t* __restrict__ roots, int k, double* __restrict__ sigma) {
   const int r = threadIdx.x;
@@ -432,15 +438,15 @@ __global__ __launch_bounds__((P + 1) * kWave, P <= kHubSmall ? 7 : 1) void MbDel
   }
 }
 
-// Vertices with at least kHubFold out-edges, split at kHubWide (once per
+// Vertices with at least kHubFold out-edges, split at wide_min (once per
 // graph).
-__global__ __launch_bounds__(kMbBS) void MbHubList(const int64_t* __restrict__ off, int64_t n, int32_t* small,
-                                                   int32_t* wide, int32_t* tails) {
+__global__ __launch_bounds__(kMbBS) void MbHubList(const int64_t* __restrict__ off, int64_t n, int64_t wide_min,
+                                                   int32_t* small, int32_t* wide, int32_t* tails) {
   for (int64_t base = int64_t(blockIdx.x) * kMbBS; base < n; base += int64_t(gridDim.x) * kMbBS) {
     const int64_t v = base + threadIdx.x;
     const int64_t d = v < n ? off[v + 1] - off[v] : 0;
-    WaveAppend(d >= kHubFold && d < kHubWide, static_cast<int32_t>(v), small, tails);
-    WaveAppend(d >= kHubWide, static_cast<int32_t>(v), wide, tails + 1);
+    WaveAppend(d >= kHubFold && d < wide_min, static_cast<int32_t>(v), small, tails);
+    WaveAppend(d >= wide_min, static_cast<int32_t>(v), wide, tails + 1);
   }
 }
 
@@ -579,13 +585,14 @@ void RunBatchBrandes(gg_graph* g, const int32_t* droots, int k, float* scores, g
   // Hubs (their folds split across a block, MbDeltaHub): listed once per
   // graph, at most m / kHubFold of them.
   const int64_t max_hubs = std::min<int64_t>(n, g->out_entries / kHubFold + 1);
+  const int64_t wide_min = HubWide(g->out_entries);
   int32_t* hubs = g->Scratch<int32_t>("mb.hubs", max_hubs);
-  int32_t* wide = g->Scratch<int32_t>("mb.wide_hubs", std::min<int64_t>(n, g->out_entries / kHubWide + 1));
+  int32_t* wide = g->Scratch<int32_t>("mb.wide_hubs", std::min<int64_t>(n, g->out_entries / wide_min + 1));
   if (g->mb_hubs < 0) {
     int32_t* tails = g->Scratch<int32_t>("mb.hub_tails", 2);
     GG_HIP(hipMemsetAsync(tails, 0, 2 * sizeof(int32_t), st));
     Run(g, "msbc_hub_list", 0, MbHubList, dim3(GridFor(n, kMbBS, g->cu_count * 4)), blk,
-        static_cast<const int64_t*>(g->out_off), n, hubs, wide, tails);
+        static_cast<const int64_t*>(g->out_off), n, wide_min, hubs, wide, tails);
     int32_t h[2] = {0, 0};
     GG_HIP(hipMemcpyAsync(h, tails, sizeof(h), hipMemcpyDeviceToHost, st));
     GG_HIP(hipStreamSynchronize(st));
