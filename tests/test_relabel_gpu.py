@@ -65,3 +65,14 @@ def test_relabel_rejects_directed_and_weighted():
     with pytest.raises(gpu.GpuError) as e:
         gpu.relabel_by_degree(gpu.DeviceGraph(Graph.kronecker(8, weighted=True)))
     assert e.value.code == -95
+
+
+def test_relabel_row_lengths():
+    # Rows at and around every row-sorting tier's limit.
+    print("[relabel] row lengths", flush=True)
+    rng = np.random.default_rng(4)
+    lens = [31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1024, 2047, 2048, 2049, 3000]
+    hubs = np.arange(len(lens))
+    u = np.repeat(hubs, lens)
+    v = np.concatenate([rng.choice(np.arange(len(lens), 20000), d, replace=False) for d in lens])
+    check(Graph.from_edges(u, v))
