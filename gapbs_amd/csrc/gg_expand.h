@@ -166,7 +166,8 @@ __device__ __forceinline__ void LdsQueueInit(LdsQueue<CAP>& q) {
   __syncthreads();
 }
 
-// Wave-wide: K pushes per lane for one reservation.
+// K pushes per lane for one reservation: every active lane of the wavefront
+// calls it together.
 template <int CAP, int K>
 __device__ __forceinline__ void LdsQueuePushMany(LdsQueue<CAP>& q, const bool (&take)[K], const int32_t (&v)[K],
                                                  int32_t* gout, int32_t* gtail) {
@@ -178,14 +179,14 @@ __device__ __forceinline__ void LdsQueuePushMany(LdsQueue<CAP>& q, const bool (&
     cnt += __popcll(m[k]);
   }
   if (cnt == 0) return;
-  const int lane = LaneId();
+  const bool leader = LanesBelow(__ballot(true)) == 0;  // the first active lane
   int base = 0;
-  if (lane == 0) base = atomicAdd(&q.count, cnt);
+  if (leader) base = atomicAdd(&q.count, cnt);
   base = __builtin_amdgcn_readfirstlane(base);
   const int fit = base >= CAP ? 0 : CAP - base;
   int gbase = 0;
   if (cnt > fit) {
-    if (lane == 0) gbase = atomicAdd(gtail, cnt - fit);
+    if (leader) gbase = atomicAdd(gtail, cnt - fit);
     gbase = __builtin_amdgcn_readfirstlane(gbase);
   }
   int rank0 = 0;

@@ -196,51 +196,56 @@ struct RelaxCtx {
   int32_t fmin;
 };
 
-// Relaxes edges [b, e) of u for the lanes with `active` (distance du).
-// Called by whole groups; groups of one wavefront may diverge.
-__device__ __forceinline__ void RelaxRange(RelaxCtx& c, const Group& g, int32_t u, int64_t b, int64_t e, bool active,
+// Relaxes edges [b, e) for the lanes with `active` (distance du).  Called by
+// whole groups; groups of one wavefront may diverge.  Each kind of access is
+// issued for all kUnroll edges before the first result is used: ids,
+// distances, atomic minima, then the queue stamps.  Taking the edges one
+// after the other put two atomic round trips per improving edge in a row
+// (Kronecker 19, 16 roots: 7.3 and 4.1 ms in the two kernels, now 6.2 and 3.5).
+__device__ __forceinline__ void RelaxRange(RelaxCtx& c, const Group& g, int64_t b, int64_t e, bool active,
                                            int32_t du) {
-  (void)u;
   for (int64_t base = b; base < e; base += kUnroll) {
     int2 vw[kUnroll];
-    int32_t cur[kUnroll];
+    int32_t v[kUnroll], old[kUnroll];
+    int64_t nd[kUnroll];
+    bool imp[kUnroll], push_near[kUnroll], push_fresh[kUnroll];
+    // (entries past the end: the first edge again, dropped below)
+#pragma unroll
+    for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[base + j < e ? base + j : b];
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
-      vw[j] = base + j < e ? c.wdst[base + j] : make_int2(0, 0);
+      v[j] = vw[j].x;
+      nd[j] = static_cast<int64_t>(du) + vw[j].y;
+      old[j] = c.dist[(int64_t(v[j]) << c.lg) + g.r];
     }
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
-      cur[j] = active && base + j < e ? c.dist[(int64_t(vw[j].x) << c.lg) + g.r] : 0;
+      const bool in = active && base + j < e;
+      c.relaxed += in;
+      imp[j] = in && nd[j] < kDistInf && nd[j] < old[j];
+      if (imp[j]) old[j] = atomicMin(&c.dist[(int64_t(v[j]) << c.lg) + g.r], static_cast<int32_t>(nd[j]));
     }
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
-      if (base + j >= e) break;  // group-uniform
-      const int32_t v = vw[j].x;
-      bool imp = false, to_near = false;
-      int32_t nd32 = 0;
-      if (active) {
-        c.relaxed++;
-        const int64_t nd = static_cast<int64_t>(du) + vw[j].y;
-        if (nd < kDistInf && nd < cur[j]) {
-          nd32 = static_cast<int32_t>(nd);
-          const int32_t old = atomicMin(&c.dist[(int64_t(v) << c.lg) + g.r], nd32);
-          imp = nd32 < old;
-          to_near = imp && nd < c.hi;
-          if (imp && !to_near && nd32 < c.fmin) c.fmin = nd32;
-        }
-      }
-      const uint64_t bits = GroupBallot(g, imp);
-      const uint64_t nbits = GroupBallot(g, to_near);
-      bool push_near = false, push_fresh = false;
+      imp[j] = imp[j] && nd[j] < old[j];
+      const bool here = nd[j] < c.hi;
+      if (imp[j] && !here && nd[j] < c.fmin) c.fmin = static_cast<int32_t>(nd[j]);
+      const uint64_t bits = GroupBallot(g, imp[j]), nbits = GroupBallot(g, imp[j] && here);
+      push_near[j] = push_fresh[j] = false;
       if (bits && LaneId() == g.leader) {
         c.improved += __popcll(bits);
-        atomicOr(reinterpret_cast<unsigned long long*>(&c.chg[v]), static_cast<unsigned long long>(bits));
-        if (nbits) push_near = atomicExch(&c.stamp[v], c.near_tag) != c.near_tag;
-        if (bits & ~nbits) push_fresh = atomicExch(&c.freshstamp[v], c.fresh_tag) != c.fresh_tag;
+        atomicOr(reinterpret_cast<unsigned long long*>(&c.chg[v[j]]), static_cast<unsigned long long>(bits));
+        push_near[j] = nbits != 0;
+        push_fresh[j] = (bits & ~nbits) != 0;
       }
-      LdsQueuePush(*c.lnear, push_near, v, c.near, &c.S->near_tail);
-      LdsQueuePush(*c.lfresh, push_fresh, v, c.fresh, &c.S->fresh_tail);
     }
+#pragma unroll
+    for (int j = 0; j < kUnroll; j++) {
+      if (push_near[j]) push_near[j] = atomicExch(&c.stamp[v[j]], c.near_tag) != c.near_tag;
+      if (push_fresh[j]) push_fresh[j] = atomicExch(&c.freshstamp[v[j]], c.fresh_tag) != c.fresh_tag;
+    }
+    LdsQueuePushMany(*c.lnear, push_near, v, c.near, &c.S->near_tail);
+    LdsQueuePushMany(*c.lfresh, push_fresh, v, c.fresh, &c.S->fresh_tail);
     if (LaneId() == g.leader) c.scanned += (e - base < kUnroll ? e - base : kUnroll);
   }
 }
@@ -296,7 +301,7 @@ __device__ __forceinline__ void GroupExpand(RelaxCtx& c, const Group& g, int32_t
     }
     return;
   }
-  RelaxRange(c, g, u, b, e, active, du);
+  RelaxRange(c, g, b, e, active, du);
 }
 
 // Expands frontier vertex u with one lane, for the few roots pending there
@@ -445,7 +450,7 @@ __global__ __launch_bounds__(kBS) void SbRelaxChunks(const int2* __restrict__ wd
     const SbChunk ch = chunks[i];
     const bool active = (ch.mask >> g.r) & 1;
     const int32_t du = active ? LoadC(&dist[(int64_t(ch.u) << lg) + g.r]) : kDistInf;
-    RelaxRange(c, g, ch.u, ch.beg, ch.end, active, du);
+    RelaxRange(c, g, ch.beg, ch.end, active, du);
   }
   RelaxFlush(c, s_red, s_min);
 }
