@@ -117,3 +117,20 @@ def test_sssp_and_bfs_list_lengths(delta):
     assert np.array_equal(gpu.sssp(gpu.DeviceGraph(g), 0, delta).dist, oracle.dijkstra(g, 0))
     plain = g.strip_weights()
     assert np.array_equal(gpu.bfs(gpu.DeviceGraph(plain), 0, alpha=1).depth, oracle.bfs_depth(plain, 0))
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+@pytest.mark.parametrize("delta", [1, 7, 8, 9, 100])
+def test_sssp_light_and_heavy_edges(delta, ordered):
+    # Weights at and around the width that parts light from heavy edges, and
+    # hubs whose chunks hold both kinds.
+    print(f"[sssp] weights around 8, delta {delta}, ordered {ordered}", flush=True)
+    rng = np.random.default_rng(delta)
+    n = 6000
+    u = np.concatenate([rng.integers(0, n, 20000), np.zeros(5000, int), np.ones(300, int)])
+    v = np.concatenate([rng.integers(0, n, 20000), rng.choice(np.arange(2, n), 5000, replace=False),
+                        rng.choice(np.arange(2, n), 300, replace=False)])
+    g = Graph.from_edges(u, v, rng.choice([1, 7, 8, 9, 60], len(u)))
+    dg = gpu.DeviceGraph(g, order_by_degree=ordered)
+    for r in (0, 1, 77):
+        assert np.array_equal(gpu.sssp(dg, r, delta).dist, oracle.dijkstra(g, r))
