@@ -199,25 +199,31 @@ struct RelaxCtx {
 // Relaxes edges [b, e) for the lanes with `active` (distance du).  Called by
 // whole groups; groups of one wavefront may diverge.  Each kind of access is
 // issued for all kUnroll edges before the first result is used: ids,
-// distances, atomic minima, then the queue stamps.  Taking the edges one
-// after the other put two atomic round trips per improving edge in a row
-// (Kronecker 19, 16 roots: 7.3 and 4.1 ms in the two kernels, now 6.2 and 3.5).
+// distances, atomic minima, then the queue stamps; the next edges' ids are
+// loaded along with this step's distances.  A group's chain of round trips
+// sets the time: with two atomic round trips per improving edge in a row,
+// Kronecker 19 with 16 roots took 7.3 and 4.1 ms in the two kernels, with
+// batched atomics 6.2 and 3.5, with the ids ahead 5.8 and 3.2 (eight edges a
+// step: 6.1 and 3.6).
 __device__ __forceinline__ void RelaxRange(RelaxCtx& c, const Group& g, int64_t b, int64_t e, bool active,
                                            int32_t du) {
+  if (b >= e) return;
+  // (entries past the end: the first edge again, dropped below)
+  int2 vw[kUnroll];
+#pragma unroll
+  for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[b + j < e ? b + j : b];
   for (int64_t base = b; base < e; base += kUnroll) {
-    int2 vw[kUnroll];
     int32_t v[kUnroll], old[kUnroll];
     int64_t nd[kUnroll];
     bool imp[kUnroll], push_near[kUnroll], push_fresh[kUnroll];
-    // (entries past the end: the first edge again, dropped below)
-#pragma unroll
-    for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[base + j < e ? base + j : b];
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
       v[j] = vw[j].x;
       nd[j] = static_cast<int64_t>(du) + vw[j].y;
       old[j] = c.dist[(int64_t(v[j]) << c.lg) + g.r];
     }
+#pragma unroll
+    for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[base + kUnroll + j < e ? base + kUnroll + j : b];
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
       const bool in = active && base + j < e;
