@@ -362,6 +362,14 @@ constexpr int kWave = 64;
 
 __device__ __forceinline__ int LaneId() { return __lane_id(); }
 
+// Orders the wavefront's LDS accesses before it with those after it, lane
+// against lane (no instruction: a wavefront's LDS accesses are in order).
+__device__ __forceinline__ void WaveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ uint64_t LanesBelow(uint64_t mask) {
   return mask & ((uint64_t(1) << LaneId()) - 1);
 }

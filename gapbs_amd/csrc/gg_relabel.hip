@@ -8,8 +8,9 @@
 // The result here is byte-identical to that.
 //
 // Device steps:
-//   1. key = ~((degree << 32) | id) per vertex, radix-sorted ascending over
-//      the id bits and the degree bits (gg_sort.h): descending (degree, id);
+//   1. key = ~((degree << 32) | id) per vertex, listed from the largest id
+//      down and radix-sorted (stable) ascending over the degree bits
+//      (gg_sort.h): descending (degree, id);
 //   2. new_id[old] = rank, new offsets = exclusive scan of the sorted
 //      degrees;
 //   3. every list copied through new_id into its new row (tile expansion,
@@ -42,7 +43,7 @@ __global__ void RlZero(int32_t* p) {
 __global__ __launch_bounds__(kBS) void RlKeys(const int64_t* __restrict__ off, int64_t n, uint64_t* __restrict__ keys) {
   for (int64_t v = blockIdx.x * int64_t(kBS) + threadIdx.x; v < n; v += int64_t(gridDim.x) * kBS) {
     const uint64_t deg = static_cast<uint64_t>(off[v + 1] - off[v]);
-    keys[v] = ~((deg << 32) | static_cast<uint64_t>(v));
+    keys[n - 1 - v] = ~((deg << 32) | static_cast<uint64_t>(v));
   }
 }
 
@@ -258,11 +259,9 @@ void RankByDegree(gg_graph* g, int32_t* new_id, int32_t* old_id, int64_t* new_of
   uint64_t* tmp = g->Scratch<uint64_t>("rl.tmp", n + 1);
   const double N = static_cast<double>(n);
   Run(g, "relabel_keys", 16.0 * N, RlKeys, grid_n, blk, static_cast<const int64_t*>(g->out_off), n, keys);
-  const int id_bits = BitsFor(n > 0 ? static_cast<uint64_t>(n - 1) : 0);
   const int deg_bits = BitsFor(static_cast<uint64_t>(g->max_degree));
-  uint64_t* sorted = RadixSort(g, "rl.sort", keys, tmp, n, 0, id_bits);
-  sorted = RadixSort(g, "rl.sort", sorted, sorted == keys ? tmp : keys, n, 32, 32 + deg_bits);
-  Run(g, "relabel_ranks", (old_id ? 24.0 : 20.0) * N, RlRanks, grid_n, blk, static_cast<const uint64_t*>(sorted),
+  const uint64_t* sorted = RadixSort(g, "rl.sort", keys, tmp, n, 32, 32 + deg_bits);
+  Run(g, "relabel_ranks", (old_id ? 24.0 : 20.0) * N, RlRanks, grid_n, blk, sorted,
       n, new_id, old_id, new_off);
   DeviceScan<int64_t>(g, "rl.offscan", new_off, n + 1, static_cast<int64_t*>(nullptr));
 }

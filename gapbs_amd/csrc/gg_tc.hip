@@ -378,7 +378,7 @@ __global__ __launch_bounds__(kBS) void TcCountShort(const int64_t* __restrict__ 
     int32_t p;
     const int len = Partner(dst, fdeg, xb, deg, d, int64_t(item.pb) + lane, p).d;
     const int64_t lbeg = off[p];
-    __builtin_amdgcn_wave_barrier();
+    WaveSync();
     for (int i = 0; i < len; i++) {
       const int32_t w = dst[lbeg + i];
       int at = 0;
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(kBS) void TcCountShort(const int64_t* __restrict__ 
       count += mine[at] == w;
     }
     probes += static_cast<unsigned long long>(len);
-    __builtin_amdgcn_wave_barrier();
+    WaveSync();
   }
   FlushCounts(count, probes, counts, s_red);
 }

@@ -76,3 +76,15 @@ def test_relabel_row_lengths():
     u = np.repeat(hubs, lens)
     v = np.concatenate([rng.choice(np.arange(len(lens), 20000), d, replace=False) for d in lens])
     check(Graph.from_edges(u, v))
+
+
+@pytest.mark.parametrize("n", [1, 2, 64, 65, 1024, 4095, 4096, 4097, 8193, 12289])
+def test_relabel_sort_tiles(n):
+    # One vertex to several 4096-key tiles, whole and ragged, with many equal
+    # degrees and, from 2048 vertices, degrees of more than one digit.
+    print(f"[relabel] {n} vertices", flush=True)
+    i = np.arange(1, n, dtype=np.int32)
+    hubs = i[: n // 2] if n > 2048 else i[:0]
+    u = np.concatenate([i - 1, np.zeros(len(hubs), np.int32), [0] * (n == 1)]).astype(np.int32)
+    v = np.concatenate([i, hubs, [0] * (n == 1)]).astype(np.int32)
+    check(Graph.from_edges(u, v))
