@@ -10,27 +10,28 @@
 namespace gg {
 namespace {
 
-constexpr int kOutRoots = 8;  // roots per read-out pass: one 16-byte load of a depth row
+constexpr int kOutRoots = 8;  // roots of one 16-byte load of a depth row
 
-// depth16[v][r] -> out[j][v] of the kOutRoots roots r = r0 + j below k (-1
-// where seen has no bit r: the slot is undefined there); with new_id, out is
-// indexed by original ids.  A thread reads its vertex's 16 bytes of the row
+// depth16[v][r] -> out[r - r0][v] of the roots r0 <= r < r1, all in one group
+// of kOutRoots (-1 where seen has no bit r: the slot is undefined there); with
+// new_id, out is indexed by original ids.  A thread reads its vertex's 16 bytes of the row
 // and the stores are coalesced per root.  One root per pass read a 128-byte
 // line for 2 bytes: 17 us each for 64 roots of 2^20 vertices (1.08 ms),
 // against 0.24 ms for the eight passes.
 __global__ __launch_bounds__(kBS) void MsDepthOut(const uint16_t* __restrict__ d16, const uint64_t* __restrict__ seen,
-                                                  const int32_t* __restrict__ new_id, int64_t n, int r0, int k,
+                                                  const int32_t* __restrict__ new_id, int64_t n, int r0, int r1,
                                                   int32_t* __restrict__ out) {
+  const int group = r0 & ~(kOutRoots - 1);
   for (int64_t v = blockIdx.x * int64_t(kBS) + threadIdx.x; v < n; v += int64_t(gridDim.x) * kBS) {
     const int64_t dv = new_id ? int64_t(new_id[v]) : v;
-    const uint32_t bits = static_cast<uint32_t>(seen[dv] >> r0);
-    const uint4 w = *reinterpret_cast<const uint4*>(d16 + dv * 64 + r0);
+    const uint32_t bits = static_cast<uint32_t>(seen[dv] >> group);
+    const uint4 w = *reinterpret_cast<const uint4*>(d16 + dv * 64 + group);
     const uint32_t pair[kOutRoots / 2] = {w.x, w.y, w.z, w.w};
 #pragma unroll
     for (int j = 0; j < kOutRoots; j++) {
-      if (r0 + j >= k) break;
+      if (group + j < r0 || group + j >= r1) continue;
       const uint32_t x = (pair[j / 2] >> (16 * (j & 1))) & 0xFFFF;
-      out[j * n + v] = ((bits >> j) & 1) && x != kNoDepth ? static_cast<int32_t>(x) : -1;
+      out[(group + j - r0) * n + v] = ((bits >> j) & 1) && x != kNoDepth ? static_cast<int32_t>(x) : -1;
     }
   }
 }
@@ -64,11 +65,22 @@ extern "C" int gg_bfs_batch(gg_graph* g, const int32_t* roots, int k, int alpha,
     GG_HIP(hipGetLastError());
     FinishTiming(g, stats, wt);
     if (depths) {
-      int32_t* d32 = g->Scratch<int32_t>("ms.depth_out", n * std::min(k, kOutRoots));
-      for (int r = 0; r < k; r += kOutRoots) {
-        MsDepthOut<<<grid_n, blk, 0, st>>>(depth16, t.seen, g->new_id, n, r, k, d32);
-        GG_HIP(hipMemcpyAsync(depths + int64_t(r) * n, d32, sizeof(int32_t) * n * std::min(k - r, kOutRoots),
-                              hipMemcpyDeviceToHost, st));
+      // A pass reads out a group of roots; one root where the group's buffer
+      // (4 bytes per vertex and root) does not fit beside the graph.
+      int step = std::min(k, kOutRoots);
+      int32_t* d32 = nullptr;
+      try {
+        d32 = g->Scratch<int32_t>("ms.depth_out", n * step);
+      } catch (const Failure& e) {
+        if (e.status != GG_ENOMEM || step == 1) throw;
+        (void)hipGetLastError();
+        step = 1;
+        d32 = g->Scratch<int32_t>("ms.depth_out", n);
+      }
+      for (int r = 0; r < k; r += step) {
+        const int r1 = std::min(k, r + step);
+        MsDepthOut<<<grid_n, blk, 0, st>>>(depth16, t.seen, g->new_id, n, r, r1, d32);
+        GG_HIP(hipMemcpyAsync(depths + int64_t(r) * n, d32, sizeof(int32_t) * n * (r1 - r), hipMemcpyDeviceToHost, st));
       }
       GG_HIP(hipStreamSynchronize(st));
     }

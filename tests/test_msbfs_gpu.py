@@ -301,3 +301,21 @@ def test_batch_read_out_groups(k, ordered):
     res = gpu.bfs_batch(gpu.DeviceGraph(g, order_by_degree=ordered), roots)
     for i, r in enumerate(roots):
         assert np.array_equal(res.depths[i], oracle.bfs_depth(g, int(r)))
+
+
+def test_batch_read_out_at_the_memory_cap(monkeypatch):
+    # The cap rises in 2 MB steps until the call fits: 2^18 vertices read one
+    # root at a time through 1 MB where the 8 MB of a group of eight do not fit.
+    print("[msbfs] read-out at the cap", flush=True)
+    g = cached_graph("u18", lambda: Graph.uniform(18))
+    dg = gpu.DeviceGraph(g)
+    roots = g.pick_sources(9)
+    want = gpu.bfs_batch(gpu.DeviceGraph(g), roots).depths
+    for cap in range(2 << 20, 64 << 30, 2 << 20):
+        monkeypatch.setenv("GAPGPU_MEM_CAP_BYTES", str(cap))
+        try:
+            res = gpu.bfs_batch(dg, roots)
+            break
+        except gpu.GpuError as e:
+            assert e.code == -12
+    assert np.array_equal(res.depths, want)
