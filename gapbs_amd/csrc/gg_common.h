@@ -80,9 +80,17 @@ struct Workspace {
   size_t Bytes() const;
 };
 
+// Counts the handles alive, for what the process keeps while there are any.
+void HandleCreated();
+void HandleFreed();
+
 }  // namespace gg
 
 struct gg_graph {
+  struct Alive {
+    Alive() { gg::HandleCreated(); }
+    ~Alive() { gg::HandleFreed(); }
+  } alive;
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
@@ -211,12 +219,17 @@ void DeviceVertices(gg_graph* g, int32_t* d, int64_t k);
 // mapped too.  Synchronous.
 void CopyOutVertexI32(gg_graph* g, const int32_t* src, int32_t* host, bool ids);
 void CopyOutVertexF32(gg_graph* g, const float* src, float* host);
+// Device memory to the caller's array, on g->stream; synchronous.  Pageable
+// destinations are staged through page-locked slots (gg_readout.hip).
+void CopyToHost(gg_graph* g, void* host, const void* dev, size_t bytes);
 // Component labels in device order, each the smallest device id of its
 // component -> host, each the smallest original id of its component.
 void CopyOutComponents(gg_graph* g, const int32_t* comp, int32_t* host);
 // The same with the caller's two device work arrays of n int32 (unused, and
 // may be null, when the handle is not degree-ordered).
-void CopyOutComponentsWith(gg_graph* g, const int32_t* comp, int32_t* host, int32_t* least, int32_t* tmp);
+// Allocates nothing; the copy to the host is the runtime's unless `staged`.
+void CopyOutComponentsWith(gg_graph* g, const int32_t* comp, int32_t* host, int32_t* least, int32_t* tmp,
+                           bool staged = false);
 // The out-lists in uploaded order: g->out_dst unless the handle is
 // degree-ordered and unweighted (its rows are sorted by device id), then
 // g->fold_dst, built here on first use (device ids, each row sorted by

@@ -80,9 +80,9 @@ extern "C" int gg_bfs_batch(gg_graph* g, const int32_t* roots, int k, int alpha,
       for (int r = 0; r < k; r += step) {
         const int r1 = std::min(k, r + step);
         MsDepthOut<<<grid_n, blk, 0, st>>>(depth16, t.seen, g->new_id, n, r, r1, d32);
-        GG_HIP(hipMemcpyAsync(depths + int64_t(r) * n, d32, sizeof(int32_t) * n * (r1 - r), hipMemcpyDeviceToHost, st));
+        GG_HIP(hipGetLastError());
+        CopyToHost(g, depths + int64_t(r) * n, d32, sizeof(int32_t) * n * (r1 - r));
       }
-      GG_HIP(hipStreamSynchronize(st));
     }
     if (stats) {
       unsigned long long* sums = g->Scratch<unsigned long long>("ms.reach", 2);
@@ -235,8 +235,8 @@ extern "C" int gg_bfs_packed(gg_graph* g, const int64_t* part, int nparts, const
       int32_t* d32 = g->Scratch<int32_t>("pk.depth_out", n * R);
       PkDepthOut<<<dim3(GridFor(n * R, kBS, g->cu_count * 16)), blk, 0, st>>>(depth16, t.seen, n, dpart, nparts, R,
                                                                                 d32);
-      GG_HIP(hipMemcpyAsync(depths, d32, sizeof(int32_t) * n * R, hipMemcpyDeviceToHost, st));
-      GG_HIP(hipStreamSynchronize(st));
+      GG_HIP(hipGetLastError());
+      CopyToHost(g, depths, d32, sizeof(int32_t) * n * R);
     }
     if (stats) {
       unsigned long long* sums = g->Scratch<unsigned long long>("ms.reach", 2);

@@ -84,7 +84,7 @@ template <class T>
 void CopyOutVertex(gg_graph* g, const T* src, T* host, bool ids) {
   const int64_t n = g->n;
   if (!g->new_id) {
-    GG_HIP(hipMemcpyAsync(host, src, sizeof(T) * n, hipMemcpyDeviceToHost, g->stream));
+    CopyToHost(g, host, src, sizeof(T) * n);
   } else {
     T* tmp = g->Scratch<T>("order.out", n);
     const dim3 grid(GridFor(n, kBS, g->cu_count * 16)), blk(kBS);
@@ -100,9 +100,8 @@ void CopyOutVertex(gg_graph* g, const T* src, T* host, bool ids) {
       hipLaunchKernelGGL(OrGather<T>, grid, blk, 0, g->stream, src, static_cast<const int32_t*>(g->new_id), n, tmp);
     }
     GG_HIP(hipGetLastError());
-    GG_HIP(hipMemcpyAsync(host, tmp, sizeof(T) * n, hipMemcpyDeviceToHost, g->stream));
+    CopyToHost(g, host, tmp, sizeof(T) * n);
   }
-  GG_HIP(hipStreamSynchronize(g->stream));
 }
 
 }  // namespace
@@ -128,7 +127,8 @@ void CopyOutVertexI32(gg_graph* g, const int32_t* src, int32_t* host, bool ids) 
 
 void CopyOutVertexF32(gg_graph* g, const float* src, float* host) { CopyOutVertex<float>(g, src, host, false); }
 
-void CopyOutComponentsWith(gg_graph* g, const int32_t* comp, int32_t* host, int32_t* least, int32_t* tmp) {
+void CopyOutComponentsWith(gg_graph* g, const int32_t* comp, int32_t* host, int32_t* least, int32_t* tmp,
+                           bool staged) {
   const int64_t n = g->n;
   if (!g->new_id) {
     GG_HIP(hipMemcpyAsync(host, comp, sizeof(int32_t) * n, hipMemcpyDeviceToHost, g->stream));
@@ -142,6 +142,10 @@ void CopyOutComponentsWith(gg_graph* g, const int32_t* comp, int32_t* host, int3
   hipLaunchKernelGGL(OrComponentOut, grid, blk, 0, g->stream, comp, static_cast<const int32_t*>(least),
                      static_cast<const int32_t*>(g->new_id), n, tmp);
   GG_HIP(hipGetLastError());
+  if (staged) {
+    CopyToHost(g, host, tmp, sizeof(int32_t) * n);
+    return;
+  }
   GG_HIP(hipMemcpyAsync(host, tmp, sizeof(int32_t) * n, hipMemcpyDeviceToHost, g->stream));
   GG_HIP(hipStreamSynchronize(g->stream));
 }
@@ -152,7 +156,7 @@ void CopyOutComponents(gg_graph* g, const int32_t* comp, int32_t* host) {
     return;
   }
   CopyOutComponentsWith(g, comp, host, g->Scratch<int32_t>("order.least", g->n),
-                        g->Scratch<int32_t>("order.out", g->n));
+                        g->Scratch<int32_t>("order.out", g->n), true);
 }
 
 }  // namespace gg

@@ -809,8 +809,7 @@ extern "C" int gg_sssp_batch(gg_graph* g, const int32_t* roots, int k, int32_t d
       SbDistOut<<<dim3(GridFor(n * k, kBS, g->cu_count * 16)), blk, 0, st>>>(
           b.dist, n, k, lg, static_cast<const int32_t*>(g->new_id), out);
       GG_HIP(hipGetLastError());
-      GG_HIP(hipMemcpyAsync(dist_out, out, sizeof(int32_t) * n * k, hipMemcpyDeviceToHost, st));
-      GG_HIP(hipStreamSynchronize(st));
+      CopyToHost(g, dist_out, out, sizeof(int32_t) * n * k);
     }
     if (stats) {
       unsigned long long* acc = g->Scratch<unsigned long long>("sb.reach", 2);

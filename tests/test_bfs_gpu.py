@@ -6,6 +6,8 @@ the reference's direction schedule, the number of top-down / bottom-up
 steps and the adjacency entries examined must also equal the oracle's.
 """
 
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -200,3 +202,32 @@ def test_bfs_parent_only_matches_depth_run():
     r = int(g.pick_sources(1)[0])
     p = gpu.DOBFS(dg, r)
     assert np.array_equal(oracle.depth_from_parent(p, r), oracle.bfs_depth(g, r))
+
+
+def _tree(n):
+    i = np.arange(1, n, dtype=np.int32)
+    return Graph.from_edges(i, (i - 1) // 16)
+
+
+@pytest.mark.parametrize("n", [(1 << 19) - 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 77])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_bfs_read_out_sizes(n, ordered):
+    # Results around the 2 MB from which they are staged, and several rounds
+    # of the 1 MB slots with a ragged last one.
+    print(f"[bfs] read-out of {n} depths, ordered {ordered}", flush=True)
+    g = _tree(n)
+    res = gpu.bfs(gpu.DeviceGraph(g, order_by_degree=ordered), 5)
+    assert np.array_equal(res.depth, oracle.bfs_depth(g, 5))
+
+
+def test_bfs_read_out_from_threads():
+    # Four handles read out at the same time: one copy is staged, the others
+    # take the runtime's path.
+    print("[bfs] read-out, 4 threads", flush=True)
+    g = _tree((1 << 20) + 3)
+    handles = [gpu.DeviceGraph(g) for _ in range(4)]
+    want = [oracle.bfs_depth(g, r) for r in range(4)]
+    with ThreadPoolExecutor(4) as pool:
+        for _ in range(3):
+            got = list(pool.map(lambda i: gpu.bfs(handles[i], i).depth, range(4)))
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
