@@ -196,64 +196,93 @@ struct RelaxCtx {
   int32_t fmin;
 };
 
+// Queue pushes whose stamps are still on their way: kUnroll vertices, the
+// leader lanes' flags as bits.
+struct PendingPush {
+  int32_t v[kUnroll];
+  int32_t near_was[kUnroll], fresh_was[kUnroll];  // the stamps found
+  uint32_t near, fresh;                           // bit j: the stamp was asked for
+};
+
+__device__ __forceinline__ void PushPending(RelaxCtx& c, const PendingPush& p) {
+  bool push_near[kUnroll], push_fresh[kUnroll];
+#pragma unroll
+  for (int j = 0; j < kUnroll; j++) {
+    push_near[j] = ((p.near >> j) & 1) && p.near_was[j] != c.near_tag;
+    push_fresh[j] = ((p.fresh >> j) & 1) && p.fresh_was[j] != c.fresh_tag;
+  }
+  LdsQueuePushMany(*c.lnear, push_near, p.v, c.near, &c.S->near_tail);
+  LdsQueuePushMany(*c.lfresh, push_fresh, p.v, c.fresh, &c.S->fresh_tail);
+}
+
 // Relaxes edges [b, e) for the lanes with `active` (distance du).  Called by
-// whole groups; groups of one wavefront may diverge.  Each kind of access is
-// issued for all kUnroll edges before the first result is used: ids,
-// distances, atomic minima, then the queue stamps; the next edges' ids are
-// loaded along with this step's distances.  A group's chain of round trips
-// sets the time: with two atomic round trips per improving edge in a row,
-// Kronecker 19 with 16 roots took 7.3 and 4.1 ms in the two kernels, with
-// batched atomics 6.2 and 3.5, with the ids ahead 5.8 and 3.2 (eight edges a
-// step: 6.1 and 3.6).
+// whole groups; groups of one wavefront may diverge.  A group's chain of round
+// trips sets the time, so steps of kUnroll edges are pipelined: while a step's
+// atomic minima are on their way the next step's distances and the ids after
+// them are loaded, and a step's queue stamps are looked at one step later.
+// Kronecker 19, 16 roots, the two kernels: 7.3 and 4.1 ms with each improving
+// edge's two atomic round trips in a row, 6.2 and 3.5 with a step's atomics
+// issued together, 5.8 and 3.2 with the ids ahead, 5.3 and 2.7 as here.
 __device__ __forceinline__ void RelaxRange(RelaxCtx& c, const Group& g, int64_t b, int64_t e, bool active,
                                            int32_t du) {
   if (b >= e) return;
   // (entries past the end: the first edge again, dropped below)
-  int2 vw[kUnroll];
+  int2 vw[kUnroll], nx[kUnroll];
+  int32_t row[kUnroll];
 #pragma unroll
   for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[b + j < e ? b + j : b];
+#pragma unroll
+  for (int j = 0; j < kUnroll; j++) nx[j] = c.wdst[b + kUnroll + j < e ? b + kUnroll + j : b];
+#pragma unroll
+  for (int j = 0; j < kUnroll; j++) row[j] = c.dist[(int64_t(vw[j].x) << c.lg) + g.r];
+  PendingPush pend;
+  pend.near = pend.fresh = 0;
   for (int64_t base = b; base < e; base += kUnroll) {
-    int32_t v[kUnroll], old[kUnroll];
-    int64_t nd[kUnroll];
-    bool imp[kUnroll], push_near[kUnroll], push_fresh[kUnroll];
-#pragma unroll
-    for (int j = 0; j < kUnroll; j++) {
-      v[j] = vw[j].x;
-      nd[j] = static_cast<int64_t>(du) + vw[j].y;
-      old[j] = c.dist[(int64_t(v[j]) << c.lg) + g.r];
-    }
-#pragma unroll
-    for (int j = 0; j < kUnroll; j++) vw[j] = c.wdst[base + kUnroll + j < e ? base + kUnroll + j : b];
+    int32_t v[kUnroll], nd[kUnroll], old[kUnroll];
+    uint32_t want = 0;
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
       const bool in = active && base + j < e;
+      const int64_t d = static_cast<int64_t>(du) + vw[j].y;
+      v[j] = vw[j].x;
+      nd[j] = static_cast<int32_t>(d);
+      old[j] = row[j];
       c.relaxed += in;
-      imp[j] = in && nd[j] < kDistInf && nd[j] < old[j];
-      if (imp[j]) old[j] = atomicMin(&c.dist[(int64_t(v[j]) << c.lg) + g.r], static_cast<int32_t>(nd[j]));
+      const bool lower = in && d < kDistInf && d < row[j];
+      want |= static_cast<uint32_t>(lower) << j;
+      if (lower) old[j] = atomicMin(&c.dist[(int64_t(v[j]) << c.lg) + g.r], nd[j]);
     }
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
-      imp[j] = imp[j] && nd[j] < old[j];
+      vw[j] = nx[j];
+      row[j] = c.dist[(int64_t(vw[j].x) << c.lg) + g.r];
+    }
+#pragma unroll
+    for (int j = 0; j < kUnroll; j++) nx[j] = c.wdst[base + 2 * kUnroll + j < e ? base + 2 * kUnroll + j : b];
+    PushPending(c, pend);
+    pend.near = pend.fresh = 0;
+#pragma unroll
+    for (int j = 0; j < kUnroll; j++) {
+      const bool imp = ((want >> j) & 1) && nd[j] < old[j];
       const bool here = nd[j] < c.hi;
-      if (imp[j] && !here && nd[j] < c.fmin) c.fmin = static_cast<int32_t>(nd[j]);
-      const uint64_t bits = GroupBallot(g, imp[j]), nbits = GroupBallot(g, imp[j] && here);
-      push_near[j] = push_fresh[j] = false;
+      if (imp && !here && nd[j] < c.fmin) c.fmin = nd[j];
+      const uint64_t bits = GroupBallot(g, imp), nbits = GroupBallot(g, imp && here);
+      pend.v[j] = v[j];
       if (bits && LaneId() == g.leader) {
         c.improved += __popcll(bits);
         atomicOr(reinterpret_cast<unsigned long long*>(&c.chg[v[j]]), static_cast<unsigned long long>(bits));
-        push_near[j] = nbits != 0;
-        push_fresh[j] = (bits & ~nbits) != 0;
+        pend.near |= static_cast<uint32_t>(nbits != 0) << j;
+        pend.fresh |= static_cast<uint32_t>((bits & ~nbits) != 0) << j;
       }
     }
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
-      if (push_near[j]) push_near[j] = atomicExch(&c.stamp[v[j]], c.near_tag) != c.near_tag;
-      if (push_fresh[j]) push_fresh[j] = atomicExch(&c.freshstamp[v[j]], c.fresh_tag) != c.fresh_tag;
+      if ((pend.near >> j) & 1) pend.near_was[j] = atomicExch(&c.stamp[v[j]], c.near_tag);
+      if ((pend.fresh >> j) & 1) pend.fresh_was[j] = atomicExch(&c.freshstamp[v[j]], c.fresh_tag);
     }
-    LdsQueuePushMany(*c.lnear, push_near, v, c.near, &c.S->near_tail);
-    LdsQueuePushMany(*c.lfresh, push_fresh, v, c.fresh, &c.S->fresh_tail);
     if (LaneId() == g.leader) c.scanned += (e - base < kUnroll ? e - base : kUnroll);
   }
+  PushPending(c, pend);
 }
 
 __device__ __forceinline__ void RelaxFlush(RelaxCtx& c, unsigned long long* s_red, int32_t* s_min) {
