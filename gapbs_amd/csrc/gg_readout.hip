@@ -5,8 +5,8 @@
 // allocated: 16 MB of depths into a fresh array took 1.0 ms, three times the
 // transfer.  CopyToHost stages it through page-locked slots instead: the copy
 // engine fills a slot while a few threads move earlier ones out, faults
-// included (BFS on Kronecker 22 with its depths: 1.37 ms before, 0.99 with it).  Page-locked destinations and small results are copied
-// straight.
+// included (BFS on Kronecker 22 with its depths: 1.37 ms before, 0.99 with it).
+// Page-locked destinations and small results are copied straight.
 //
 // The slots are one per process (kSlots x kSlotBytes), taken by one copy at a
 // time -- a copy that finds them taken uses the runtime's path -- and freed
