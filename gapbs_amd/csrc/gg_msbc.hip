@@ -62,6 +62,29 @@ __global__ void MbRootSigma(const int32_t* __restrict__ roots, int k, double* __
   if (r < k) sigma[int64_t(roots[r]) * 64 + r] = 1.0;
 }
 
+// Lane j's value, j wave-uniform, in a scalar register: addresses and masks
+// made of it are scalar too.  (A shuffle goes through LDS: in the batches
+// below, each neighbour's loads waited for its shuffles.  MbDelta with 64 roots,
+// all levels: Kronecker 19 2.24 ms with shuffles, 1.33 now; Kronecker 22 21.4
+// and 11.2.)
+__device__ __forceinline__ int32_t LaneValue(int32_t x, int j) { return __builtin_amdgcn_readlane(x, j); }
+__device__ __forceinline__ uint64_t LaneValue(uint64_t x, int j) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), j));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x >> 32), j));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+__device__ __forceinline__ int64_t LaneValue(int64_t x, int j) {
+  return static_cast<int64_t>(LaneValue(static_cast<uint64_t>(x), j));
+}
+
+// Whether this lane's bit is set in the wave-uniform m.
+__device__ __forceinline__ bool MyBit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// The wavefront's index in the grid, in a scalar register.
+__device__ __forceinline__ int64_t WaveIndex() {
+  return int64_t(blockIdx.x) * (kMbBS / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+}
+
 // Pops up to B set bits of `any` (lowest first) into j[]; the rest are -1.
 // Wave-uniform.
 template <int B>
@@ -88,7 +111,7 @@ __global__ __launch_bounds__(kMbBS) void MbSigma(const int64_t* __restrict__ in_
                                                  unsigned long long* work) {
   __shared__ unsigned long long s_red[kMbBS / kWave];
   const int lane = LaneId();
-  const int64_t wave = (int64_t(blockIdx.x) * kMbBS + threadIdx.x) / kWave;
+  const int64_t wave = WaveIndex();
   const int64_t nwaves = int64_t(gridDim.x) * (kMbBS / kWave);
   unsigned long long ex = 0, pairs = 0;
   for (int64_t base = wave; base < n; base += nwaves * kWave) {
@@ -107,9 +130,9 @@ __global__ __launch_bounds__(kMbBS) void MbSigma(const int64_t* __restrict__ in_
       const int i = __builtin_ctzll(act);
       act &= act - 1;
       const int64_t v = base + i * nwaves;
-      const uint64_t fv = __shfl(fl, i);
-      const int64_t b = __shfl(bl, i), e = __shfl(el, i);
-      const bool mine = (fv >> lane) & 1;
+      const uint64_t fv = LaneValue(fl, i);
+      const int64_t b = LaneValue(bl, i), e = LaneValue(el, i);
+      const bool mine = MyBit(fv);
       double* row = sigma + v * 64;
       if (e - b >= kHeavyEdges) {
         if (mine) row[lane] = 0.0;
@@ -134,9 +157,9 @@ __global__ __launch_bounds__(kMbBS) void MbSigma(const int64_t* __restrict__ in_
           for (int t = 0; t < kSigmaLoads; t++) {
             x[t] = 0.0;
             if (j[t] >= 0) {
-              const uint64_t m = __shfl(ml, j[t]);
-              const int32_t u = __shfl(ul, j[t]);
-              if ((m >> lane) & 1) x[t] = sigma[int64_t(u) * 64 + lane];
+              const uint64_t m = LaneValue(ml, j[t]);
+              const int32_t u = LaneValue(ul, j[t]);
+              if (MyBit(m)) x[t] = sigma[int64_t(u) * 64 + lane];
             }
           }
 #pragma unroll
@@ -161,7 +184,7 @@ __global__ __launch_bounds__(kMbBS) void MbSigmaHeavy(const int32_t* __restrict_
                                                       unsigned long long* work) {
   __shared__ unsigned long long s_red[kMbBS / kWave];
   const int lane = LaneId();
-  const int64_t wave = (int64_t(blockIdx.x) * kMbBS + threadIdx.x) / kWave;
+  const int64_t wave = WaveIndex();
   const int64_t nwaves = int64_t(gridDim.x) * (kMbBS / kWave);
   unsigned long long ex = 0, pairs = 0;
   for (int64_t it = wave; it < nch; it += nwaves) {
@@ -187,9 +210,9 @@ __global__ __launch_bounds__(kMbBS) void MbSigmaHeavy(const int32_t* __restrict_
         for (int t = 0; t < kSigmaLoads; t++) {
           x[t] = 0.0;
           if (j[t] >= 0) {
-            const uint64_t m = __shfl(ml, j[t]);
-            const int32_t u = __shfl(ul, j[t]);
-            if ((m >> lane) & 1) x[t] = sigma[int64_t(u) * 64 + lane];
+            const uint64_t m = LaneValue(ml, j[t]);
+            const int32_t u = LaneValue(ul, j[t]);
+            if (MyBit(m)) x[t] = sigma[int64_t(u) * 64 + lane];
           }
         }
 #pragma unroll
@@ -228,7 +251,7 @@ __device__ __forceinline__ int64_t DeltaVertex(const int32_t* __restrict__ dst, 
                                                const double* __restrict__ sigma, T* __restrict__ delta, int64_t u,
                                                uint64_t fu, int64_t b, int64_t e, unsigned long long& pairs) {
   const int lane = LaneId();
-  const bool mine = (fu >> lane) & 1;
+  const bool mine = MyBit(fu);
   const double su = mine ? sigma[u * 64 + lane] : 1.0;
   T acc = T(0);
   int32_t vn = 0;
@@ -261,9 +284,9 @@ __device__ __forceinline__ int64_t DeltaVertex(const int32_t* __restrict__ dst, 
         sv[t] = 1.0;
         dv[t] = T(0);
         if (j[t] >= 0) {
-          const uint64_t m = __shfl(ml, j[t]);
-          const int32_t v = __shfl(vl, j[t]);
-          on[t] = (m >> lane) & 1;
+          const uint64_t m = LaneValue(ml, j[t]);
+          const int32_t v = LaneValue(vl, j[t]);
+          on[t] = MyBit(m);
           if (on[t]) {
             sv[t] = sigma[int64_t(v) * 64 + lane];
             dv[t] = delta[int64_t(v) * 64 + lane];
@@ -292,7 +315,7 @@ __global__ __launch_bounds__(kMbBS) void MbDelta(const int64_t* __restrict__ off
                                                  unsigned long long* work) {
   __shared__ unsigned long long s_red[kMbBS / kWave];
   const int lane = LaneId();
-  const int64_t wave = (int64_t(blockIdx.x) * kMbBS + threadIdx.x) / kWave;
+  const int64_t wave = WaveIndex();
   const int64_t nwaves = int64_t(gridDim.x) * (kMbBS / kWave);
   unsigned long long ex = 0, pairs = 0;
   for (int64_t base = wave; base < n; base += nwaves * kWave) {
@@ -313,8 +336,8 @@ __global__ __launch_bounds__(kMbBS) void MbDelta(const int64_t* __restrict__ off
       const int i = __builtin_ctzll(act);
       act &= act - 1;
       ex += static_cast<unsigned long long>(
-          DeltaVertex<T>(dst, next, sigma, delta, base + i * nwaves, __shfl(fl, i), __shfl(bl, i), __shfl(el, i),
-                         pairs));
+          DeltaVertex<T>(dst, next, sigma, delta, base + i * nwaves, LaneValue(fl, i), LaneValue(bl, i),
+                         LaneValue(el, i), pairs));
     }
   }
   ex = BlockSum<kMbBS>(lane == 0 ? ex : 0ull, s_red);
@@ -355,7 +378,7 @@ __global__ __launch_bounds__((P + 1) * kWave, P <= kHubSmall ? 7 : 1) void MbDel
     const int64_t e = next ? off[u + 1] : b;  // deepest level: no successors
     const int64_t rounds = (e - b + kHubRound - 1) / kHubRound;
     if (wid < P) {
-      const double su = ((fu >> lane) & 1) ? sigma[u * 64 + lane] : 1.0;
+      const double su = MyBit(fu) ? sigma[u * 64 + lane] : 1.0;
       const int64_t mine = b + wid * kHubEdges;  // slot 0 of round 0
       // Lane j < kHubEdges: successor slot j of round k (any in-range entry
       // past the end; such slots are dropped below).
@@ -379,9 +402,9 @@ __global__ __launch_bounds__((P + 1) * kWave, P <= kHubSmall ? 7 : 1) void MbDel
         uint32_t on = 0;
 #pragma unroll
         for (int j = 0; j < kHubEdges; j++) {
-          const int32_t v = __shfl(v_cur, j);
-          const uint64_t m = __shfl(m_cur, j) & fu;
-          const bool o = first + j < e && ((m >> lane) & 1);
+          const int32_t v = LaneValue(v_cur, j);
+          const uint64_t m = LaneValue(m_cur, j) & fu;
+          const bool o = MyBit(first + j < e ? m : 0);
           const int64_t row = (o ? int64_t(v) : u) * 64 + lane;
           sv[j] = sigma[row];
           dv[j] = delta[row];
