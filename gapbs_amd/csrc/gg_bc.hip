@@ -51,6 +51,7 @@ constexpr int64_t kWaveEdges = 64;   // vertices with this many edges use a wave
 constexpr int64_t kSigmaChunk = 1024;  // ... per this many (sigma pull)
 constexpr int kThreadUnroll = 4;     // edges in flight per thread below that
 constexpr int kBcWaveUnroll = 4;     // 64-edge runs per wavefront step
+constexpr int32_t kSideLevel = 65536;  // vertices of a level from which its kernels take three streams
 constexpr int64_t kBcHubEdges = 4096;  // ... and with this many, a block (BcDeltaHub)
 constexpr int kBcHubProducers = 15;
 constexpr int kBcHubUnroll = 4;  // 64-edge runs per producer wavefront and round
@@ -449,27 +450,78 @@ __device__ __forceinline__ void AddScore(double* score, double*, int32_t u, doub
   score[u] = __dadd_rn(score[u], d);
 }
 
-// Thread per vertex below kWaveEdges edges; larger vertices are listed for
-// BcDeltaWave, and those with kBcHubEdges or more for BcDeltaHub.
+// The level's vertices of kWaveEdges or more edges, listed for BcDeltaWave, and
+// those of kBcHubEdges or more for BcDeltaHub, each in the queue's order within
+// a block's tile.  A list of its own, ahead of the level's work, lets the three
+// dependency kernels run side by side; one reservation per tile, because
+// additions to a list's one counter follow each other at 12 ns.
+constexpr int kListRows = 8;
+constexpr int kListTile = kBS * kListRows;
+__global__ __launch_bounds__(kBS) void BcDeltaLists(const int64_t* __restrict__ off, const int32_t* __restrict__ queue,
+                                                    int32_t qb, int32_t qn, int32_t* __restrict__ wave_list,
+                                                    int32_t* __restrict__ hub_list, BcCounters* c) {
+  constexpr int kWaves = kBS / kWave;
+  __shared__ int32_t s_at[2][kWaves];  // a wavefront's entries in each list, then their place
+  const int lane = LaneId(), wid = threadIdx.x / kWave;
+  for (int64_t base = int64_t(blockIdx.x) * kListTile; base < qn; base += int64_t(gridDim.x) * kListTile) {
+    const int64_t first = base + wid * (kListRows * kWave) + lane;
+    int32_t u[kListRows];
+    int64_t d[kListRows];
+#pragma unroll
+    for (int j = 0; j < kListRows; j++) u[j] = queue[qb + (first + j * kWave < qn ? first + j * kWave : qn - 1)];
+#pragma unroll
+    for (int j = 0; j < kListRows; j++) d[j] = off[u[j] + 1] - off[u[j]];
+    int nw = 0, nh = 0;
+#pragma unroll
+    for (int j = 0; j < kListRows; j++) {
+      if (first + j * kWave >= qn) d[j] = 0;
+      nw += __popcll(__ballot(d[j] >= kWaveEdges && d[j] < kBcHubEdges));
+      nh += __popcll(__ballot(d[j] >= kBcHubEdges));
+    }
+    if (lane == 0) {
+      s_at[0][wid] = nw;
+      s_at[1][wid] = nh;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      int32_t sum = 0;
+      for (int w = 0; w < kWaves; w++) sum += s_at[threadIdx.x][w];
+      int32_t at = sum ? atomicAdd(threadIdx.x ? &c->nhub : &c->nwave, sum) : 0;
+      for (int w = 0; w < kWaves; w++) {
+        const int32_t mine = s_at[threadIdx.x][w];
+        s_at[threadIdx.x][w] = at;
+        at += mine;
+      }
+    }
+    __syncthreads();
+    int32_t aw = s_at[0][wid], ah = s_at[1][wid];
+#pragma unroll
+    for (int j = 0; j < kListRows; j++) {
+      const bool wave = d[j] >= kWaveEdges && d[j] < kBcHubEdges, hub = d[j] >= kBcHubEdges;
+      const uint64_t mw = __ballot(wave), mh = __ballot(hub);
+      if (wave) wave_list[aw + __popcll(LanesBelow(mw))] = u[j];
+      if (hub) hub_list[ah + __popcll(LanesBelow(mh))] = u[j];
+      aw += __popcll(mw);
+      ah += __popcll(mh);
+    }
+    __syncthreads();  // read by all before the next tile's counts
+  }
+}
+
+// Thread per vertex below kWaveEdges edges (the others: BcDeltaLists).
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBS) void BcDelta(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
                                                OnLevel next, BcNode<T>* node, T* __restrict__ score,
                                                T* __restrict__ comp, const int32_t* __restrict__ queue, int32_t qb,
-                                               int32_t qn, int32_t* __restrict__ wave_list,
-                                               int32_t* __restrict__ hub_list, BcCounters* c,
-                                               unsigned long long* work) {
+                                               int32_t qn, unsigned long long* work) {
   __shared__ unsigned long long s_red[kBS / kWave];
   unsigned long long ent = 0, mat = 0;
   for (int64_t base = int64_t(blockIdx.x) * kBS; base < qn; base += int64_t(gridDim.x) * kBS) {
     const int64_t i = base + threadIdx.x;
-    bool big = false, hub = false;
-    int32_t u = 0;
     if (i < qn) {
-      u = queue[qb + i];
+      const int32_t u = queue[qb + i];
       const int64_t b = off[u], e = off[u + 1];
-      big = e - b >= kWaveEdges;
-      hub = e - b >= kBcHubEdges;
-      if (!big) {
+      if (e - b < kWaveEdges) {
         const double su = node[u].sigma;
         typename AccFor<T, kKahan>::Type acc = AccFor<T, kKahan>::Type::Zero();
         for (int64_t k = b; k < e; k += kThreadUnroll) {
@@ -495,8 +547,6 @@ __global__ __launch_bounds__(kBS) void BcDelta(const int64_t* __restrict__ off, 
         AddScore<kKahan>(score, comp, u, d);
       }
     }
-    WaveAppend(big && !hub, u, wave_list, &c->nwave);
-    WaveAppend(hub, u, hub_list, &c->nhub);
   }
   WorkAdd(work, BlockSum<kBS>(ent, s_red), BlockSum<kBS>(mat, s_red));
 }
@@ -965,19 +1015,28 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
       const int32_t qb = bounds[d], qn = bounds[d + 1] - bounds[d];
       // (below the deepest level nothing is marked: no bitmap, no depth)
       const OnLevel next = d < level ? on_level(d + 1) : OnLevel{nullptr, depth, d + 1};
-      note(kWDelta, Run(g, "bc_delta", (16.0 + 2 * sizeof(T) + 8.0) * qn, BcDelta<T, kKahan>,
-                        dim3(GridFor(qn, kBS, g->cu_count * 16)), blk, static_cast<const int64_t*>(g->out_off),
-                        fold_dst, next, node, score, comp, static_cast<const int32_t*>(queue), qb, qn, wave_list,
-                        hub_list, dc, wk(kWDelta)));
-      launches++;
-      if (g->max_degree >= kWaveEdges) {
-        // Hubs fold on the side stream beside the wavefront kernel (disjoint
-        // vertices; both only read level d + 1); both finish before the
-        // list is cleared.
-        const bool hubs = g->max_degree >= kBcHubEdges;
-        if (hubs) {
+      auto delta = [&] {
+        note(kWDelta, Run(g, "bc_delta", (16.0 + 2 * sizeof(T) + 8.0) * qn, BcDelta<T, kKahan>,
+                          dim3(GridFor(qn, kBS, g->cu_count * 16)), blk, static_cast<const int64_t*>(g->out_off),
+                          fold_dst, next, node, score, comp, static_cast<const int32_t*>(queue), qb, qn, wk(kWDelta)));
+        launches++;
+      };
+      if (!longs) {
+        delta();
+      } else {
+        // The three kernels write disjoint vertices and only read level
+        // d + 1, so they run on three streams; all finish before the lists
+        // are cleared.  A level below kSideLevel is over sooner than the
+        // second fork costs.
+        const bool hubs = g->max_degree >= kBcHubEdges, side_wave = qn >= kSideLevel;
+        Run(g, "bc_delta_lists", 0, BcDeltaLists, dim3(GridFor(qn, kListTile, g->cu_count * 8)), blk,
+            static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(queue), qb, qn, wave_list, hub_list,
+            dc);
+        if (hubs || side_wave) {
           EnsureSideStream(g);
           GG_HIP(hipEventRecord(g->ev_fork, st));
+        }
+        if (hubs) {
           GG_HIP(hipStreamWaitEvent(g->side, g->ev_fork, 0));
           note(kWDeltaHub,
                RunOn(g, g->side, "bc_delta_hub", 0, BcDeltaHub<T, kKahan>, dim3(g->cu_count * kBcHubGrid), dim3(kBcHubBS),
@@ -986,11 +1045,17 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
           GG_HIP(hipEventRecord(g->ev_join, g->side));
           launches++;
         }
+        hipStream_t ws = side_wave ? g->side2 : st;
+        if (side_wave) GG_HIP(hipStreamWaitEvent(ws, g->ev_fork, 0));
         note(kWDeltaWave,
-             Run(g, "bc_delta_wave", 0, BcDeltaWave<T, kKahan>, dim3(GridFor(qn, kBS / kWave, g->cu_count * 8)),
-                 blk, static_cast<const int64_t*>(g->out_off), fold_dst, next, node, score, comp,
-                 static_cast<const int32_t*>(wave_list), static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
+             RunOn(g, ws, "bc_delta_wave", 0, BcDeltaWave<T, kKahan>, dim3(GridFor(qn, kBS / kWave, g->cu_count * 8)),
+                   blk, static_cast<const int64_t*>(g->out_off), fold_dst, next, node, score, comp,
+                   static_cast<const int32_t*>(wave_list), static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
+        if (side_wave) GG_HIP(hipEventRecord(g->ev_join2, ws));
+        launches++;
+        delta();
         if (hubs) GG_HIP(hipStreamWaitEvent(st, g->ev_join, 0));
+        if (side_wave) GG_HIP(hipStreamWaitEvent(st, g->ev_join2, 0));
         Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
         launches += 2;
       }

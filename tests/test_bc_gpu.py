@@ -153,3 +153,17 @@ def test_bc_level_bitmaps_and_depths(n):
         if not order:
             assert np.array_equal(gpu.bc(dg, roots).scores, oracle.brandes(g, roots))
         assert np.abs(gpu.bc(dg, roots, fp64=True).scores - oracle.brandes(g, roots, fp64=True)).max() < 1e-7
+
+
+@pytest.mark.parametrize("width", [2047, 2049, 70000])
+def test_bc_delta_lists(width):
+    # Levels of one and several list tiles, and one above the size from which
+    # the three dependency kernels take three streams; every 50th vertex of
+    # the level has a list for the wavefront kernel, one for the hub kernel.
+    print(f"[bc] level of {width}", flush=True)
+    mid = np.arange(1, 1 + width)
+    par = np.concatenate([np.repeat(mid[::50], 70), np.full(5000, mid[7])])
+    leaf = np.arange(len(par)) + 1 + width
+    g = Graph.from_edges(np.concatenate([np.zeros(width, int), par]), np.concatenate([mid, leaf]))
+    roots = np.array([0, int(mid[3]), int(leaf[-1])], dtype=np.int32)
+    assert np.array_equal(gpu.bc(gpu.DeviceGraph(g), roots).scores, oracle.brandes(g, roots))
