@@ -1261,29 +1261,34 @@ __global__ __launch_bounds__(kPbBuildBS) void PbOctIndex(int64_t k, const uint32
 }
 
 // The width the Jacobi run of this precision uses (0: no blocks).  By
-// default the narrowest of 2^10 to 2^14 with at least `want` in-entries per
-// (tile, bin) block on average: a block is padded to whole octets, so blocks
-// of a few entries are mostly padding, while narrower bins mean smaller LDS
-// footprints and fewer bins summed in several chunks.  Where degrees are
-// skewed most entries sit in few blocks and a lower average is enough.
+// default the narrowest of 2^10 to 2^14 with at most kPbTiles tiles and at
+// least `want` in-entries per (tile, bin) block on average: a block is padded
+// to whole octets, so blocks of a few entries are mostly padding, while
+// narrower bins mean smaller LDS footprints and fewer bins summed in several
+// chunks.  Where degrees are skewed most entries sit in few blocks and a lower
+// average is enough, lower still when the ids follow the degrees.
 // Measured (FP32 / FP64 ms of a run, by width): Kronecker 22 as uploaded 2^10
 // 6.18 / 7.61 (padding 1.46), 2^11 3.20 / 5.08, 2^12 3.06 / 5.05, 2^14 3.36 /
 // 5.11; degree-ordered 2^10 3.22 / 4.83, 2^11 3.12 / 4.78, 2^12 3.37 / 5.11,
 // 2^14 4.36 / 5.83; Kronecker 20 ordered 2^10 1.10 / 1.83, 2^11 1.21 / 1.93;
-// uniform, 3 M vertices, degree 32, FP64 2^10 4.44 (padding 1.31), 2^12 3.39.
+// uniform, 3 M vertices, degree 32, FP64 2^10 4.44 (padding 1.31), 2^12 3.39;
+// uniform 24 2^12 11.9 / 20.0, 2^13 10.4 / 19.1, 2^14 12.8 / 20.1; uniform 25
+// 2^13 21.2 / 38.8, 2^14 21.8 / 37.1.
 constexpr int64_t kPbSkew = 32;  // max over average degree from which a graph counts as skewed
-constexpr int64_t kPbBlockEntries = 96, kPbBlockEntriesSkewed = 24;
+constexpr int64_t kPbBlockEntries = 60, kPbBlockEntriesSkewed = 24, kPbBlockEntriesOrdered = 6;
+constexpr int64_t kPbTiles = 4096;
 int BlockWidth(const gg_graph* g, bool fp64) {
   const int knob = g->tune.pr_blocks_log2;
   if (knob > 0) return knob;
   if (knob < 0 || g->tune.pr_segment_log2[fp64 ? 1 : 0] != 0) return 0;
   const int64_t n = g->n;
   if (n < (int64_t(1) << 20) || n > (int64_t(1) << 27)) return 0;
-  const int64_t want = g->max_degree * n >= kPbSkew * g->in_entries ? kPbBlockEntriesSkewed : kPbBlockEntries;
+  const bool skewed = g->max_degree * n >= kPbSkew * g->in_entries;
+  const int64_t want = !skewed ? kPbBlockEntries : g->new_id ? kPbBlockEntriesOrdered : kPbBlockEntriesSkewed;
   int lg = 10;
   for (; lg < kPbMaxLog; lg++) {
     const int64_t k = (n + (int64_t(1) << lg) - 1) >> lg;
-    if (k <= kPbMaxTiles && g->in_entries >= want * k * k) break;
+    if (k <= kPbTiles && g->in_entries >= want * k * k) break;
   }
   return lg;
 }
