@@ -37,6 +37,7 @@
 //     carrying a float compensation term; GG_BC_FP64: double dependencies
 //     and scores.
 #include <algorithm>
+#include <type_traits>
 
 #include "gg_common.h"
 #include "gg_expand.h"
@@ -685,15 +686,30 @@ __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict
         const int h = (k - 1) & 1;
         for (int p = 0; p < kBcHubProducers; p++) {
           const int cnt = counts[h][p];
-          double t[kBcHubUnroll];
-          uint64_t m[kBcHubUnroll];
+          if constexpr (std::is_same_v<decltype(acc), RefAcc<float>>) {
+            double t[kBcHubUnroll];
+            uint64_t m[kBcHubUnroll];
 #pragma unroll
-          for (int r = 0; r < kBcHubUnroll; r++) {
-            const int left = cnt - r * kWave;  // of this run
-            t[r] = lane < left ? terms[h][p][r * kWave + lane] : 0.0;
-            m[r] = left >= kWave ? ~uint64_t(0) : left > 0 ? (uint64_t(1) << left) - 1 : 0;
+            for (int r = 0; r < kBcHubUnroll; r++) {
+              const int left = cnt - r * kWave;  // of this run
+              t[r] = lane < left ? terms[h][p][r * kWave + lane] : 0.0;
+              m[r] = left >= kWave ? ~uint64_t(0) : left > 0 ? (uint64_t(1) << left) - 1 : 0;
+            }
+            FoldRuns(acc, t, m);
+          } else {
+            // One after another: every lane reads the same term, eight ahead
+            // of the ordered fold (taking them lane by lane from a register
+            // costs several times an addition each).
+            int j = 0;
+            for (; j + 8 <= cnt; j += 8) {
+              double t[8];
+#pragma unroll
+              for (int q = 0; q < 8; q++) t[q] = terms[h][p][j + q];
+#pragma unroll
+              for (int q = 0; q < 8; q++) acc.Add(t[q]);
+            }
+            for (; j < cnt; j++) acc.Add(terms[h][p][j]);
           }
-          FoldRuns(acc, t, m);
         }
       }
       __syncthreads();
