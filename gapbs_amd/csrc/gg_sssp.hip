@@ -47,6 +47,12 @@ constexpr int kQueueCap = 2048;
 constexpr int32_t kDistInf = INT32_MAX / 2;
 constexpr int kStripes = 64;
 constexpr int64_t kWindow = 8;  // buckets per mid window
+// Entries per vertex from which heavy edges are relaxed apart.  Graphs of lower
+// degree have few edges a bucket and many buckets, and each bucket's extra
+// launch costs more than the relaxations it saves: a 122 x 122 grid, delta 256,
+// weights to 1000: 3.6 ms without, 4.3 with; directed R-MAT, 8 k vertices of
+// degree 8, delta 16: 3.3 without, 2.2 with.
+constexpr int64_t kSplitDegree = 6;
 // Grid caps of the per-bucket kernels, in blocks per CU.  Bucket frontiers
 // and piles are often a few hundred thousand entries; many small blocks keep
 // more relaxations and row reads in flight than a few blocks looping over
@@ -422,7 +428,7 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
       GG_HIP(hipStreamSynchronize(st));
       g->max_weight = h;
     }
-    const bool split = g->max_weight >= delta;
+    const bool split = g->max_weight >= delta && g->out_entries >= kSplitDegree * n;
     int32_t* settled = split ? g->Scratch<int32_t>("sssp.settled", n + 64) : nullptr;
     int32_t* setstamp = split ? g->Scratch<int32_t>("sssp.setstamp", n) : nullptr;
 
