@@ -802,12 +802,13 @@ __global__ __launch_bounds__(kBS) void BcLevelScatter(const int32_t* __restrict_
     });
 }
 
-// Zeroes the level counts and bitmap words.
+// Zeroes the level counts and bitmap words.  (There can be one level more
+// than the grid has threads: the search's last, empty step counts as one.)
 __global__ __launch_bounds__(kBS) void BcLevelClear(int32_t* __restrict__ counts, int nlev,
                                                     uint64_t* __restrict__ bits, int64_t words) {
-  const int64_t i0 = blockIdx.x * int64_t(kBS) + threadIdx.x;
-  if (i0 < nlev) counts[i0] = 0;
-  for (int64_t i = i0; i < words; i += int64_t(gridDim.x) * kBS) bits[i] = 0;
+  const int64_t i0 = blockIdx.x * int64_t(kBS) + threadIdx.x, stride = int64_t(gridDim.x) * kBS;
+  for (int64_t i = i0; i < nlev; i += stride) counts[i] = 0;
+  for (int64_t i = i0; i < words; i += stride) bits[i] = 0;
 }
 
 __global__ __launch_bounds__(kBS) void BcClearReduce(BcCounters* c) {

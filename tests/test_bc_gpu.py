@@ -155,6 +155,24 @@ def test_bc_level_bitmaps_and_depths(n):
         assert np.abs(gpu.bc(dg, roots, fp64=True).scores - oracle.brandes(g, roots, fp64=True)).max() < 1e-7
 
 
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("n", [255, 256, 257, 512, 3840])
+def test_bc_as_many_levels_as_vertices(n, directed):
+    # A bare path from its end, and a directed cycle: the search's steps are
+    # one more than the vertices (the last finds nothing), so at a multiple of
+    # the block size one level count more than there are threads per vertex is
+    # to be cleared.  A freed handle's counts come before, whose memory the new
+    # handle may be given.
+    print(f"[bc] {n} vertices in a row, directed {directed}", flush=True)
+    before = gpu.DeviceGraph(Graph.from_edges(np.arange(4000), np.arange(1, 4001)))
+    gpu.bc(before, [0])
+    before.free()
+    u = np.arange(n if directed else n - 1)
+    g = Graph.from_edges(u, (u + 1) % n, symmetrize=not directed)
+    roots = np.array([0, n - 1], dtype=np.int32)
+    assert np.array_equal(gpu.bc(gpu.DeviceGraph(g), roots).scores, oracle.brandes(g, roots))
+
+
 @pytest.mark.parametrize("width", [2047, 2049, 70000])
 def test_bc_delta_lists(width):
     # Levels of one and several list tiles, and one above the size from which
