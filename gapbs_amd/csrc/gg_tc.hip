@@ -21,6 +21,8 @@
 //     (block prefix sums; no atomics), long lists and short lists apart;
 //   * TcNarrow: the ids of N+(x) below 2^16 as 16-bit values, packed;
 //   * TcCountLong: a block per item, d+(x) >= kLongList, the set in LDS bits;
+//     where most ids are above 2^16, TcCountHash instead, the set in LDS hash
+//     tables (and no TcNarrow);
 //   * TcCountShort: a wavefront per item, the set a sorted LDS array.
 // Counts are summed per block and added to 64 striped counters.
 #include "gg_common.h"
@@ -40,7 +42,7 @@ constexpr int kShortPartners = kWave;  // partners per short item, one per lane
 // kFilter bits (id mod kFilter) and a hit there is checked against the list.
 // kExact is where 16-bit ids end: on a degree-ordered graph nearly every
 // probed id is a hub's (Kronecker 21: 98.6% below 2^16), so the probe streams
-// are 2 B per entry.  12 KB of bits and 6 KB of partner lists leave eight
+// are 2 B per entry.  12 KB of bits and 4 KB of partner lists leave eight
 // 256-thread blocks, every wavefront slot, per CU.
 constexpr int kExact = 1 << 16;
 constexpr int kFilter = 1 << 15;
@@ -50,6 +52,19 @@ static_assert(kExact % kFilter == 0, "SetBit ORs the shared bit's index into kEx
 constexpr int kUnroll = 3;        // loads of a probe list in flight per lane,
 constexpr int kLists = 4;         // for this many lists
 constexpr int kCountBlocksPerCu = 64;
+// TcCountHash: entries of N+(x) staged at a time, table slots (load factor
+// <= 1/2) and list entries in flight per thread.
+constexpr int kSetSlice = 2048;
+constexpr int kTable = 2 * kSetSlice;
+constexpr int kHashUnroll = 4;
+constexpr unsigned kSliceWays = 4;  // blocks per item where a list can have several slices
+// Share of the forward entries below kExact from which TcCountLong counts the
+// long lists.  The whole call in ms, with it / with TcCountHash, by the share
+// of entries at kExact or above: Kronecker 17, degree 64 (25%) 4.4 / 6.3, and
+// degree 32 1.09 / 1.05; uniform 2^17, degree 256 (25%) 2.7 / 4.4; Kronecker
+// 18 (55%) 3.6 / 2.1; uniform 2^18, degree 256 (56%) 9.0 / 8.5; Kronecker 19
+// (77%) 11.9 / 5.0.
+constexpr double kBitsShare = 0.5;
 
 // d+(x), and how many of the entries are below kExact.
 struct alignas(8) TcDegrees {
@@ -158,7 +173,7 @@ __global__ __launch_bounds__(kBS) void TcItemScan(unsigned long long* span_items
   }
 }
 
-// The items, and every vertex's first 16-bit id.
+// The items, and (low_off non-null) every vertex's first 16-bit id.
 __global__ __launch_bounds__(kBS) void TcItemFill(const int64_t* __restrict__ off,
                                                   const TcDegrees* __restrict__ fdeg, int64_t n,
                                                   const unsigned long long* __restrict__ span_base,
@@ -186,7 +201,7 @@ __global__ __launch_bounds__(kBS) void TcItemFill(const int64_t* __restrict__ of
     }
     const unsigned long long nlow = static_cast<unsigned long long>(f.low);
     const unsigned long long pos = base[2] + BlockScan64(nlow, &total, s_scan) - nlow;
-    if (x < hi) low_off[x] = static_cast<int64_t>(pos);
+    if (low_off && x < hi) low_off[x] = static_cast<int64_t>(pos);
     base[2] += total;
   }
 }
@@ -356,6 +371,91 @@ __global__ __launch_bounds__(kBS) void TcCountLong(const int64_t* __restrict__ o
   FlushCounts(total, probes, counts, s_red);
 }
 
+// Long lists where most ids have no bit of their own.  The block stages N+(x)
+// kSetSlice entries at a time in an LDS hash table and probes it with all of
+// the item's lists, laid out as one flat range (block prefix sum, owner by
+// binary search).  The slices of a list are shared out among gridDim.y blocks,
+// or the largest hubs outlast the launch (Kronecker 18, the whole call: 3.1 ms
+// with one block, 2.05 with four, 1.95 with eight).  A slice holds the sorted
+// values [lo_w, hi_w]; probes outside skip the table.  In TcCountLong such ids
+// share kFilter bits, one wavefront walks a list of them at a time, and where
+// N+(x) fills the shared bits every probe is a binary search in memory:
+// Kronecker 21 as uploaded (94% of the entries at 2^16 or above) 90.3 ms, 37.2
+// here; uniform 2^22, degree 64 (97%) 36.4 and 14.5.
+__device__ __forceinline__ uint32_t Hash(int32_t w, uint32_t mask) {
+  return (static_cast<uint32_t>(w) * 2654435761u >> 7) & mask;
+}
+
+__global__ __launch_bounds__(kBS) void TcCountHash(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
+                                                   const TcDegrees* __restrict__ fdeg,
+                                                   const TcItem* __restrict__ items, int64_t nitems,
+                                                   unsigned long long* counts) {
+  __shared__ int32_t table[kTable];
+  __shared__ int64_t s_beg[kLongPartners];
+  __shared__ int s_pre[kLongPartners];
+  __shared__ int s_scan[kBS / kWave];
+  __shared__ unsigned long long s_red[kBS / kWave];
+  static_assert(kLongPartners == kBS, "a partner per thread");
+  const int tid = threadIdx.x;
+  unsigned long long count = 0, probes = 0;
+  for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
+    const TcItem item = items[it];
+    const int64_t xb = off[item.x], deg = off[item.x + 1] - xb;
+    const int32_t d = fdeg[item.x].d, sb0 = blockIdx.y * kSetSlice;
+    if (sb0 >= d) continue;  // uniform: another block's
+    int32_t p;
+    const int len = Partner(dst, fdeg, xb, deg, d, int64_t(item.pb) + tid, p).d;
+    s_beg[tid] = off[p];
+    if (sb0 == 0) probes += static_cast<unsigned long long>(len);
+    int total = 0;
+    s_pre[tid] = BlockExclusiveScan<kBS>(len, &total, s_scan);
+    for (int32_t sb = sb0; sb < d && total > 0; sb += gridDim.y * kSetSlice) {
+      const int32_t slice = sb + kSetSlice < d ? kSetSlice : d - sb;
+      uint32_t size = 64;
+      while (size < 2u * static_cast<uint32_t>(slice)) size <<= 1;
+      const uint32_t mask = size - 1;
+      for (uint32_t i = tid; i < size; i += kBS) table[i] = -1;
+      __syncthreads();
+      for (int32_t i = tid; i < slice; i += kBS) {
+        const int32_t w = dst[xb + sb + i];
+        uint32_t h = Hash(w, mask);
+        while (atomicCAS(&table[h], -1, w) != -1) h = (h + 1) & mask;
+      }
+      const int32_t lo_w = dst[xb + sb], hi_w = dst[xb + sb + slice - 1];
+      __syncthreads();
+      for (int j0 = 0; j0 < total; j0 += kBS * kHashUnroll) {
+        int32_t w[kHashUnroll];
+#pragma unroll
+        for (int k = 0; k < kHashUnroll; k++) {
+          const int j = j0 + k * kBS + tid;
+          int at = 0;  // the last list starting at or before j: the one that owns it
+#pragma unroll
+          for (int step = kLongPartners / 2; step > 0; step >>= 1)
+            if (s_pre[at + step] <= j) at += step;
+          w[k] = j < total ? dst[s_beg[at] + (j - s_pre[at])] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < kHashUnroll; k++) {
+          if (w[k] < lo_w || w[k] > hi_w) continue;
+          uint32_t h = Hash(w[k], mask);
+          while (true) {
+            const int32_t t = table[h];
+            if (t == w[k]) {
+              count++;
+              break;
+            }
+            if (t < 0) break;
+            h = (h + 1) & mask;
+          }
+        }
+      }
+      __syncthreads();
+    }
+    __syncthreads();  // (also where no list is probed: the next item rewrites s_pre)
+  }
+  FlushCounts(count, probes, counts, s_red);
+}
+
 // Short lists: the wavefront keeps N+(x) sorted in LDS; each lane walks one
 // partner's list (shorter than kLongList) and binary-searches it there.
 __global__ __launch_bounds__(kBS) void TcCountShort(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
@@ -416,8 +516,7 @@ extern "C" int gg_tc(gg_graph* g, uint64_t* count, gg_stats* stats) {
     const int spans = static_cast<int>(GridFor(n, kBS * 2, g->cu_count * 8));
     // One buffer per phase: a fresh handle pays for every allocation (a
     // relabelled graph is counted once).  8-byte arrays first.
-    int64_t* low_off = g->Scratch<int64_t>("tc.work", 2 * (n + 1) + 2 * kStripes + kSpanKinds * (1 + int64_t(spans)));
-    TcDegrees* fdeg = reinterpret_cast<TcDegrees*>(low_off + n + 1);
+    TcDegrees* fdeg = g->Scratch<TcDegrees>("tc.work", n + 1 + 2 * kStripes + kSpanKinds * (1 + int64_t(spans)));
     unsigned long long* counts = reinterpret_cast<unsigned long long*>(fdeg + n + 1);
     unsigned long long* span_items = counts + 2 * kStripes + kSpanKinds;
     const dim3 blk(kBS);
@@ -433,10 +532,14 @@ extern "C" int gg_tc(gg_graph* g, uint64_t* count, gg_stats* stats) {
     GG_HIP(hipMemcpyAsync(h, counts + 2 * kStripes, kSpanKinds * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     GG_HIP(hipStreamSynchronize(st));
     const int64_t nlong = static_cast<int64_t>(h[0]), nshort = static_cast<int64_t>(h[1]), nlow = static_cast<int64_t>(h[2]);
-    TcItem* items = g->Scratch<TcItem>("tc.items", nlong + nshort + (nlow + 3) / 4 + 1);
+    // Entries are counted once per edge in the lists N+: half of all.
+    const bool bits = nlow >= static_cast<int64_t>(kBitsShare * 0.5 * static_cast<double>(g->out_entries));
+    // Items; then, for TcCountLong, the first 16-bit id of every vertex and the
+    // ids, readable to the end of the pair after the last one.
+    TcItem* items = g->Scratch<TcItem>("tc.items", nlong + nshort + 1 + (bits ? n + 1 + (nlow + 3) / 4 : 0));
     TcItem* shorts = items + nlong;
-    // 16-bit ids, readable to the end of the pair after the last one.
-    uint16_t* low = reinterpret_cast<uint16_t*>(shorts + nshort);
+    int64_t* low_off = bits ? reinterpret_cast<int64_t*>(shorts + nshort) : nullptr;
+    uint16_t* low = bits ? reinterpret_cast<uint16_t*>(low_off + n + 1) : nullptr;
     Run(g, "tc_items", 24.0 * N + 8.0 * (nlong + nshort), TcItemFill, dim3(spans), blk,
         static_cast<const int64_t*>(g->out_off), static_cast<const TcDegrees*>(fdeg), n,
         static_cast<const unsigned long long*>(span_items), items, shorts, low_off);
@@ -444,16 +547,23 @@ extern "C" int gg_tc(gg_graph* g, uint64_t* count, gg_stats* stats) {
     // Compulsory bytes: one pass over the CSR, 8 (n + 1) + 4 m.  The merge
     // work (probes, stats->edges_examined) is reported apart: its re-reads
     // of lists and LDS probes are not compulsory traffic.
-    if (nlong > 0) {
+    const double csr = 8.0 * (N + 1) + 4.0 * static_cast<double>(g->out_entries);
+    const dim3 grid_long(GridFor(nlong, 1, g->cu_count * kCountBlocksPerCu));
+    if (nlong > 0 && bits) {
       Run(g, "tc_narrow", 16.0 * N + 6.0 * nlow, TcNarrow, dim3(GridFor(n, kBS / kNarrowLanes, g->cu_count * 32)), blk,
           static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst),
           static_cast<const TcDegrees*>(fdeg), static_cast<const int64_t*>(low_off), n, low);
-      Run(g, "tc_count", 8.0 * (N + 1) + 4.0 * static_cast<double>(g->out_entries), TcCountLong,
-          dim3(GridFor(nlong, 1, g->cu_count * kCountBlocksPerCu)), blk, static_cast<const int64_t*>(g->out_off),
+      Run(g, "tc_count", csr, TcCountLong, grid_long, blk, static_cast<const int64_t*>(g->out_off),
           static_cast<const int32_t*>(g->out_dst), static_cast<const TcDegrees*>(fdeg),
           static_cast<const int64_t*>(low_off), static_cast<const uint16_t*>(low),
           static_cast<const TcItem*>(items), nlong, counts);
       launches += 2;
+    } else if (nlong > 0) {
+      const unsigned ways = g->max_degree > kSetSlice ? kSliceWays : 1;
+      Run(g, "tc_count", csr, TcCountHash, dim3(grid_long.x, ways), blk, static_cast<const int64_t*>(g->out_off),
+          static_cast<const int32_t*>(g->out_dst), static_cast<const TcDegrees*>(fdeg),
+          static_cast<const TcItem*>(items), nlong, counts);
+      launches++;
     }
     if (nshort > 0) {
       Run(g, "tc_count_short", 0, TcCountShort, dim3(GridFor(nshort, kBS / kWave, g->cu_count * kCountBlocksPerCu)),
