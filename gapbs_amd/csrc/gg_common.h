@@ -114,7 +114,6 @@ struct gg_graph {
   // UploadOrderLists.  Null otherwise.
   int32_t* fold_dst = nullptr;
   int64_t max_degree = 0;  // max out-degree (in-degree for the inverse), set at upload
-  int32_t max_weight = -1;  // largest list weight (computed on first SSSP)
   int64_t no_in_count = -1;  // vertices without in-neighbours (computed on first BFS)
   gg_tuning tune = {15, 18, 15, 32, 32, 1024, 16, 0, {0, 0, 0, 0}, {0, 0}, {0, 0}, 0, 0, 0};  // gg_autotune results
   int64_t pr_bins[3] = {-1, -1, -1};     // PageRank in-degree bins (vertex counts)

@@ -8,15 +8,13 @@
 // current bucket again until it stays empty (the effect of the reference's
 // bucket fusion, sssp.cc:113-120).  Shortest distances are unique, so the
 // result equals the reference's bit for bit whatever the processing order.
-//
-// Light and heavy edges (Meyer and Sanders, J. Algorithms 2003; the reference
-// relaxes all alike).  An edge of weight delta or more leads out of the
-// bucket, so what it gives while its vertex's distance may still drop is
-// wasted: with such edges in the graph, the launches that empty a bucket skip
-// them and list the vertices they expand, and one launch then relaxes the
-// listed vertices' heavy edges from their final distances.  A skipped edge
-// costs its 8 bytes of list but no distance read.  Kronecker 22, weights to
-// 255, delta 16: 271 M relaxations without, 137 M with.
+// (Edges of weight delta or more relaxed apart, once per bucket and from final
+// distances, after Meyer and Sanders: fewer relaxations, but a launch more per
+// bucket and a pass over the skipped edges.  Kronecker 26, delta 8: 2.12
+// against 2.59 G relaxations, 61 against 55 ms; a 1000 x 1000 lattice with
+// diagonals, delta 64 and weights to 1000: 275 against 227 ms; faster only on
+// large skewed graphs with a delta near the weights, Kronecker 22, delta 64:
+// 6.45 against 7.38.)
 //
 // GPU design: the current bucket is a device queue F.  A relax launch
 // expands F's edges (gg_expand.h, the source distance carried as payload)
@@ -34,7 +32,6 @@
 // pile to one kept and one fresh copy of a vertex, which bounds near and F
 // by N and the piles by 2N, so no append can overflow.
 #include <climits>
-#include <type_traits>
 
 #include "gg_common.h"
 #include "gg_expand.h"
@@ -47,21 +44,15 @@ constexpr int kQueueCap = 2048;
 constexpr int32_t kDistInf = INT32_MAX / 2;
 constexpr int kStripes = 64;
 constexpr int64_t kWindow = 8;  // buckets per mid window
-// Entries per vertex from which heavy edges are relaxed apart.  Graphs of lower
-// degree have few edges a bucket and many buckets, and each bucket's extra
-// launch costs more than the relaxations it saves: a 122 x 122 grid, delta 256,
-// weights to 1000: 3.6 ms without, 4.3 with; directed R-MAT, 8 k vertices of
-// degree 8, delta 16: 3.3 without, 2.2 with.
-constexpr int64_t kSplitDegree = 6;
 // Grid caps of the per-bucket kernels, in blocks per CU.  Bucket frontiers
 // and piles are often a few hundred thousand entries; many small blocks keep
 // more relaxations and row reads in flight than a few blocks looping over
 // tiles.  At Kronecker 26 (4 roots, delta 8) 64 took the step from 703 to
 // 294 ms (8 and 4: 703 ms; 16: 501 ms; 32: 328 ms; 128: no better).
 constexpr unsigned kBucketBlocksPerCu = 64;
-// Of the launches whose work only the device knows (hub chunks, the pile
-// after a heavy launch): all blocks resident, those without work leave.
-constexpr unsigned kRelaxBlocksPerCu = 8;
+// Of the hub chunks, whose number only the device knows: all blocks resident,
+// those without work leave.
+constexpr unsigned kChunkBlocksPerCu = 8;
 enum { kRelaxed, kImproved, kNumSums };
 
 struct SsspCounters {
@@ -72,7 +63,6 @@ struct SsspCounters {
   int32_t fout_tail;   // split output (entries beyond the window)
   int32_t min_far;     // smallest pile distance >= bucket end
   int32_t nchunks;
-  int32_t settled_tail;  // vertices expanded in this bucket (heavy edges to relax)
   unsigned long long sums[kStripes][kNumSums];
 };
 
@@ -83,29 +73,25 @@ __global__ __launch_bounds__(kBS) void SsspReset(SsspCounters* c) {
     c->near_tail = c->fresh_tail = c->f_tail = c->mid2_tail = c->fout_tail = 0;
     c->min_far = kDistInf;
     c->nchunks = 0;
-    c->settled_tail = 0;
   }
 }
 
 __global__ __launch_bounds__(kBS) void SsspInit(int32_t* __restrict__ dist, int32_t* __restrict__ stamp,
                                                 int32_t* __restrict__ freshstamp, int32_t* __restrict__ midstamp,
-                                                int32_t* __restrict__ farstamp, int32_t* __restrict__ setstamp,
-                                                int64_t n, int32_t src, int32_t* __restrict__ frontier) {
+                                                int32_t* __restrict__ farstamp, int64_t n, int32_t src,
+                                                int32_t* __restrict__ frontier) {
   for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBS) {
     dist[i] = i == src ? 0 : kDistInf;
     stamp[i] = -1;
     freshstamp[i] = -1;
     midstamp[i] = -1;
     farstamp[i] = -1;
-    if (setstamp) setstamp[i] = -1;
     if (i == src) frontier[0] = src;
   }
 }
 
 enum PublishMode { kAfterRelax = 0, kAfterMin = 1, kAfterSplit = 2 };
-enum {
-  kMailNear, kMailFresh, kMailF, kMailMid, kMailFout, kMailMin, kMailSettled, kMailRelaxed, kMailImproved, kMailValues
-};
+enum { kMailNear, kMailFresh, kMailF, kMailMid, kMailFout, kMailMin, kMailRelaxed, kMailImproved, kMailValues };
 
 // Posts the counters the host needs after each kind of step and resets the
 // ones the next step appends to.  One block.
@@ -129,7 +115,6 @@ __global__ __launch_bounds__(kBS) void SsspPublish(SsspCounters* c, int mode, un
     vals[kMailMid] = static_cast<unsigned long long>(c->mid2_tail);
     vals[kMailFout] = static_cast<unsigned long long>(c->fout_tail);
     vals[kMailMin] = static_cast<unsigned long long>(c->min_far);
-    vals[kMailSettled] = static_cast<unsigned long long>(c->settled_tail);
     vals[kMailRelaxed] = tot[kRelaxed];
     vals[kMailImproved] = tot[kImproved];
     if (mode == kAfterRelax) {
@@ -137,8 +122,6 @@ __global__ __launch_bounds__(kBS) void SsspPublish(SsspCounters* c, int mode, un
       c->nchunks = 0;
     } else if (mode == kAfterMin) {
       c->min_far = kDistInf;
-      c->nchunks = 0;  // the heavy edges' chunks
-      c->settled_tail = 0;
     } else {  // a split consumed the fresh pile; the host takes its outputs' sizes
       c->fresh_tail = c->f_tail = c->mid2_tail = c->fout_tail = 0;
     }
@@ -146,18 +129,14 @@ __global__ __launch_bounds__(kBS) void SsspPublish(SsspCounters* c, int mode, un
   }
 }
 
-// Which edges a launch relaxes: all, those below delta or the others.
-enum EdgePart { kAllEdges, kLightEdges, kHeavyEdges };
-
 // Relaxes edges e[k] of frontier vertices (payload = the vertex's distance when
 // it was loaded).
-template <EdgePart kPart>
 struct RelaxVisit {
   const int2* wdst;
   int32_t* dist;
   int32_t* stamp;
   int32_t* freshstamp;
-  int32_t bucket_end, delta;
+  int32_t bucket_end;
   int32_t near_tag, fresh_tag;
   LdsQueue<kQueueCap>* lnear;
   LdsQueue<kQueueCap>* lfresh;
@@ -171,21 +150,19 @@ struct RelaxVisit {
     int2 vw[kExpandEdges];
     int32_t v[kExpandEdges], old[kExpandEdges];
     int64_t nd[kExpandEdges];
-    bool take[kExpandEdges], to_near[kExpandEdges], to_fresh[kExpandEdges], better[kExpandEdges];
+    bool to_near[kExpandEdges], to_fresh[kExpandEdges], better[kExpandEdges];
 #pragma unroll
     for (int k = 0; k < kExpandEdges; k++) vw[k] = wdst[e[k]];
 #pragma unroll
     for (int k = 0; k < kExpandEdges; k++) {
-      take[k] = valid[k] && (kPart == kAllEdges || (vw[k].y >= delta) == (kPart == kHeavyEdges));
       v[k] = vw[k].x;
       nd[k] = static_cast<int64_t>(du[k]) + vw[k].y;
-      // (an edge that is not taken reads one hot word)
-      old[k] = dist[kPart == kAllEdges || take[k] ? v[k] : 0];
-      relaxed += take[k];
+      old[k] = dist[v[k]];
+      relaxed += valid[k];
     }
 #pragma unroll
     for (int k = 0; k < kExpandEdges; k++) {
-      better[k] = take[k] && nd[k] < kDistInf && nd[k] < old[k];
+      better[k] = valid[k] && nd[k] < kDistInf && nd[k] < old[k];
       if (better[k]) old[k] = atomicMin(&dist[v[k]], static_cast<int32_t>(nd[k]));
     }
 #pragma unroll
@@ -207,8 +184,7 @@ struct RelaxVisit {
   }
 };
 
-template <EdgePart kPart>
-__device__ __forceinline__ void FlushRelax(RelaxVisit<kPart>& rv, SsspCounters* c, unsigned long long* s_red) {
+__device__ __forceinline__ void FlushRelax(RelaxVisit& rv, SsspCounters* c, unsigned long long* s_red) {
   LdsQueueFlush(*rv.lnear, rv.near, &c->near_tail);
   LdsQueueFlush(*rv.lfresh, rv.fresh, &c->fresh_tail);
   const unsigned long long r = BlockSum<kBS>(rv.relaxed, s_red);
@@ -220,24 +196,19 @@ __device__ __forceinline__ void FlushRelax(RelaxVisit<kPart>& rv, SsspCounters* 
   }
 }
 
-// kLightEdges: also lists each vertex once per bucket (settled, set_tag).
-template <EdgePart kPart>
 __global__ __launch_bounds__(kBS) void SsspRelax(const int64_t* __restrict__ off, const int2* __restrict__ wdst,
                                                  int32_t* __restrict__ dist, int32_t* __restrict__ stamp,
                                                  int32_t* __restrict__ freshstamp,
                                                  const int32_t* __restrict__ frontier, int32_t fn,
-                                                 int32_t bucket_end, int32_t delta, int32_t near_tag,
-                                                 int32_t fresh_tag, int32_t* __restrict__ near,
-                                                 int32_t* __restrict__ fresh, SsspCounters* c, EdgeChunk* chunks,
-                                                 int32_t* __restrict__ settled,
-                                                 int32_t* __restrict__ setstamp, int32_t set_tag) {
+                                                 int32_t bucket_end, int32_t near_tag, int32_t fresh_tag,
+                                                 int32_t* __restrict__ near, int32_t* __restrict__ fresh,
+                                                 SsspCounters* c, EdgeChunk* chunks) {
   __shared__ ExpandShared sh;
-  __shared__ int s_append[kBS / kWave + 1];
   __shared__ LdsQueue<kQueueCap> lnear, lfresh;
   __shared__ unsigned long long s_red[kBS / kWave];
   LdsQueueInit(lnear);
   LdsQueueInit(lfresh);
-  RelaxVisit<kPart> rv{wdst, dist, stamp, freshstamp, bucket_end, delta, near_tag, fresh_tag, &lnear, &lfresh, near, fresh, c};
+  RelaxVisit rv{wdst, dist, stamp, freshstamp, bucket_end, near_tag, fresh_tag, &lnear, &lfresh, near, fresh, c};
   for (int64_t tile = int64_t(blockIdx.x) * kBS; tile < fn; tile += int64_t(gridDim.x) * kBS) {
     const int64_t i = tile + threadIdx.x;
     int32_t u = 0, du = 0;
@@ -248,18 +219,15 @@ __global__ __launch_bounds__(kBS) void SsspRelax(const int64_t* __restrict__ off
       beg = off[u];
       end = off[u + 1];
     }
-    if (kPart == kLightEdges)
-      BlockAppend(i < fn && atomicExch(&setstamp[u], set_tag) != set_tag, u, settled, &c->settled_tail, s_append);
     ExpandTile<FrontierCut>(sh, u, du, beg, end, rv, chunks, &c->nchunks);
   }
   FlushRelax(rv, c, s_red);
 }
 
-template <EdgePart kPart>
 __global__ __launch_bounds__(kBS) void SsspRelaxChunks(const int2* __restrict__ wdst, int32_t* __restrict__ dist,
                                                        int32_t* __restrict__ stamp,
                                                        int32_t* __restrict__ freshstamp, int32_t bucket_end,
-                                                       int32_t delta, int32_t near_tag, int32_t fresh_tag,
+                                                       int32_t near_tag, int32_t fresh_tag,
                                                        int32_t* __restrict__ near, int32_t* __restrict__ fresh,
                                                        SsspCounters* c, const EdgeChunk* chunks) {
   const int32_t nchunks = c->nchunks;
@@ -268,18 +236,16 @@ __global__ __launch_bounds__(kBS) void SsspRelaxChunks(const int2* __restrict__ 
   __shared__ unsigned long long s_red[kBS / kWave];
   LdsQueueInit(lnear);
   LdsQueueInit(lfresh);
-  RelaxVisit<kPart> rv{wdst, dist, stamp, freshstamp, bucket_end, delta, near_tag, fresh_tag, &lnear, &lfresh, near, fresh, c};
+  RelaxVisit rv{wdst, dist, stamp, freshstamp, bucket_end, near_tag, fresh_tag, &lnear, &lfresh, near, fresh, c};
   ExpandChunks<FrontierCut>(chunks, nchunks, rv);
   FlushRelax(rv, c, s_red);
 }
 
-// Smallest distance >= bucket_end among the entries of a pile and the fresh
-// pile (whose size the host need not know yet).
+// Smallest distance >= bucket_end among the entries of two piles.
 __global__ __launch_bounds__(kBS) void SsspPileMin(const int32_t* __restrict__ pa, int32_t na,
-                                                   const int32_t* __restrict__ pb,
+                                                   const int32_t* __restrict__ pb, int32_t nb,
                                                    const int32_t* __restrict__ dist, int32_t bucket_end,
                                                    SsspCounters* c) {
-  const int32_t nb = c->fresh_tail;
   __shared__ int32_t s_min[kBS / kWave];
   int32_t m = kDistInf;
   const int64_t total = int64_t(na) + nb;
@@ -342,26 +308,6 @@ __global__ __launch_bounds__(kBS) void SsspSplit(const int32_t* __restrict__ pa,
   LdsQueueFlush(lk, fout, &c->fout_tail);
 }
 
-// Largest weight of the lists (at least 0).
-__global__ __launch_bounds__(kBS) void SsspMaxWeight(const int2* __restrict__ wdst, int64_t m, int32_t* out) {
-  __shared__ int32_t s_max[kBS / kWave];
-  int32_t w = 0;
-  for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < m; i += int64_t(gridDim.x) * kBS) {
-    const int32_t x = wdst[i].y;
-    w = x > w ? x : w;
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    const int32_t t = __shfl_xor(w, o);
-    w = t > w ? t : w;
-  }
-  if (LaneId() == 0) s_max[threadIdx.x / kWave] = w;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < kBS / kWave; i++) w = s_max[i] > w ? s_max[i] : w;
-    atomicMax(out, w);
-  }
-}
-
 // Reached vertices and their summed out-degree (for GTEPS).
 __global__ __launch_bounds__(kBS) void SsspReach(const int32_t* __restrict__ dist, const int64_t* __restrict__ off,
                                                  int64_t n, unsigned long long* out) {
@@ -416,22 +362,6 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
     EdgeChunk* chunks =
         use_chunks ? g->Scratch<EdgeChunk>("sssp.chunks", FrontierCut::Bound(n, g->out_entries)) : nullptr;
 
-    // The largest weight says whether any edge is heavy (once per handle: the
-    // lists do not change).
-    if (g->max_weight < 0) {
-      int32_t* mw = g->Scratch<int32_t>("sssp.max_weight", 1);
-      GG_HIP(hipMemsetAsync(mw, 0, sizeof(int32_t), st));
-      SsspMaxWeight<<<dim3(GridFor(g->out_entries, kBS, g->cu_count * 8)), dim3(kBS), 0, st>>>(wdst, g->out_entries,
-                                                                                            mw);
-      int32_t h = 0;
-      GG_HIP(hipMemcpyAsync(&h, mw, sizeof(h), hipMemcpyDeviceToHost, st));
-      GG_HIP(hipStreamSynchronize(st));
-      g->max_weight = h;
-    }
-    const bool split = g->max_weight >= delta && g->out_entries >= kSplitDegree * n;
-    int32_t* settled = split ? g->Scratch<int32_t>("sssp.settled", n + 64) : nullptr;
-    int32_t* setstamp = split ? g->Scratch<int32_t>("sssp.setstamp", n) : nullptr;
-
     const dim3 blk(kBS);
     const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
     const double N = static_cast<double>(n);
@@ -446,8 +376,7 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
 
     BeginTiming(g);
     Run(g, "sssp_reset", 0, SsspReset, dim3(1), blk, dc);
-    Run(g, "sssp_init", (split ? 24 : 20) * N, SsspInit, grid_n, blk, dist, stamp, freshstamp, midstamp, farstamp,
-        setstamp, n, source, fq);
+    Run(g, "sssp_init", 20 * N, SsspInit, grid_n, blk, dist, stamp, freshstamp, midstamp, farstamp, n, source, fq);
     launches += 2;
     auto clamp = [](int64_t x) { return static_cast<int32_t>(x < kDistInf ? x : kDistInf); };
     int64_t fsize = 1, fresh_size = 0, mid_size = 0, far_size = 0;
@@ -462,69 +391,52 @@ extern "C" int gg_sssp(gg_graph* g, int32_t source, int32_t delta, int32_t* dist
     // so this bound is never reached by a correct run; it only turns a
     // logic error into an error instead of an endless loop.
     const int64_t max_launches = 64 * n + 100000;
-    // Smallest live distance (>= bucket_end) over a pile and the fresh pile,
-    // kDistInf if none; fresh_size is known afterwards.
-    auto pile_min = [&](const int32_t* pa, int64_t na, bool fresh_known) {
-      if (fresh_known && na + fresh_size == 0) return static_cast<int64_t>(kDistInf);
-      const unsigned cap = g->cu_count * (fresh_known ? kBucketBlocksPerCu : kRelaxBlocksPerCu);
-      Run(g, "sssp_pile_min", 8.0 * (na + fresh_size), SsspPileMin,
-          dim3(fresh_known ? GridFor(na + fresh_size, kBS, cap) : cap), blk, pa, static_cast<int32_t>(na),
-          static_cast<const int32_t*>(fresh), static_cast<const int32_t*>(dist), clamp(bucket_end), dc);
+    // Smallest live distance (>= bucket_end) over two piles, kDistInf if none.
+    auto pile_min = [&](const int32_t* pa, int64_t na, const int32_t* pb, int64_t nb) {
+      const int64_t total = na + nb;
+      if (total == 0) return static_cast<int64_t>(kDistInf);
+      Run(g, "sssp_pile_min", 8.0 * total, SsspPileMin, dim3(GridFor(total, kBS, g->cu_count * kBucketBlocksPerCu)), blk, pa,
+          static_cast<int32_t>(na), pb, static_cast<int32_t>(nb), static_cast<const int32_t*>(dist),
+          clamp(bucket_end), dc);
       launches++;
       publish(kAfterMin);
-      relaxed += static_cast<int64_t>(mail[kMailRelaxed]);
-      fresh_size = static_cast<int64_t>(mail[kMailFresh]);
       return static_cast<int64_t>(mail[kMailMin]);
     };
-    // One relax launch (and its hub chunks) over q[0, size).
-    auto relax = [&](const int32_t* q, int64_t size, auto part, int32_t near_tag, int32_t fresh_tag, int32_t set_tag) {
-      constexpr EdgePart kPart = decltype(part)::value;
-      const int32_t end32 = clamp(bucket_end);
-      const int idx = Run(g, "sssp_relax", 12.0 * size, SsspRelax<kPart>,
-                          dim3(GridFor(size, kBS, g->cu_count * kBucketBlocksPerCu)), blk, g->out_off, wdst, dist,
-                          stamp, freshstamp, q, static_cast<int32_t>(size), end32, delta, near_tag, fresh_tag, nq,
-                          fresh, dc, use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), settled,
-                          setstamp, set_tag);
-      launches++;
-      if (use_chunks) {
-        Run(g, "sssp_relax_chunks", 0, SsspRelaxChunks<kPart>, dim3(g->cu_count * kRelaxBlocksPerCu), blk, wdst, dist,
-            stamp, freshstamp, end32, delta, near_tag, fresh_tag, nq, fresh, dc,
-            static_cast<const EdgeChunk*>(chunks));
-        launches++;
-      }
-      relax_launches++;
-      return idx;
-    };
-    using All = std::integral_constant<EdgePart, kAllEdges>;
-    using Light = std::integral_constant<EdgePart, kLightEdges>;
-    using Heavy = std::integral_constant<EdgePart, kHeavyEdges>;
     while (true) {
-      const int32_t fresh_tag = ++tag, set_tag = ++tag;
-      int64_t nsettled = 0;
+      const int32_t fresh_tag = ++tag;
       while (fsize > 0) {
         GG_REQUIRE(relax_launches < max_launches, GG_EHIP, "SSSP did not converge");
         const int32_t near_tag = ++tag;
-        const int idx = split ? relax(fq, fsize, Light{}, near_tag, fresh_tag, set_tag)
-                              : relax(fq, fsize, All{}, near_tag, fresh_tag, set_tag);
+        const int32_t end32 = clamp(bucket_end);
+        const int idx = Run(g, "sssp_relax", 12.0 * fsize, SsspRelax,
+                            dim3(GridFor(fsize, kBS, g->cu_count * kBucketBlocksPerCu)), blk, g->out_off, wdst, dist,
+                            stamp, freshstamp, static_cast<const int32_t*>(fq),
+                            static_cast<int32_t>(fsize), end32, near_tag, fresh_tag, nq, fresh, dc,
+                            use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr));
+        launches++;
+        if (use_chunks) {
+          Run(g, "sssp_relax_chunks", 0, SsspRelaxChunks, dim3(g->cu_count * kChunkBlocksPerCu), blk, wdst, dist,
+              stamp, freshstamp, end32, near_tag, fresh_tag, nq, fresh, dc,
+              static_cast<const EdgeChunk*>(chunks));
+          launches++;
+        }
         publish(kAfterRelax);
+        relax_launches++;
         relaxed += static_cast<int64_t>(mail[kMailRelaxed]);
         CreditBytes(g, idx, 8.0 * mail[kMailRelaxed] + 8.0 * mail[kMailImproved]);
         fsize = static_cast<int64_t>(mail[kMailNear]);
         fresh_size = static_cast<int64_t>(mail[kMailFresh]);
-        nsettled = static_cast<int64_t>(mail[kMailSettled]);
         std::swap(fq, nq);
       }
-      if (split && nsettled > 0) relax(settled, nsettled, Heavy{}, ++tag, fresh_tag, set_tag);
-      const bool fresh_known = !(split && nsettled > 0);
       // The bucket is done.  Next: the smallest live distance of mid and
       // fresh when it lies inside the window (far holds only distances at or
       // beyond the window's end), else a new window from far and fresh.
       GG_REQUIRE(buckets < max_launches, GG_EHIP, "SSSP did not converge");
-      int64_t m = pile_min(mid, mid_size, fresh_known);
+      int64_t m = pile_min(mid, mid_size, fresh, fresh_size);
       // (kDistInf, "no live entry", can lie below a window end past it.)
       const bool in_window = m < kDistInf && m < window_end;
       if (!in_window) {
-        m = pile_min(far, far_size, true);
+        m = pile_min(far, far_size, fresh, fresh_size);
         if (m >= kDistInf) break;
       }
       const int64_t next_end = (m / delta + 1) * static_cast<int64_t>(delta);
