@@ -49,7 +49,10 @@ constexpr int kBS = 256;
 constexpr int kQueueCap = 2048;
 constexpr int kStripes = 64;
 constexpr int64_t kWaveEdges = 64;   // vertices with this many edges use a wavefront ...
-constexpr int64_t kSigmaChunk = 1024;  // ... per this many (sigma pull)
+constexpr int kSigmaChunkLog2 = 10;    // ... per this many, as a power of two (sigma pull)
+constexpr int64_t kDeepWaveEdges = 256;  // the same two where levels are discovered one by one
+constexpr int kDeepChunkLog2 = 12;
+constexpr int64_t kKindsVertices = int64_t(1) << 20;  // up to this many BcLevelKinds looks at every search
 constexpr int kThreadUnroll = 4;     // edges in flight per thread below that
 constexpr int kBcWaveUnroll = 4;     // 64-edge runs per wavefront step
 constexpr int32_t kSideLevel = 65536;  // vertices of a level from which BcDeltaWave takes a stream too
@@ -172,15 +175,16 @@ __global__ __launch_bounds__(kBS) void BcDiscoverChunks(const int32_t* __restric
 }
 
 // sigma[v] for the new level: sum of sigma over in-neighbours one level up.
-// Vertices with kWaveEdges in-edges or more are listed in chunks of
-// kSigmaChunk edges (one reservation per wavefront) and summed by
-// BcSigmaChunks; those of several chunks start from sigma = 0 here.
+// Vertices with wave_min in-edges or more are listed in chunks of 2^chunk_log2
+// edges (one reservation per wavefront) and summed by BcSigmaChunks; those of
+// several chunks start from sigma = 0 here.
 template <class T>
 __global__ __launch_bounds__(kBS) void BcSigma(const int64_t* __restrict__ in_off, const int32_t* __restrict__ in_dst,
                                                OnLevel prev, BcNode<T>* node, const int32_t* __restrict__ queue,
-                                               int32_t qb, int32_t qn, EdgeChunk* __restrict__ chunks, BcCounters* c,
-                                               unsigned long long* work) {
+                                               int32_t qb, int32_t qn, EdgeChunk* __restrict__ chunks, int64_t wave_min,
+                                               int chunk_log2, BcCounters* c, unsigned long long* work) {
   __shared__ unsigned long long s_red[kBS / kWave];
+  const int64_t chunk = int64_t(1) << chunk_log2;
   unsigned long long ent = 0, mat = 0;
   for (int64_t base = int64_t(blockIdx.x) * kBS; base < qn; base += int64_t(gridDim.x) * kBS) {
     const int64_t i = base + threadIdx.x;
@@ -191,7 +195,7 @@ __global__ __launch_bounds__(kBS) void BcSigma(const int64_t* __restrict__ in_of
       b = in_off[v];
       e = in_off[v + 1];
     }
-    const int nc = e - b >= kWaveEdges ? static_cast<int>((e - b + kSigmaChunk - 1) / kSigmaChunk) : 0;
+    const int nc = e - b >= wave_min ? static_cast<int>((e - b + chunk - 1) >> chunk_log2) : 0;
     const int upto = WaveInclusiveScan(nc);
     const int total = __builtin_amdgcn_readlane(upto, kWave - 1);
     if (total) {
@@ -199,9 +203,9 @@ __global__ __launch_bounds__(kBS) void BcSigma(const int64_t* __restrict__ in_of
       if (LaneId() == 0) at = atomicAdd(&c->nred, total);
       at = __builtin_amdgcn_readfirstlane(at) + upto - nc;
       for (int k = 0; k < nc; k++) {
-        const int64_t cb = b + k * kSigmaChunk;
+        const int64_t cb = b + k * chunk;
         // payload: whether the chunk is the whole list (its sum is stored)
-        chunks[at + k] = EdgeChunk{cb, cb + kSigmaChunk < e ? cb + kSigmaChunk : e, v, nc == 1};
+        chunks[at + k] = EdgeChunk{cb, cb + chunk < e ? cb + chunk : e, v, nc == 1};
       }
       if (nc > 1) node[v].sigma = 0.0;
     }
@@ -811,6 +815,44 @@ __global__ __launch_bounds__(kBS) void BcLevelClear(int32_t* __restrict__ counts
   for (int64_t i = i0; i < words; i += stride) bits[i] = 0;
 }
 
+// Which levels hold vertices for the wavefront and hub kernels, one bit per
+// level and kind: in-lists of in_min entries or more (kLongIn), out-lists of
+// kWaveEdges (kWaveOut) and of kBcHubEdges (kHubOut) or more.  Most such
+// vertices find their bit set already; collected per block in LDS, unless the
+// levels are too many, since on few levels every block would want the same words.
+enum { kLongIn, kWaveOut, kHubOut, kLevelKinds };
+constexpr int kKindWords = kLevelKinds * kBucketLevels / 32;
+__device__ __forceinline__ void SetBits(uint32_t* word, uint32_t bits) {
+  if (bits & ~*word) atomicOr(word, bits);
+}
+__global__ __launch_bounds__(kBS) void BcLevelKinds(const int32_t* __restrict__ depth,
+                                                    const int64_t* __restrict__ out_off,
+                                                    const int64_t* __restrict__ in_off, int64_t n, int64_t in_min,
+                                                    uint32_t* flags, int words) {
+  __shared__ uint32_t s_flags[kKindWords];
+  const bool few = kLevelKinds * words <= kKindWords;
+  for (int i = threadIdx.x; few && i < kLevelKinds * words; i += kBS) s_flags[i] = 0;
+  __syncthreads();
+  for (int64_t v = blockIdx.x * int64_t(kBS) + threadIdx.x; v < n; v += int64_t(gridDim.x) * kBS) {
+    const int32_t d = depth[v];
+    const int64_t out = out_off[v + 1] - out_off[v], in = in_off[v + 1] - in_off[v];
+    if (d < 0) continue;
+    const bool has[kLevelKinds] = {in >= in_min, out >= kWaveEdges && out < kBcHubEdges, out >= kBcHubEdges};
+#pragma unroll
+    for (int kind = 0; kind < kLevelKinds; kind++) {
+      if (!has[kind]) continue;
+      const int at = kind * words + (d >> 5);
+      if (few)
+        SetBits(&s_flags[at], 1u << (d & 31));
+      else
+        SetBits(&flags[at], 1u << (d & 31));
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; few && i < kLevelKinds * words; i += kBS)
+    if (s_flags[i]) SetBits(&flags[i], s_flags[i]);
+}
+
 __global__ __launch_bounds__(kBS) void BcClearReduce(BcCounters* c) {
   if (threadIdx.x == 0) {
     c->nred = 0;
@@ -916,15 +958,16 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     if (rec[kind] < 0) rec[kind] = idx;
   };
   auto wk = [&](int kind) { return work + kind * kWorkCounters; };
-  int32_t* lvl_counts = g->Scratch<int32_t>("bc.level_counts", kBucketLevels);
+  // Vertices per level, after the words of BcLevelKinds.
+  int32_t* lvl_counts = g->Scratch<int32_t>("bc.level_counts", kKindWords + kBucketLevels);
   int32_t* lvl_cursor = g->Scratch<int32_t>("bc.level_cursor", kBucketLevels);
-  std::vector<int32_t> h_counts(kBucketLevels);
+  std::vector<int32_t> h_counts(kKindWords + kBucketLevels);
   const int64_t entries = g->out_entries > g->in_entries ? g->out_entries : g->in_entries;
   EdgeChunk* chunks = g->Scratch<EdgeChunk>("bc.chunks", FrontierCut::Bound(n, entries));
   const bool hubs = g->max_degree >= FrontierCut::kMin, longs = g->max_degree >= kWaveEdges;
-  // Sigma chunks: sum of ceil(d / kSigmaChunk) over the vertices of kWaveEdges or more.
+  // Sigma chunks: sum of ceil(d / 2^kSigmaChunkLog2) over the vertices of kWaveEdges or more.
   EdgeChunk* rchunks =
-      longs ? g->Scratch<EdgeChunk>("bc.rchunks", entries / kSigmaChunk + std::min(n, entries / kWaveEdges) + 2)
+      longs ? g->Scratch<EdgeChunk>("bc.rchunks", (entries >> kSigmaChunkLog2) + std::min(n, entries / kWaveEdges) + 2)
             : nullptr;
   const int64_t nwords = (n + 63) / 64;
   const dim3 blk(kBS);
@@ -958,13 +1001,35 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     auto on_level = [&](int32_t d) {
       return OnLevel{bits ? reinterpret_cast<const uint32_t*>(bits + d * nwords) : nullptr, depth, d};
     };
+    // Cut-offs of the sigma pull; level by level, with no kinds known ahead,
+    // those that give fewer launches.
+    const bool buckets = nlev <= kBucketLevels;
+    const int64_t wave_min = buckets ? kWaveEdges : kDeepWaveEdges;
+    const int chunk_log2 = buckets ? kSigmaChunkLog2 : kDeepChunkLog2;
+    // Whether level d may hold vertices of a kind (BcLevelKinds, from depths of
+    // nlev levels).  A kernel left out of a level that holds none saves its
+    // launch and, on the side streams, a fork and join: a 500 x 500 lattice
+    // (999 levels) with one vertex of 5000 leaves takes 29.7 ms, 71.4 with all
+    // kernels at every level; Kronecker 20, 4 roots, 4.7 and 5.3.
+    const int kind_words = (nlev + 31) / 32;
+    std::vector<uint32_t> kinds;
+    auto holds = [&](int kind, int32_t d) {
+      return kinds.empty() || ((kinds[kind * kind_words + (d >> 5)] >> (d & 31)) & 1);
+    };
+    auto mark_kinds = [&](int32_t* flags) {
+      Run(g, "bc_level_kinds", 20.0 * N, BcLevelKinds, dim3(GridFor(n, kBS, g->cu_count * 8)), blk, static_cast<const int32_t*>(depth),
+          static_cast<const int64_t*>(g->out_off), static_cast<const int64_t*>(g->in_off), n, wave_min,
+          reinterpret_cast<uint32_t*>(flags), kind_words);
+      launches++;
+    };
     // Path counts of level d, queue[nb, nb + nn).
     auto pull_sigma = [&](int32_t d, int32_t nb, int32_t nn) {
       note(kWSigma, Run(g, "bc_sigma", 20.0 * nn, BcSigma<T>, dim3(GridFor(nn, kBS, g->cu_count * 16)), blk,
                         static_cast<const int64_t*>(g->in_off), static_cast<const int32_t*>(g->in_dst),
-                        on_level(d - 1), node, static_cast<const int32_t*>(queue), nb, nn, rchunks, dc, wk(kWSigma)));
+                        on_level(d - 1), node, static_cast<const int32_t*>(queue), nb, nn, rchunks, wave_min, chunk_log2, dc,
+                        wk(kWSigma)));
       launches++;
-      if (longs) {
+      if (g->max_degree >= wave_min && holds(kLongIn, d)) {
         note(kWSigmaChunks,
              Run(g, "bc_sigma_chunks", 0, BcSigmaChunks<T>, dim3(g->cu_count * 8), blk,
                  static_cast<const int32_t*>(g->in_dst), on_level(d - 1), node,
@@ -973,21 +1038,28 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
         launches += 2;
       }
     };
-    if (nlev <= kBucketLevels) {
+    if (buckets) {
       if (nlev <= kBitLevels) bits = g->Scratch<uint64_t>("bc.level_bits", kBitLevels * nwords);
       const int64_t chunk = BucketChunk(n);
       const dim3 grid_b(GridFor(n, static_cast<int>(chunk)));
-      Run(g, "bc_level_count", 0, BcLevelClear, grid_n, blk, lvl_counts, nlev, bits, bits ? nlev * nwords : 0);
+      // (a large graph's few levels are worth no look at every degree)
+      const int nkinds = longs && (n <= kKindsVertices || nlev > kBitLevels) ? kLevelKinds * kind_words : 0;
+      int32_t* counts = lvl_counts + nkinds;
+      Run(g, "bc_level_count", 0, BcLevelClear, grid_n, blk, lvl_counts, nkinds + nlev, bits,
+          bits ? nlev * nwords : 0);
       Run(g, "bc_level_count", 4 * N, BcLevelCount, dim3(GridFor(nwords, kBS / kWave, g->cu_count * 8)), blk,
-          static_cast<const int32_t*>(depth), n, nlev, lvl_counts, bits);
+          static_cast<const int32_t*>(depth), n, nlev, counts, bits);
       launches++;
-      GG_HIP(hipMemcpyAsync(h_counts.data(), lvl_counts, sizeof(int32_t) * nlev, hipMemcpyDeviceToHost, st));
+      if (nkinds) mark_kinds(lvl_counts);
+      GG_HIP(hipMemcpyAsync(h_counts.data(), lvl_counts, sizeof(int32_t) * (nkinds + nlev), hipMemcpyDeviceToHost, st));
       GG_HIP(hipStreamSynchronize(st));
+      kinds.assign(h_counts.begin(), h_counts.begin() + nkinds);
+      const int32_t* level_size = h_counts.data() + nkinds;
       int last = 0;
       for (int d = 0; d < nlev; d++)
-        if (h_counts[d]) last = d;
+        if (level_size[d]) last = d;
       bounds.assign(1, 0);
-      for (int d = 0; d <= last; d++) bounds.push_back(bounds.back() + h_counts[d]);
+      for (int d = 0; d <= last; d++) bounds.push_back(bounds.back() + level_size[d]);
       GG_HIP(hipMemcpyAsync(lvl_cursor, bounds.data(), sizeof(int32_t) * (last + 1), hipMemcpyHostToDevice, st));
       Run(g, "bc_level_scatter", 8 * N, BcLevelScatter, grid_b, blk, static_cast<const int32_t*>(depth), n, chunk, last + 1,
           lvl_cursor, queue);
@@ -1026,6 +1098,16 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
       pull_sigma(level + 1, nb, nn);
       level++;
     }
+    if (!bucketed && longs) {
+      int32_t* flags = g->Scratch<int32_t>("bc.deep_kinds", kLevelKinds * kind_words);
+      Run(g, "bc_level_kinds", 0, BcLevelClear, dim3(GridFor(kLevelKinds * kind_words, kBS)), blk, flags,
+          kLevelKinds * kind_words, static_cast<uint64_t*>(nullptr), int64_t(0));
+      mark_kinds(flags);
+      launches++;
+      kinds.resize(kLevelKinds * kind_words);
+      GG_HIP(hipMemcpyAsync(kinds.data(), flags, sizeof(uint32_t) * kinds.size(), hipMemcpyDeviceToHost, st));
+      GG_HIP(hipStreamSynchronize(st));
+    }
     reached_total += bounds.back();
     levels_total += level + 1;
     // Backward: deepest level first; delta of level d reads level d + 1.
@@ -1039,14 +1121,15 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
                           fold_dst, next, node, score, comp, static_cast<const int32_t*>(queue), qb, qn, wk(kWDelta)));
         launches++;
       };
-      if (!longs) {
+      const bool waves = longs && holds(kWaveOut, d), hubs = g->max_degree >= kBcHubEdges && holds(kHubOut, d);
+      if (!waves && !hubs) {
         delta();
       } else {
         // The three kernels write disjoint vertices and only read level
         // d + 1, so they run on three streams; all finish before the lists
         // are cleared.  A level below kSideLevel is over sooner than the
         // second fork costs.
-        const bool hubs = g->max_degree >= kBcHubEdges, side_wave = qn >= kSideLevel;
+        const bool side_wave = waves && qn >= kSideLevel;
         Run(g, "bc_delta_lists", 0, BcDeltaLists, dim3(GridFor(qn, kListTile, g->cu_count * 8)), blk,
             static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(queue), qb, qn, wave_list, hub_list,
             dc);
@@ -1063,14 +1146,17 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
           GG_HIP(hipEventRecord(g->ev_join, g->side));
           launches++;
         }
-        hipStream_t ws = side_wave ? g->side2 : st;
-        if (side_wave) GG_HIP(hipStreamWaitEvent(ws, g->ev_fork, 0));
-        note(kWDeltaWave,
-             RunOn(g, ws, "bc_delta_wave", 0, BcDeltaWave<T, kKahan>, dim3(GridFor(qn, kBS / kWave, g->cu_count * 8)),
-                   blk, static_cast<const int64_t*>(g->out_off), fold_dst, next, node, score, comp,
-                   static_cast<const int32_t*>(wave_list), static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
-        if (side_wave) GG_HIP(hipEventRecord(g->ev_join2, ws));
-        launches++;
+        if (waves) {
+          hipStream_t ws = side_wave ? g->side2 : st;
+          if (side_wave) GG_HIP(hipStreamWaitEvent(ws, g->ev_fork, 0));
+          note(kWDeltaWave,
+               RunOn(g, ws, "bc_delta_wave", 0, BcDeltaWave<T, kKahan>,
+                     dim3(GridFor(qn, kBS / kWave, g->cu_count * 8)), blk, static_cast<const int64_t*>(g->out_off),
+                     fold_dst, next, node, score, comp, static_cast<const int32_t*>(wave_list),
+                     static_cast<const BcCounters*>(dc), wk(kWDeltaWave)));
+          if (side_wave) GG_HIP(hipEventRecord(g->ev_join2, ws));
+          launches++;
+        }
         delta();
         if (hubs) GG_HIP(hipStreamWaitEvent(st, g->ev_join, 0));
         if (side_wave) GG_HIP(hipStreamWaitEvent(st, g->ev_join2, 0));

@@ -173,6 +173,34 @@ def test_bc_as_many_levels_as_vertices(n, directed):
     assert np.array_equal(gpu.bc(gpu.DeviceGraph(g), roots).scores, oracle.brandes(g, roots))
 
 
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("length", [12, 40, 4000, 4200])
+def test_bc_levels_with_and_without_long_lists(length, directed):
+    # A path on which a few levels hold vertices for the wavefront and hub
+    # kernels and the others none: fans of 63 to 5000 leaves, and joins of 64
+    # and 300 in-neighbours (directed: long in-lists beside short out-lists);
+    # levels bucketed with bitmaps, with depths, and found one by one.
+    print(f"[bc] path of {length} with fans, directed {directed}", flush=True)
+    u, v = list(range(length - 1)), list(range(1, length))
+    at = length
+    for k, d in enumerate((63, 64, 300, 4095, 4096, 5000)):
+        u += [length // 2 + k % 4] * d
+        v += list(range(at, at + d))
+        at += d
+    for k, d in enumerate((64, 300)):  # path vertex -> d vertices -> one vertex -> a leaf
+        mids = list(range(at, at + d))
+        u += [3 + k] * d + mids + [at + d]
+        v += mids + [at + d] * d + [at + d + 1]
+        at += d + 2
+    g = Graph.from_edges(np.array(u), np.array(v), symmetrize=not directed)
+    dg = gpu.DeviceGraph(g)
+    roots = np.array([0, length - 1, at - 1], dtype=np.int32)
+    assert np.array_equal(gpu.bc(dg, roots).scores, oracle.brandes(g, roots))
+    want = oracle.brandes(g, roots, fp64=True)
+    assert np.abs(gpu.bc(dg, roots, fp64=True).scores - want).max() < 1e-7
+    assert np.abs(gpu.bc(dg, roots, kahan=True).scores - want).max() < 2e-6
+
+
 @pytest.mark.parametrize("width", [2047, 2049, 70000])
 def test_bc_delta_lists(width):
     # Levels of one and several list tiles, and one above the size from which
