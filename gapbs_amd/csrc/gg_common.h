@@ -149,6 +149,9 @@ struct gg_graph {
     int64_t n_multi = 0, slots = 0;   // bins summed in several chunks, their partial-sum slots
     double build_ms = 0;
   } pr_blocks;
+  // PageRank blocks: entries per occupied block at each width, from a sample
+  // of the tiles (empty: not sampled yet).
+  std::vector<double> pr_spread;
   int64_t cc_samples_n = -1;             // n the uploaded Afforest sample positions are for
   int64_t ms_heavy = -1;                 // batched BFS: heavy vertices (listed once per graph)
   int64_t ms_heavy_chunks = 0;           // and their in-edge chunks

@@ -888,6 +888,7 @@ const gg_graph::PrSegments* Segments(gg_graph* g) {
 //         old value for its TwoSum, and measured 2.2x slower at Kronecker
 //         scale 26.)
 //   FP64  a double, added in arrival order.
+constexpr int kPbMinLog = 10;      // the narrowest width chosen by default
 constexpr int kPbMaxLog = 14;      // 2^14 accumulators of 8 bytes fill 128 KB of LDS
 constexpr int kPbMaxTiles = 8192;  // build tables hold k x k octet counts
 constexpr int kPbWriteBS = 1024;
@@ -1260,24 +1261,66 @@ __global__ __launch_bounds__(kPbBuildBS) void PbOctIndex(int64_t k, const uint32
   }
 }
 
+// How the in-entries of a few source tiles spread over the bins, for each
+// width from 2^kPbMinLog up (blockIdx.y): a tile's entries are its vertices'
+// out-lists, one range.  blockIdx.x: the first tile of every so many vertices.
+struct PbSpread {
+  unsigned long long entries[kPbMaxLog - kPbMinLog + 1], blocks[kPbMaxLog - kPbMinLog + 1];
+};
+constexpr int kPbSamples = 64;
+constexpr int64_t kPbSampleEntries = 1 << 18;  // of one tile; the rest is not looked at
+__global__ __launch_bounds__(kPbBuildBS) void PbSpreadOf(const int64_t* __restrict__ out_off,
+                                                         const int32_t* __restrict__ out_dst, int64_t n,
+                                                         PbSpread* out) {
+  constexpr int kWords = (1 << (27 - kPbMinLog)) / 32;  // a bit per bin of 2^27 vertices
+  __shared__ uint32_t s_bin[kWords];
+  __shared__ unsigned long long s_red[kPbBuildBS / kWave];
+  const int lg = kPbMinLog + blockIdx.y;
+  const int64_t words = (((n + (int64_t(1) << lg) - 1) >> lg) + 31) / 32;
+  for (int64_t i = threadIdx.x; i < words; i += kPbBuildBS) s_bin[i] = 0;
+  __syncthreads();
+  const int64_t first = n / gridDim.x * blockIdx.x >> kPbMaxLog << kPbMaxLog;
+  const int64_t b = out_off[first], end = out_off[first + (int64_t(1) << lg) < n ? first + (int64_t(1) << lg) : n];
+  const int64_t e = end - b < kPbSampleEntries ? end : b + kPbSampleEntries;
+  for (int64_t i = b + threadIdx.x; i < e; i += kPbBuildBS) {
+    const int32_t bin = out_dst[i] >> lg;
+    if (!((s_bin[bin >> 5] >> (bin & 31)) & 1)) atomicOr(&s_bin[bin >> 5], 1u << (bin & 31));
+  }
+  __syncthreads();
+  unsigned long long blocks = 0;
+  for (int64_t i = threadIdx.x; i < words; i += kPbBuildBS) blocks += static_cast<unsigned long long>(__popc(s_bin[i]));
+  blocks = BlockSum<kPbBuildBS>(blocks, s_red);
+  if (threadIdx.x == 0) {
+    atomicAdd(&out->entries[blockIdx.y], static_cast<unsigned long long>(e - b));
+    atomicAdd(&out->blocks[blockIdx.y], blocks);
+  }
+}
+
 // The width the Jacobi run of this precision uses (0: no blocks).  By
 // default the narrowest of 2^10 to 2^14 with at most kPbTiles tiles and at
 // least `want` in-entries per (tile, bin) block on average: a block is padded
 // to whole octets, so blocks of a few entries are mostly padding, while
 // narrower bins mean smaller LDS footprints and fewer bins summed in several
 // chunks.  Where degrees are skewed most entries sit in few blocks and a lower
-// average is enough, lower still when the ids follow the degrees.
+// average is enough, lower still when the ids follow the degrees.  The average
+// is over all blocks or, where neighbours' ids lie close together (lattices,
+// meshes: most blocks are empty), over those that hold entries, sampled once
+// per graph; tiles then hold at least kPbTileEntries.
 // Measured (FP32 / FP64 ms of a run, by width): Kronecker 22 as uploaded 2^10
 // 6.18 / 7.61 (padding 1.46), 2^11 3.20 / 5.08, 2^12 3.06 / 5.05, 2^14 3.36 /
 // 5.11; degree-ordered 2^10 3.22 / 4.83, 2^11 3.12 / 4.78, 2^12 3.37 / 5.11,
 // 2^14 4.36 / 5.83; Kronecker 20 ordered 2^10 1.10 / 1.83, 2^11 1.21 / 1.93;
 // uniform, 3 M vertices, degree 32, FP64 2^10 4.44 (padding 1.31), 2^12 3.39;
 // uniform 24 2^12 11.9 / 20.0, 2^13 10.4 / 19.1, 2^14 12.8 / 20.1; uniform 25
-// 2^13 21.2 / 38.8, 2^14 21.8 / 37.1.
+// 2^13 21.2 / 38.8, 2^14 21.8 / 37.1.  Close ids: 4000 x 4000 lattice 2^12
+// 1.71 / 2.02, 2^13 1.71 / 2.07, 2^14 2.10 / 2.52; 2047 x 2047 2^10 0.485 /
+// 0.562, 2^11 0.463 / 0.547, 2^12 0.455 / 0.545; 2^22 vertices of degree 16,
+// neighbours at most 5000 away, 2^10 1.98 / 2.84, 2^12 2.32 / 3.51; 2^21 of
+// degree 32, 100 away, 2^10 1.47 / 2.24, 2^12 1.79 / 2.63.
 constexpr int64_t kPbSkew = 32;  // max over average degree from which a graph counts as skewed
 constexpr int64_t kPbBlockEntries = 60, kPbBlockEntriesSkewed = 24, kPbBlockEntriesOrdered = 6;
-constexpr int64_t kPbTiles = 4096;
-int BlockWidth(const gg_graph* g, bool fp64) {
+constexpr int64_t kPbTiles = 4096, kPbTileEntries = 8192;
+int BlockWidth(gg_graph* g, bool fp64) {
   const int knob = g->tune.pr_blocks_log2;
   if (knob > 0) return knob;
   if (knob < 0 || g->tune.pr_segment_log2[fp64 ? 1 : 0] != 0) return 0;
@@ -1285,10 +1328,24 @@ int BlockWidth(const gg_graph* g, bool fp64) {
   if (n < (int64_t(1) << 20) || n > (int64_t(1) << 27)) return 0;
   const bool skewed = g->max_degree * n >= kPbSkew * g->in_entries;
   const int64_t want = !skewed ? kPbBlockEntries : g->new_id ? kPbBlockEntriesOrdered : kPbBlockEntriesSkewed;
-  int lg = 10;
+  int lg = kPbMinLog;
   for (; lg < kPbMaxLog; lg++) {
     const int64_t k = (n + (int64_t(1) << lg) - 1) >> lg;
-    if (k <= kPbTiles && g->in_entries >= want * k * k) break;
+    if (k > kPbTiles) continue;
+    if (g->in_entries >= want * k * k) break;
+    if ((skewed && g->new_id) || g->in_entries < kPbTileEntries * k) continue;
+    if (g->pr_spread.empty()) {
+      PbSpread h{};
+      PbSpread* d = g->Scratch<PbSpread>("pr.spread", 1);
+      GG_HIP(hipMemcpyAsync(d, &h, sizeof(h), hipMemcpyHostToDevice, g->stream));
+      PbSpreadOf<<<dim3(kPbSamples, kPbMaxLog - kPbMinLog + 1), kPbBuildBS, 0, g->stream>>>(g->out_off, g->out_dst, n, d);
+      GG_HIP(hipGetLastError());
+      GG_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, g->stream));
+      GG_HIP(hipStreamSynchronize(g->stream));
+      for (int i = 0; i <= kPbMaxLog - kPbMinLog; i++)
+        g->pr_spread.push_back(static_cast<double>(h.entries[i]) / static_cast<double>(std::max(1ull, h.blocks[i])));
+    }
+    if (g->pr_spread[lg - kPbMinLog] >= static_cast<double>(want)) break;
   }
   return lg;
 }

@@ -351,3 +351,23 @@ def test_pr_and_batch_bfs_blocks_build_splits_hubs_and_items():
         assert np.array_equal(res.depths[i], oracle.bfs_depth(g, r)), r
         assert np.array_equal(again.depths[i], res.depths[i]), r
     dg.free()
+
+
+def test_pr_block_width_follows_close_ids():
+    # The default width: a lattice of 2^20 vertices, whose blocks hold many
+    # entries or none, and a uniform graph of the same size and degree, whose
+    # entries fill all blocks thinly.
+    print("[pr] width, lattice and uniform", flush=True)
+    at = np.arange(1 << 20, dtype=np.int32).reshape(1024, 1024)
+    ends = [np.concatenate([a.reshape(-1), b.reshape(-1), c.reshape(-1)]) for a, b, c in
+            ((at[:, :-1], at[:-1], at[:-1, :-1]), (at[:, 1:], at[1:], at[1:, 1:]))]
+    rng = np.random.default_rng(3)
+    for close, (u, v) in ((True, ends), (False, rng.integers(0, 1 << 20, (2, len(ends[0])), dtype=np.int32))):
+        u[0] = (1 << 20) - 1
+        dg, _ = gpu.build_graph(u, v)
+        assert gpu.pagerank_blocks(dg)["width_log2"] == (11 if close else 12)
+        b32, b64 = gpu.pagerank(dg, 20, 1e-4), gpu.pagerank(dg, 20, 1e-4, fp64=True)
+        gpu.set_tuning(dg, {"pr_blocks_log2": -1, "pr_segment_log2": [-1, -1]})
+        plain = gpu.pagerank(dg, 20, 1e-4, fp64=True)
+        assert np.abs(b64.scores.astype(np.float64) - plain.scores).max() < 1e-7
+        assert np.abs(b32.scores.astype(np.float64) - plain.scores).max() < 1e-7
