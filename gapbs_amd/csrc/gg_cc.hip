@@ -114,16 +114,19 @@ __global__ __launch_bounds__(kBS) void CcHook(const int64_t* __restrict__ off, c
 
 // Sampled round r: link u with its r-th out-neighbour, if it has one; with
 // `first`, also with its first where CcHook did not hook it.  Two launches:
-// the first takes one wavefront's vertices in kLinkSample (`sample`), the
+// the first takes one wavefront's vertices in kLinkSample, the
 // second the others.  The trees that most vertices belong to are then merged
 // by few threads, and the rest find their labels joined instead of queueing
 // compare-and-swaps on the same roots (Kronecker 22: 325 us in one launch,
-// 156 us in two).
+// 156 us in two).  Graphs of less than kSampleVertices vertices, whose rounds
+// are launches rather than work, are linked in one (`part` kLinkAll).
 constexpr int kLinkSample = 64;
+constexpr int64_t kSampleVertices = 1 << 16;
+enum LinkPart { kLinkSampled, kLinkOthers, kLinkAll };
 __global__ __launch_bounds__(kBS) void CcLinkRound(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
-                                                   int32_t* comp, int64_t n, int r, bool first, bool sample) {
+                                                   int32_t* comp, int64_t n, int r, bool first, LinkPart part) {
   for (int64_t i = blockIdx.x * int64_t(kBS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBS) {
-    if ((i / kWave % kLinkSample == 0) != sample) continue;  // wavefront-uniform
+    if (part != kLinkAll && (i / kWave % kLinkSample == 0) != (part == kLinkSampled)) continue;  // wavefront-uniform
     const int32_t u = static_cast<int32_t>(i);
     const int64_t b = off[i], e = off[i + 1];
     if (first && e > b && dst[b] > u) Link(u, dst[b], comp);
@@ -329,18 +332,22 @@ int64_t RunAfforest(gg_graph* g, int neighbor_rounds, const CcBuffers& b, int32_
     Run(g, "cc_init", 4 * N, CcInit, grid_n, blk, b.comp, n);
   } else {
     // Round 0 is CcHook; the first neighbours it left are linked with the
-    // next round's, once the labels are compressed.  Offsets, the first
-    // neighbour, comp.
+    // next round's.  Offsets, the first neighbour, comp.
     Run(g, "cc_hook", 16 * N, CcHook, grid_n, blk, static_cast<const int64_t*>(g->out_off),
         static_cast<const int32_t*>(g->out_dst), b.comp, n);
-    compress();
+    // (of a single round, links and labels are compressed together)
+    if (neighbor_rounds > 1) compress();
+    const bool small = n < kSampleVertices;
     for (int r = neighbor_rounds == 1 ? 0 : 1; r < neighbor_rounds; r++) {
       // offsets 16 B (both ends), the r-th neighbour, comp read/write.
-      for (const bool sample : {true, false})
-        Run(g, "cc_link_round", sample ? 0 : 16 * N + 4 * N + 8 * N, CcLinkRound, grid_n, blk,
+      auto link = [&](LinkPart part) {
+        Run(g, "cc_link_round", part == kLinkSampled ? 0 : 16 * N + 4 * N + 8 * N, CcLinkRound, grid_n, blk,
             static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), b.comp, n, r, r <= 1,
-            sample);
-      launches += 2;
+            part);
+        launches++;
+      };
+      if (!small) link(kLinkSampled);
+      link(small ? kLinkAll : kLinkOthers);
       compress();
     }
   }
