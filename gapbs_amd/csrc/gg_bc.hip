@@ -615,9 +615,11 @@ __global__ __launch_bounds__(kBS) void BcDeltaWave(const int64_t* __restrict__ o
 // and packs the matched ones, in edge order, into one half of an LDS double
 // buffer; the last wavefront folds the previous round's terms in edge
 // order (FoldTerms).  Same terms, same order, same arithmetic as
-// BcDeltaWave.  Blocks take hubs from a counter, so a block held by a large
-// hub takes no others meanwhile (the list follows the level's queue, which
-// on a degree-ordered layout runs roughly from the largest hub down).
+// BcDeltaWave.  Two blocks fit a CU, of the compensated variant one (68
+// registers; held to 64 it took the same time: Kronecker 22, 4 roots, 22.1 and
+// 22.3 ms).  Blocks take hubs from a counter, so a block held by a large hub
+// takes no others meanwhile (the list follows the level's queue, which on a
+// degree-ordered layout runs roughly from the largest hub down).
 template <class T, bool kKahan>
 __global__ __launch_bounds__(kBcHubBS) void BcDeltaHub(const int64_t* __restrict__ off,
                                                        const int32_t* __restrict__ dst,
