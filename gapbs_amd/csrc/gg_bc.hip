@@ -50,8 +50,10 @@ constexpr int kQueueCap = 2048;
 constexpr int kStripes = 64;
 constexpr int64_t kWaveEdges = 64;   // vertices with this many edges use a wavefront ...
 constexpr int kSigmaChunkLog2 = 10;    // ... per this many, as a power of two (sigma pull)
-constexpr int64_t kDeepWaveEdges = 256;  // the same two where levels are discovered one by one
-constexpr int kDeepChunkLog2 = 12;
+// The same two where levels are discovered one by one, or where the longer
+// chunk list does not fit.
+constexpr int64_t kFewWaveEdges = 256;
+constexpr int kFewChunkLog2 = 12;
 constexpr int64_t kKindsVertices = int64_t(1) << 20;  // up to this many BcLevelKinds looks at every search
 constexpr int kThreadUnroll = 4;     // edges in flight per thread below that
 constexpr int kBcWaveUnroll = 4;     // 64-edge runs per wavefront step
@@ -68,6 +70,7 @@ struct alignas(16) BcNode {
   double sigma;
   T delta;
 };
+static_assert(sizeof(BcNode<float>) == sizeof(BcNode<double>), "one buffer serves both precisions");
 
 // Tells whether a vertex lies on one level: its bit in the level's bitmap,
 // or, without bitmaps (deep traversals), its depth.
@@ -941,14 +944,14 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   hipStream_t st = g->stream;
   const char* tag = sizeof(T) == 4 ? "32" : "64";
   int32_t* depth = g->Scratch<int32_t>("bc.depth", n);
-  BcNode<T>* node = g->Scratch<BcNode<T>>((std::string("bc.node") + tag).c_str(), n);
+  BcNode<T>* node = g->Scratch<BcNode<T>>("bc.node", n);
   int32_t* queue = g->Scratch<int32_t>("bc.queue", n + 64);
   T* score = g->Scratch<T>((std::string("bc.score") + tag).c_str(), n);
   T* comp = sizeof(T) == 4 ? g->Scratch<T>("bc.comp32", n) : nullptr;  // zero unless kKahan
   int32_t* wave_list = g->Scratch<int32_t>("bc.wave_list", n + 64);
   // A vertex with kBcHubEdges successors owns that many list entries.
   int32_t* hub_list = g->Scratch<int32_t>("bc.hub_list", g->out_entries / kBcHubEdges + 64);
-  float* out32 = g->Scratch<float>("bc.out32", n);
+  float* out32 = reinterpret_cast<float*>(wave_list);  // written when no level is left to list
   unsigned long long* max_bits = g->Scratch<unsigned long long>("bc.max", 1);
   BcCounters* dc = g->Scratch<BcCounters>("bc.ctr", 1);
   // Work counters (entries read, matched in-neighbours / successors) per
@@ -965,12 +968,15 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
   int32_t* lvl_cursor = g->Scratch<int32_t>("bc.level_cursor", kBucketLevels);
   std::vector<int32_t> h_counts(kKindWords + kBucketLevels);
   const int64_t entries = g->out_entries > g->in_entries ? g->out_entries : g->in_entries;
-  EdgeChunk* chunks = g->Scratch<EdgeChunk>("bc.chunks", FrontierCut::Bound(n, entries));
   const bool hubs = g->max_degree >= FrontierCut::kMin, longs = g->max_degree >= kWaveEdges;
-  // Sigma chunks: sum of ceil(d / 2^kSigmaChunkLog2) over the vertices of kWaveEdges or more.
-  EdgeChunk* rchunks =
-      longs ? g->Scratch<EdgeChunk>("bc.rchunks", (entries >> kSigmaChunkLog2) + std::min(n, entries / kWaveEdges) + 2)
-            : nullptr;
+  // Chunks of a level's discovery, then of its sigma pull: for the latter, the
+  // sum of ceil(d / 2^log2) over the vertices of wave_min in-edges or more.
+  auto chunk_bound = [&](int64_t wave_min, int log2) {
+    return std::max(FrontierCut::Bound(n, entries), (entries >> log2) + std::min(n, entries / wave_min) + 2);
+  };
+  EdgeChunk* chunks = longs ? g->TryScratch<EdgeChunk>("bc.chunks", chunk_bound(kWaveEdges, kSigmaChunkLog2)) : nullptr;
+  const bool many_chunks = chunks != nullptr;
+  if (longs && !many_chunks) chunks = g->Scratch<EdgeChunk>("bc.chunks", chunk_bound(kFewWaveEdges, kFewChunkLog2));
   const int64_t nwords = (n + 63) / 64;
   const dim3 blk(kBS);
   const dim3 grid_n(GridFor(n, kBS, g->cu_count * 32));
@@ -1006,8 +1012,9 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     // Cut-offs of the sigma pull; level by level, with no kinds known ahead,
     // those that give fewer launches.
     const bool buckets = nlev <= kBucketLevels;
-    const int64_t wave_min = buckets ? kWaveEdges : kDeepWaveEdges;
-    const int chunk_log2 = buckets ? kSigmaChunkLog2 : kDeepChunkLog2;
+    const bool short_waves = buckets && many_chunks;
+    const int64_t wave_min = short_waves ? kWaveEdges : kFewWaveEdges;
+    const int chunk_log2 = short_waves ? kSigmaChunkLog2 : kFewChunkLog2;
     // Whether level d may hold vertices of a kind (BcLevelKinds, from depths of
     // nlev levels).  A kernel left out of a level that holds none saves its
     // launch and, on the side streams, a fork and join: a 500 x 500 lattice
@@ -1028,20 +1035,21 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     auto pull_sigma = [&](int32_t d, int32_t nb, int32_t nn) {
       note(kWSigma, Run(g, "bc_sigma", 20.0 * nn, BcSigma<T>, dim3(GridFor(nn, kBS, g->cu_count * 16)), blk,
                         static_cast<const int64_t*>(g->in_off), static_cast<const int32_t*>(g->in_dst),
-                        on_level(d - 1), node, static_cast<const int32_t*>(queue), nb, nn, rchunks, wave_min, chunk_log2, dc,
+                        on_level(d - 1), node, static_cast<const int32_t*>(queue), nb, nn, chunks, wave_min, chunk_log2, dc,
                         wk(kWSigma)));
       launches++;
       if (g->max_degree >= wave_min && holds(kLongIn, d)) {
         note(kWSigmaChunks,
              Run(g, "bc_sigma_chunks", 0, BcSigmaChunks<T>, dim3(g->cu_count * 8), blk,
                  static_cast<const int32_t*>(g->in_dst), on_level(d - 1), node,
-                 static_cast<const EdgeChunk*>(rchunks), static_cast<const BcCounters*>(dc), wk(kWSigmaChunks)));
+                 static_cast<const EdgeChunk*>(chunks), static_cast<const BcCounters*>(dc), wk(kWSigmaChunks)));
         Run(g, "bc_clear_reduce", 0, BcClearReduce, dim3(1), blk, dc);
         launches += 2;
       }
     };
     if (buckets) {
-      if (nlev <= kBitLevels) bits = g->Scratch<uint64_t>("bc.level_bits", kBitLevels * nwords);
+      // (in steps of eight levels; where they do not fit, depths are tested)
+      if (nlev <= kBitLevels) bits = g->TryScratch<uint64_t>("bc.level_bits", (nlev + 7) / 8 * 8 * nwords);
       const int64_t chunk = BucketChunk(n);
       const dim3 grid_b(GridFor(n, static_cast<int>(chunk)));
       // (a large graph's few levels are worth no look at every degree)
@@ -1101,7 +1109,7 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
       level++;
     }
     if (!bucketed && longs) {
-      int32_t* flags = g->Scratch<int32_t>("bc.deep_kinds", kLevelKinds * kind_words);
+      int32_t* flags = wave_list;  // not listed in yet; 3 bits a level, at most n + 1 levels
       Run(g, "bc_level_kinds", 0, BcLevelClear, dim3(GridFor(kLevelKinds * kind_words, kBS)), blk, flags,
           kLevelKinds * kind_words, static_cast<uint64_t*>(nullptr), int64_t(0));
       mark_kinds(flags);
@@ -1186,6 +1194,8 @@ void RunBrandes(gg_graph* g, const int32_t* roots, int k, float* scores_out, gg_
     }
   }
   FinishTiming(g, stats, wt);
+  g->ws.Spare("bc.level_bits");
+  g->ws.Spare("bc.chunks");
   if (scores_out) CopyOutVertexF32(g, out32, scores_out);
   if (stats) {
     stats->total_ms = wt.ms();

@@ -69,11 +69,15 @@ struct Workspace {
   struct Slot {
     void* p = nullptr;
     size_t bytes = 0;
+    bool spare = false;  // not in use, and not needed by a call that fits without it
   };
   std::map<std::string, Slot> slots;
   // Returns a buffer of at least `bytes`, reallocating if the cached one is
-  // smaller.  Contents are undefined.
+  // smaller.  Contents are undefined.  Spare buffers make room where it would
+  // not fit.
   void* Get(const std::string& name, size_t bytes);
+  // The call using `name` is done with it; its next Get takes it back.
+  void Spare(const std::string& name);
   void Release();
   // Frees the buffers whose names start with `prefix`.
   void Drop(const std::string& prefix);
@@ -192,6 +196,18 @@ struct gg_graph {
   template <class T>
   T* Scratch(const char* name, size_t count) {
     return static_cast<T*>(ws.Get(name, count * sizeof(T)));
+  }
+  // The same, or null where the buffer does not fit: for what a call can do
+  // without.
+  template <class T>
+  T* TryScratch(const char* name, size_t count) {
+    try {
+      return Scratch<T>(name, count);
+    } catch (const gg::Failure& e) {
+      if (e.status != GG_ENOMEM) throw;
+      (void)hipGetLastError();  // the failed allocation's
+      return nullptr;
+    }
   }
   template <class T>
   T* Pinned(size_t count);

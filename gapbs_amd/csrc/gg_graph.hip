@@ -52,15 +52,35 @@ void DeviceFree(void* p, size_t bytes) {
 
 void* Workspace::Get(const std::string& name, size_t bytes) {
   Slot& s = slots[name];
+  s.spare = false;
   if (s.p && s.bytes >= bytes) return s.p;
   DeviceFree(s.p, s.bytes);
   s.p = nullptr;
   s.bytes = 0;
   // Round up so that small growth does not reallocate every call.
   const size_t rounded = (bytes + (1u << 20) - 1) & ~size_t((1u << 20) - 1);
-  s.p = DeviceAlloc(rounded);
+  try {
+    s.p = DeviceAlloc(rounded);
+  } catch (const Failure& e) {
+    bool freed = false;
+    for (auto& kv : slots) {
+      Slot& o = kv.second;
+      if (e.status != GG_ENOMEM || !o.spare || !o.p) continue;
+      DeviceFree(o.p, o.bytes);
+      o = Slot{};
+      freed = true;
+    }
+    if (!freed) throw;
+    (void)hipGetLastError();  // the failed allocation's
+    s.p = DeviceAlloc(rounded);
+  }
   s.bytes = rounded;
   return s.p;
+}
+
+void Workspace::Spare(const std::string& name) {
+  const auto it = slots.find(name);
+  if (it != slots.end()) it->second.spare = true;
 }
 
 void Workspace::Release() {

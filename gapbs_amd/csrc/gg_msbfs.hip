@@ -68,12 +68,8 @@ extern "C" int gg_bfs_batch(gg_graph* g, const int32_t* roots, int k, int alpha,
       // A pass reads out a group of roots; one root where the group's buffer
       // (4 bytes per vertex and root) does not fit beside the graph.
       int step = std::min(k, kOutRoots);
-      int32_t* d32 = nullptr;
-      try {
-        d32 = g->Scratch<int32_t>("ms.depth_out", n * step);
-      } catch (const Failure& e) {
-        if (e.status != GG_ENOMEM || step == 1) throw;
-        (void)hipGetLastError();
+      int32_t* d32 = g->TryScratch<int32_t>("ms.depth_out", n * step);
+      if (!d32) {
         step = 1;
         d32 = g->Scratch<int32_t>("ms.depth_out", n);
       }
@@ -83,6 +79,7 @@ extern "C" int gg_bfs_batch(gg_graph* g, const int32_t* roots, int k, int alpha,
         GG_HIP(hipGetLastError());
         CopyToHost(g, depths + int64_t(r) * n, d32, sizeof(int32_t) * n * (r1 - r));
       }
+      g->ws.Spare("ms.depth_out");
     }
     if (stats) {
       unsigned long long* sums = g->Scratch<unsigned long long>("ms.reach", 2);

@@ -533,10 +533,15 @@ extern "C" int gg_tc(gg_graph* g, uint64_t* count, gg_stats* stats) {
     GG_HIP(hipStreamSynchronize(st));
     const int64_t nlong = static_cast<int64_t>(h[0]), nshort = static_cast<int64_t>(h[1]), nlow = static_cast<int64_t>(h[2]);
     // Entries are counted once per edge in the lists N+: half of all.
-    const bool bits = nlow >= static_cast<int64_t>(kBitsShare * 0.5 * static_cast<double>(g->out_entries));
     // Items; then, for TcCountLong, the first 16-bit id of every vertex and the
-    // ids, readable to the end of the pair after the last one.
-    TcItem* items = g->Scratch<TcItem>("tc.items", nlong + nshort + 1 + (bits ? n + 1 + (nlow + 3) / 4 : 0));
+    // ids, readable to the end of the pair after the last one.  Where these do
+    // not fit beside the graph, TcCountHash does without.
+    const int64_t nitems = nlong + nshort + 1, nids = n + 1 + (nlow + 3) / 4;
+    TcItem* items = nullptr;
+    if (nlow >= static_cast<int64_t>(kBitsShare * 0.5 * static_cast<double>(g->out_entries)))
+      items = g->TryScratch<TcItem>("tc.items", nitems + nids);
+    const bool bits = items != nullptr;
+    if (!bits) items = g->Scratch<TcItem>("tc.items", nitems);
     TcItem* shorts = items + nlong;
     int64_t* low_off = bits ? reinterpret_cast<int64_t*>(shorts + nshort) : nullptr;
     uint16_t* low = bits ? reinterpret_cast<uint16_t*>(low_off + n + 1) : nullptr;
@@ -580,6 +585,7 @@ extern "C" int gg_tc(gg_graph* g, uint64_t* count, gg_stats* stats) {
       probes += h[2 * i + 1];
     }
     FinishTiming(g, stats, wt);
+    g->ws.Spare("tc.items");
     *count = total;
     if (stats) {
       stats->total_ms = wt.ms();
