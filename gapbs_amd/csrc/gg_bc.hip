@@ -125,6 +125,7 @@ struct DiscoverVisit {
   LdsQueue<kQueueCap>* lq;
   int32_t* queue;
   int32_t* tail;
+  int most = 0;  // queue entries at most
   __device__ __forceinline__ void Visit(const int32_t (&)[kExpandEdges], const int32_t (&)[kExpandEdges],
                                         const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
     int32_t v[kExpandEdges];
@@ -138,7 +139,7 @@ struct DiscoverVisit {
       won[k] = valid[k] && won[k] && atomicCAS(&depth[v[k]], -1, next_depth) == -1;
     LdsQueuePushMany(*lq, won, v, queue, tail);
   }
-  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, queue, tail); }
+  __device__ __forceinline__ void StepEnd(int edges) { LdsQueueMakeRoom(*lq, queue, tail, most, edges); }
 };
 
 // Claims the next level's vertices and appends them to the queue.

@@ -146,6 +146,7 @@ struct TdVisit {
   int32_t* qtail;
   int32_t level;
   unsigned long long scout = 0, reach = 0;
+  int most = 0;  // queue entries at most
 
   __device__ __forceinline__ void Visit(const int32_t (&u)[kExpandEdges], const int32_t (&)[kExpandEdges],
                                         const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
@@ -169,7 +170,7 @@ struct TdVisit {
     }
     LdsQueuePushMany(*lq, won, v, qout, qtail);
   }
-  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, qout, qtail); }
+  __device__ __forceinline__ void StepEnd(int edges) { LdsQueueMakeRoom(*lq, qout, qtail, most, edges); }
 };
 
 __device__ __forceinline__ void FlushTdCounters(const TdVisit& visit, unsigned long long examined,

@@ -164,7 +164,7 @@ struct LinkVisit {
     for (int k = 0; k < kExpandEdges; k++)
       if (valid[k]) Link(u[k], v[k], comp);
   }
-  __device__ __forceinline__ void StepEnd() {}
+  __device__ __forceinline__ void StepEnd(int) {}
 };
 
 // Final link: every vertex outside the skipped component links with its
@@ -227,7 +227,7 @@ struct HookVisit {
       }
     }
   }
-  __device__ __forceinline__ void StepEnd() {}
+  __device__ __forceinline__ void StepEnd(int) {}
 };
 
 // One wavefront store per wavefront that hooked.

@@ -18,8 +18,9 @@
 // arrays of kExpandEdges, by every lane of a wavefront together.  It loads
 // for all its edges before it acts on the first, so a wavefront has several
 // dependent-load chains in flight; padding edges (valid[k] == false) name
-// edge 0, which may be loaded but not acted on.  op.StepEnd() follows each
-// Visit, called by the whole block.  The flat range itself needs no barrier:
+// edge 0, which may be loaded but not acted on; a wavefront all of padding
+// edges does not call it.  op.StepEnd(edges) follows each step of that many
+// edges, called by the whole block.  The flat range itself needs no barrier:
 // with one edge per thread and two barriers per 256 edges, and vertices of
 // 256 to 4095 edges taken by the whole block one after the other, the
 // single-root SSSP relaxations of Kronecker 22 took 7.9 instead of 5.3 ms.
@@ -46,7 +47,6 @@ struct ChunkCut {
 };
 using FrontierCut = ChunkCut<512, kStepEdges>;
 using WholeCut = ChunkCut<4096, 4096>;
-constexpr int64_t kChunkEdges = WholeCut::kMax;
 
 struct EdgeChunk {
   int64_t beg, end;
@@ -69,7 +69,7 @@ template <class Cut, class Op>
 __device__ __forceinline__ void ExpandTile(ExpandShared& sh, int32_t u, int32_t payload,
                                            int64_t beg, int64_t end, Op& op,
                                            EdgeChunk* chunks, int32_t* nchunks) {
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, wave_first = __builtin_amdgcn_readfirstlane(tid);
   // 0. Hubs: hand their edges to the grid-wide chunk kernel, one reservation
   // per wavefront.
   if (chunks) {
@@ -110,8 +110,8 @@ __device__ __forceinline__ void ExpandTile(ExpandShared& sh, int32_t u, int32_t 
       ep[k] = sh.payload[at];
       e[k] = valid[k] ? sh.beg[at] + (j - sh.pre[at]) : 0;
     }
-    op.Visit(eu, ep, e, valid);
-    op.StepEnd();
+    if (base + wave_first < total) op.Visit(eu, ep, e, valid);
+    op.StepEnd(total - base < kStepEdges ? total - base : kStepEdges);
   }
   __syncthreads();
 }
@@ -124,6 +124,7 @@ template <class Cut, class Op>
 __device__ __forceinline__ void ExpandChunks(const EdgeChunk* __restrict__ chunks, int32_t nchunks,
                                              Op& op) {
   constexpr int kSteps = Cut::kMax / kStepEdges;
+  const int wave_first = __builtin_amdgcn_readfirstlane(threadIdx.x);
   static_assert(kSteps * kStepEdges == Cut::kMax, "chunks are whole steps");
   const int64_t items = int64_t(nchunks) * kSteps;
   int64_t it = blockIdx.x;
@@ -134,7 +135,8 @@ __device__ __forceinline__ void ExpandChunks(const EdgeChunk* __restrict__ chunk
     const int64_t first = ch.beg + (it % kSteps) * kStepEdges + threadIdx.x;
     it += gridDim.x;
     if (it < items) next = chunks[it / kSteps];
-    if (first - threadIdx.x >= ch.end) continue;  // a short last chunk
+    const int64_t left = ch.end - (first - threadIdx.x);
+    if (left <= 0) continue;  // a short last chunk
     int32_t eu[kExpandEdges], ep[kExpandEdges];
     int64_t e[kExpandEdges];
     bool valid[kExpandEdges];
@@ -145,8 +147,8 @@ __device__ __forceinline__ void ExpandChunks(const EdgeChunk* __restrict__ chunk
       ep[k] = ch.payload;
       e[k] = valid[k] ? first + k * kExpandBS : 0;
     }
-    op.Visit(eu, ep, e, valid);
-    op.StepEnd();
+    if (wave_first < left) op.Visit(eu, ep, e, valid);
+    op.StepEnd(left < kStepEdges ? static_cast<int>(left) : kStepEdges);
   }
 }
 
@@ -239,18 +241,24 @@ __device__ __forceinline__ void LdsQueueFlush(LdsQueue<CAP>& q, int32_t* gout, i
   for (int i = threadIdx.x; i < cnt; i += blockDim.x) gout[q.base + i] = q.items[i];
 }
 
-// Block-wide, between steps that push at most kStepEdges entries per queue:
-// empties the queue while the next step still fits.  A queue that overflows
+// Block-wide, after a step that pushed at most `pushed` entries; `most` is
+// what the queue can hold since it was last looked at.  Empties the queue
+// while a whole step still fits; the barriers that a look takes are left out
+// while it surely does.  A queue that overflows
 // pushes through one global counter, an atomic per wavefront, which the chip
 // takes one after another (SSSP on Kronecker 22, largest launch: 2.0 ms
 // against 0.6).
 template <int CAP>
-__device__ __forceinline__ void LdsQueueMakeRoom(LdsQueue<CAP>& q, int32_t* gout, int32_t* gtail) {
+__device__ __forceinline__ void LdsQueueMakeRoom(LdsQueue<CAP>& q, int32_t* gout, int32_t* gtail, int& most,
+                                                 int pushed) {
   static_assert(CAP >= 2 * kStepEdges, "room for a step while half full");
+  most += pushed;
+  if (most <= CAP - kStepEdges) return;  // the same in all threads
   __syncthreads();
-  const int cnt = q.count;
+  most = q.count;
   __syncthreads();  // read by all before anyone pushes again
-  if (cnt <= CAP - kStepEdges) return;
+  if (most <= CAP - kStepEdges) return;
+  most = 0;
   LdsQueueFlush(q, gout, gtail);
   __syncthreads();
   if (threadIdx.x == 0) q.count = 0;

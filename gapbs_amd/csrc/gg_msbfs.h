@@ -310,6 +310,7 @@ struct TdVisit {
   LdsQueue<kQueueCap>* lq;
   int32_t* touched;
   int32_t* touched_tail;
+  int most = 0;  // queue entries at most
   __device__ __forceinline__ void Visit(const int32_t (&v)[kExpandEdges], const int32_t (&)[kExpandEdges],
                                         const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
     int32_t w[kExpandEdges];
@@ -330,7 +331,7 @@ struct TdVisit {
                  atomicOr(reinterpret_cast<unsigned long long*>(&acc[w[k]]), bits[k]) == 0;
     LdsQueuePushMany(*lq, first, w, touched, touched_tail);
   }
-  __device__ __forceinline__ void StepEnd() { LdsQueueMakeRoom(*lq, touched, touched_tail); }
+  __device__ __forceinline__ void StepEnd(int edges) { LdsQueueMakeRoom(*lq, touched, touched_tail, most, edges); }
 };
 
 __global__ __launch_bounds__(kBS) void MsTopDown(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,

@@ -92,7 +92,7 @@ struct RlCopy {
       if (W == 2) new_dst[W * to[k] + 1] = w[k];
     }
   }
-  __device__ __forceinline__ void StepEnd() {}
+  __device__ __forceinline__ void StepEnd(int) {}
 };
 
 template <int W>

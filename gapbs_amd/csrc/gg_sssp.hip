@@ -144,6 +144,7 @@ struct RelaxVisit {
   int32_t* fresh;
   SsspCounters* c;
   unsigned long long relaxed = 0, improved = 0;
+  int most_near = 0, most_fresh = 0;  // queue entries at most
 
   __device__ __forceinline__ void Visit(const int32_t (&)[kExpandEdges], const int32_t (&du)[kExpandEdges],
                                         const int64_t (&e)[kExpandEdges], const bool (&valid)[kExpandEdges]) {
@@ -178,9 +179,9 @@ struct RelaxVisit {
     LdsQueuePushMany(*lnear, to_near, v, near, &c->near_tail);
     LdsQueuePushMany(*lfresh, to_fresh, v, fresh, &c->fresh_tail);
   }
-  __device__ __forceinline__ void StepEnd() {
-    LdsQueueMakeRoom(*lnear, near, &c->near_tail);
-    LdsQueueMakeRoom(*lfresh, fresh, &c->fresh_tail);
+  __device__ __forceinline__ void StepEnd(int edges) {
+    LdsQueueMakeRoom(*lnear, near, &c->near_tail, most_near, edges);
+    LdsQueueMakeRoom(*lfresh, fresh, &c->fresh_tail, most_fresh, edges);
   }
 };
 
