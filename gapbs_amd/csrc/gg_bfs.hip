@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kBS) void BfsTopDown(const int64_t* __restrict__ of
       end = off[u + 1];
       examined += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile<FrontierCut>(sh, u, 0, beg, end, visit, chunks, &c->nchunks);
+    ExpandTile<FrontierCut>(sh, u, 0, beg, end, visit, chunks, &c->nchunks, qn - static_cast<int>(tile));
   }
   LdsQueueFlush(lq, qout, &c->qtail);
   FlushTdCounters(visit, examined, c, s_red);

@@ -64,11 +64,13 @@ struct ExpandShared {
 // Expands one tile.  (u, payload, beg, end) describe this thread's vertex
 // (beg == end for threads without one).  Must be called by all threads of
 // the block.  chunks == nullptr disables the chunk list (the tile's edges
-// must then number below 2^31).
+// must then number below 2^31).  Threads from nv on have no vertex: the owner
+// search of a frontier's last, small tile is that much shorter (SSSP of 2^18
+// vertices with close neighbours, a few hundred in a bucket: 463 -> 453 ms).
 template <class Cut, class Op>
 __device__ __forceinline__ void ExpandTile(ExpandShared& sh, int32_t u, int32_t payload,
                                            int64_t beg, int64_t end, Op& op,
-                                           EdgeChunk* chunks, int32_t* nchunks) {
+                                           EdgeChunk* chunks, int32_t* nchunks, int nv = kExpandBS) {
   const int tid = threadIdx.x, wave_first = __builtin_amdgcn_readfirstlane(tid);
   // 0. Hubs: hand their edges to the grid-wide chunk kernel, one reservation
   // per wavefront.
@@ -93,22 +95,28 @@ __device__ __forceinline__ void ExpandTile(ExpandShared& sh, int32_t u, int32_t 
   sh.u[tid] = u;
   sh.payload[tid] = payload;
   sh.beg[tid] = beg;
+  int top = kExpandBS / 2;  // the owner search's first step
+  while (top >= nv) top >>= 1;
   __syncthreads();
   for (int base = 0; base < total; base += kStepEdges) {
     int32_t eu[kExpandEdges], ep[kExpandEdges];
     int64_t e[kExpandEdges];
     bool valid[kExpandEdges];
+    int at[kExpandEdges];  // the last vertex starting at or before the edge: the one that owns it
+#pragma unroll
+    for (int k = 0; k < kExpandEdges; k++) at[k] = 0;
+    for (int step = top; step > 0; step >>= 1) {
+#pragma unroll
+      for (int k = 0; k < kExpandEdges; k++)
+        if (sh.pre[at[k] + step] <= base + k * kExpandBS + tid) at[k] += step;
+    }
 #pragma unroll
     for (int k = 0; k < kExpandEdges; k++) {
       const int j = base + k * kExpandBS + tid;
       valid[k] = j < total;
-      int at = 0;  // the last vertex starting at or before j: the one that owns it
-#pragma unroll
-      for (int step = kExpandBS / 2; step > 0; step >>= 1)
-        if (sh.pre[at + step] <= j) at += step;
-      eu[k] = sh.u[at];
-      ep[k] = sh.payload[at];
-      e[k] = valid[k] ? sh.beg[at] + (j - sh.pre[at]) : 0;
+      eu[k] = sh.u[at[k]];
+      ep[k] = sh.payload[at[k]];
+      e[k] = valid[k] ? sh.beg[at[k]] + (j - sh.pre[at[k]]) : 0;
     }
     if (base + wave_first < total) op.Visit(eu, ep, e, valid);
     op.StepEnd(total - base < kStepEdges ? total - base : kStepEdges);

@@ -222,7 +222,9 @@ __device__ __forceinline__ void PushPending(RelaxCtx& c, const PendingPush& p) {
 // them are loaded, and a step's queue stamps are looked at one step later.
 // Kronecker 19, 16 roots, the two kernels: 7.3 and 4.1 ms with each improving
 // edge's two atomic round trips in a row, 6.2 and 3.5 with a step's atomics
-// issued together, 5.8 and 3.2 with the ids ahead, 5.3 and 2.7 as here.
+// issued together, 5.8 and 3.2 with the ids ahead, 5.3 and 2.7 as here.  The
+// steps in flight take registers: SbRelax has 99, four wavefronts a SIMD, where
+// six fitted before the pipelining.
 __device__ __forceinline__ void RelaxRange(RelaxCtx& c, const Group& g, int64_t b, int64_t e, bool active,
                                            int32_t du) {
   if (b >= e) return;
