@@ -24,8 +24,8 @@ def _fits(monkeypatch, call, mb):
         monkeypatch.delenv("GAPGPU_MEM_CAP_BYTES")
 
 
-def _least(monkeypatch, call, start):
-    for mb in range(start, start + 1024):
+def _least(monkeypatch, call, taken):
+    for mb in range(taken, taken + 1024):
         ok, result = _fits(monkeypatch, call, mb)
         if ok:
             return mb, result
@@ -33,9 +33,17 @@ def _least(monkeypatch, call, start):
 
 
 def _allocated(monkeypatch):
-    """The MB already taken, rounded up: the least at which two offsets more fit."""
+    """The MB already taken (other handles' too), rounded up: the least at
+    which two offsets more fit."""
     two = Graph.from_edges([0], [1])
-    return _least(monkeypatch, lambda: gpu.DeviceGraph(two).free(), 1)[0]
+    low, high = 0, 1 << 19  # does not fit, fits
+    while high - low > 1:
+        mid = (low + high) // 2
+        if _fits(monkeypatch, lambda: gpu.DeviceGraph(two).free(), mid)[0]:
+            high = mid
+        else:
+            low = mid
+    return high
 
 
 # What a call needed with no optional buffer, in MB beside the graph
