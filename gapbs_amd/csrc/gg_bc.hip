@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kBS) void BcDiscover(const int64_t* __restrict__ of
       end = off[u + 1];
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile<FrontierCut>(sh, 0, 0, beg, end, visit, chunks, &c->nchunks);
+    ExpandTile<FrontierCut>(sh, 0, 0, beg, end, visit, chunks, &c->nchunks, FrontierCut::MinFor(qn));
   }
   LdsQueueFlush(lq, queue, &c->tail);
   ex = BlockSum<kBS>(ex, s_red);

@@ -208,7 +208,8 @@ __global__ __launch_bounds__(kBS) void BfsTopDown(const int64_t* __restrict__ of
       end = off[u + 1];
       examined += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile<FrontierCut>(sh, u, 0, beg, end, visit, chunks, &c->nchunks, qn - static_cast<int>(tile));
+    ExpandTile<FrontierCut>(sh, u, 0, beg, end, visit, chunks, &c->nchunks, FrontierCut::MinFor(qn),
+                            qn - static_cast<int>(tile));
   }
   LdsQueueFlush(lq, qout, &c->qtail);
   FlushTdCounters(visit, examined, c, s_red);
@@ -499,14 +500,15 @@ BfsRun RunDobfs(gg_graph* g, int32_t source, int alpha, int beta, int32_t* depth
       scout = 1;
     } else {
       edges_to_check -= scout;
-      const bool hubs = use_chunks && frontier_deg >= FrontierCut::kMin;
+      const int chunk_min = FrontierCut::MinFor(qsize);
+      const bool hubs = use_chunks && frontier_deg >= chunk_min;
       const int idx = Run(g, "bfs_top_down", 16.0 * qsize, BfsTopDown,
                           dim3(GridFor(qsize, kBS, g->cu_count * 8)), blk, g->out_off, g->out_dst,
                           parent, depth, qin, static_cast<int32_t>(qsize), qout, dc, level,
                           hubs ? chunks : static_cast<EdgeChunk*>(nullptr));
       launches++;
       if (hubs) {
-        const dim3 grid_c(GridFor(frontier_deg / FrontierCut::kMin + 1, 1, g->cu_count * 8));
+        const dim3 grid_c(GridFor(frontier_deg / chunk_min + 1, 1, g->cu_count * 8));
         Run(g, "bfs_top_down_chunks", 0, BfsTopDownChunks, grid_c, blk, g->out_off, g->out_dst,
             parent, depth, qout, dc, level, static_cast<const EdgeChunk*>(chunks));
         launches++;

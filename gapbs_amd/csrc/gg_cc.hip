@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kBS) void CcFinalLink(const int64_t* __restrict__ o
       beg = off[u] + start < end ? off[u] + start : end;
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, WholeCut::kMin);
   }
   ex = BlockSum<kBS>(ex, s_red);
   if (threadIdx.x == 0 && ex) atomicAdd(&examined[blockIdx.x & 63], ex);
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kBS) void SvHook(const int64_t* __restrict__ off, c
   for (int64_t tile = int64_t(blockIdx.x) * kBS; tile < n; tile += int64_t(gridDim.x) * kBS) {
     const int64_t u = tile + threadIdx.x;
     const int64_t beg = u < n ? off[u] : 0, end = u < n ? off[u + 1] : 0;
-    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, WholeCut::kMin);
   }
   NoteChange(hooked, change);
 }

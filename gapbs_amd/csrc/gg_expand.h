@@ -3,14 +3,16 @@
 // One 256-thread block takes a tile of 256 frontier vertices and visits all
 // their edges so that a hub with millions of edges and a vertex with three
 // cost about the same per edge:
-//   0. vertices with >= kMin edges are cut into chunks of at most kMax edges
-//      appended to a chunk list, which a second kernel (ExpandChunks) spreads
-//      over the whole grid.  Frontiers use FrontierCut: neighbouring frontier
-//      entries of a degree-ordered graph have similar degrees, so with a
-//      higher kMin one tile can hold 256 vertices of thousands of edges and
-//      outlast the rest of its launch (Kronecker 22, SSSP: 1.7 ms at 4096,
-//      0.5 ms).  Passes over all vertices
-//      use WholeCut: fewer chunks;
+//   0. vertices with >= MinFor edges are cut into chunks of at most kMax
+//      edges appended to a chunk list, which a second kernel (ExpandChunks)
+//      spreads over the whole grid.  Frontiers use FrontierCut: neighbouring
+//      frontier entries of a degree-ordered graph have similar degrees, so
+//      with a higher cut-off one tile can hold 256 vertices of thousands of
+//      edges and outlast the rest of its launch (Kronecker 22, SSSP: 1.7 ms at
+//      4096, 0.5 ms at 512); of a small frontier, whose tiles leave most of
+//      the chip idle, shorter lists are spread too (40 k vertices of 400 close
+//      neighbours: BFS 33 ms at 512, 5.3 at 256, SSSP 55 and 9.3).  Passes over
+//      all vertices use WholeCut: fewer chunks;
 //   1. the rest form one flat range of edges (block prefix sum over their
 //      edge counts); each thread takes kExpandEdges of them per step, one
 //      per kExpandBS, and finds an edge's vertex by binary search in LDS.
@@ -25,6 +27,8 @@
 // 256 to 4095 edges taken by the whole block one after the other, the
 // single-root SSSP relaxations of Kronecker 22 took 7.9 instead of 5.3 ms.
 #pragma once
+
+#include <algorithm>
 
 #include "gg_common.h"
 
@@ -45,7 +49,15 @@ struct ChunkCut {
     return entries / kMax + big + 2;
   }
 };
-using FrontierCut = ChunkCut<512, kStepEdges>;
+// The cut-off follows the frontier's size: kMin in one of few vertices.
+struct FrontierCut {
+  static constexpr int kMin = 256, kMinLarge = 512, kMax = kStepEdges;
+  static constexpr int64_t kFew = 4096;
+  __host__ __device__ static int MinFor(int64_t vertices) { return vertices <= kFew ? kMin : kMinLarge; }
+  static int64_t Bound(int64_t n, int64_t entries) {
+    return ChunkCut<kMinLarge, kMax>::Bound(n, entries) + std::min(kFew, entries / kMin);
+  }
+};
 using WholeCut = ChunkCut<4096, 4096>;
 
 struct EdgeChunk {
@@ -63,19 +75,21 @@ struct ExpandShared {
 
 // Expands one tile.  (u, payload, beg, end) describe this thread's vertex
 // (beg == end for threads without one).  Must be called by all threads of
-// the block.  chunks == nullptr disables the chunk list (the tile's edges
-// must then number below 2^31).  Threads from nv on have no vertex: the owner
+// the block.  Vertices of chunk_min edges or more (the same in every tile) go
+// to the chunk list; chunks == nullptr disables it (the tile's edges must then
+// number below 2^31).  Threads from nv on have no vertex: the owner
 // search of a frontier's last, small tile is that much shorter (SSSP of 2^18
 // vertices with close neighbours, a few hundred in a bucket: 463 -> 453 ms).
 template <class Cut, class Op>
 __device__ __forceinline__ void ExpandTile(ExpandShared& sh, int32_t u, int32_t payload,
                                            int64_t beg, int64_t end, Op& op,
-                                           EdgeChunk* chunks, int32_t* nchunks, int nv = kExpandBS) {
+                                           EdgeChunk* chunks, int32_t* nchunks, int chunk_min,
+                                           int nv = kExpandBS) {
   const int tid = threadIdx.x, wave_first = __builtin_amdgcn_readfirstlane(tid);
   // 0. Hubs: hand their edges to the grid-wide chunk kernel, one reservation
   // per wavefront.
   if (chunks) {
-    const int nc = end - beg >= Cut::kMin ? static_cast<int>((end - beg + Cut::kMax - 1) / Cut::kMax) : 0;
+    const int nc = end - beg >= chunk_min ? static_cast<int>((end - beg + Cut::kMax - 1) / Cut::kMax) : 0;
     if (__ballot(nc > 0)) {
       const int upto = WaveInclusiveScan(nc);
       int base = 0;

@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kBS) void MsTopDown(const int64_t* __restrict__ off
       end = off[v + 1];
       ex += static_cast<unsigned long long>(end - beg);
     }
-    ExpandTile<FrontierCut>(sh, v, 0, beg, end, visit, chunks, &c->nchunks);
+    ExpandTile<FrontierCut>(sh, v, 0, beg, end, visit, chunks, &c->nchunks, FrontierCut::MinFor(na));
   }
   LdsQueueFlush(lq, touched, &c->touched_tail);
   ex = BlockSum<kBS>(ex, s_red);

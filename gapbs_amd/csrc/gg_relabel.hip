@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kBS) void RlCopyRows(const int64_t* __restrict__ ol
       b = old_off[u];
       e = old_off[u + 1];
     }
-    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks, WholeCut::kMin);
   }
 }
 

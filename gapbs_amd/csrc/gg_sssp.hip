@@ -220,7 +220,8 @@ __global__ __launch_bounds__(kBS) void SsspRelax(const int64_t* __restrict__ off
       beg = off[u];
       end = off[u + 1];
     }
-    ExpandTile<FrontierCut>(sh, u, du, beg, end, rv, chunks, &c->nchunks, fn - static_cast<int>(tile));
+    ExpandTile<FrontierCut>(sh, u, du, beg, end, rv, chunks, &c->nchunks, FrontierCut::MinFor(fn),
+                            fn - static_cast<int>(tile));
   }
   FlushRelax(rv, c, s_red);
 }

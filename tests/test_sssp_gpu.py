@@ -134,3 +134,25 @@ def test_sssp_light_and_heavy_edges(delta, ordered):
     dg = gpu.DeviceGraph(g, order_by_degree=ordered)
     for r in (0, 1, 77):
         assert np.array_equal(gpu.sssp(dg, r, delta).dist, oracle.dijkstra(g, r))
+
+
+@pytest.mark.parametrize("width", [1, 300, 4096, 4097])
+def test_lists_of_small_and_large_frontiers(width):
+    # Frontiers of up to 4096 vertices spread lists of 256 entries, larger ones
+    # lists of 512: lists around both, of single and batched searches and paths.
+    print(f"[sssp] frontier of {width}", flush=True)
+    rng = np.random.default_rng(width)
+    lens = np.array([255, 256, 257, 400, 511, 512, 513, 1024, 1025] * 4)[:width]
+    mids = np.arange(1, 1 + width)
+    first, n = 1 + width, 1 + width + 6000
+    u = np.concatenate([np.zeros(width, int), np.repeat(mids[:len(lens)], lens)])
+    v = np.concatenate([mids] + [rng.choice(np.arange(first, n), d, replace=False) for d in lens])
+    g = Graph.from_edges(u, v, rng.integers(1, 256, len(u)), symmetrize=False)
+    dg = gpu.DeviceGraph(g)
+    want = oracle.dijkstra(g, 0)
+    for delta in (1, 64, 1024):
+        assert np.array_equal(gpu.sssp(dg, 0, delta).dist, want)
+    plain = g.strip_weights()
+    dp = gpu.DeviceGraph(plain)
+    assert np.array_equal(gpu.bfs(dp, 0, alpha=1).depth, oracle.bfs_depth(plain, 0))
+    assert np.array_equal(gpu.bfs_batch(dp, [0, 1], alpha=1).depths[0], oracle.bfs_depth(plain, 0))
