@@ -425,11 +425,14 @@ __global__ __launch_bounds__((P + 1) * kWave, P <= kHubSmall ? 7 : 1) void MbDel
       }
       __syncthreads();  // the consumer's last fold
     } else {
-      // The fold is the block's longest chain, so it issues ahead of the
-      // producers on its SIMD, and it takes every slot without a test (64
+      // The fold is a wide block's longest chain, so there it issues ahead of
+      // the producers on its SIMD, and it takes every slot without a test (64
       // roots, wide blocks, all levels: Kronecker 19 5.30 -> 4.25 ms,
-      // Kronecker 22 37.2 -> 32.5; the priority alone 4.58 and 31.4).
-      __builtin_amdgcn_s_setprio(3);
+      // Kronecker 22 37.2 -> 32.5; the priority alone 4.58 and 31.4).  Small
+      // blocks have other blocks to hide it behind (with the priority
+      // Kronecker 26 took 0.654 instead of 0.650 s, Kronecker 22, 16 roots,
+      // 22.9 instead of 22.1 ms).
+      if (P > kHubSmall) __builtin_amdgcn_s_setprio(3);
       T acc = T(0);
       auto fold = [&](int64_t k) {
         const double* in = terms[k & 1];
