@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kBS) void RlCopyRows(const int64_t* __restrict__ ol
                                                   const int32_t* __restrict__ old_dst,
                                                   const int64_t* __restrict__ new_off,
                                                   const int32_t* __restrict__ new_id, int32_t* new_dst, int64_t n,
-                                                  EdgeChunk* chunks, int32_t* nchunks) {
+                                                  EdgeChunk* chunks, int32_t* nchunks, int chunk_min) {
   __shared__ ExpandShared sh;
   RlCopy<W> op{old_off, old_dst, new_off, new_id, new_dst};
   for (int64_t tile = int64_t(blockIdx.x) * kBS; tile < n; tile += int64_t(gridDim.x) * kBS) {
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kBS) void RlCopyRows(const int64_t* __restrict__ ol
       b = old_off[u];
       e = old_off[u + 1];
     }
-    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks, WholeCut::kMin);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, b, e, op, chunks, nchunks, chunk_min);
   }
 }
 
@@ -272,12 +272,13 @@ void CopyLists(gg_graph* g, const int64_t* new_off, const int32_t* new_id, int32
   const int64_t n = g->n, entries = g->out_entries;
   const dim3 blk(kBS);
   int32_t* nchunks = g->Scratch<int32_t>("rl.nchunks", 1);
-  const bool use_chunks = g->max_degree >= WholeCut::kMin;
-  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("rl.chunks", WholeCut::Bound(n, entries)) : nullptr;
+  const int chunk_min = WholeCut::MinFor(n, entries);
+  const bool use_chunks = g->max_degree >= chunk_min;
+  EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("rl.chunks", WholeCut::BoundFor(n, entries)) : nullptr;
   Run(g, "relabel_clear", 0, RlZero, dim3(1), dim3(64), nchunks);
   Run(g, "relabel_copy", 8.0 * n + (8.0 * W + 4.0) * entries, RlCopyRows<W>, dim3(GridFor(n, kBS, g->cu_count * 8)),
       blk, static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), new_off, new_id,
-      new_dst, n, use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), nchunks);
+      new_dst, n, use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), nchunks, chunk_min);
   if (use_chunks)
     Run(g, "relabel_copy", 0, RlCopyChunks<W>, dim3(g->cu_count * 4), blk, static_cast<const int64_t*>(g->out_off),
         static_cast<const int32_t*>(g->out_dst), new_off, new_id, new_dst, static_cast<const EdgeChunk*>(chunks),

@@ -1,8 +1,8 @@
 """Device relabelling by degree (gg_relabel_by_degree) against the host
 restatement of BuilderBase::RelabelByDegree (src/builder.h:367-402): the
 offsets and destinations must be byte-identical, on graphs whose rows
-exercise every sort tier (<= 32 entries: one thread; <= 2048: a block
-bitonic sort; longer: the (row, value) radix sort) and multi-tile radix
+exercise every sort tier (<= 32 entries: one thread; <= 2048: a wavefront
+in registers; longer: the (row, value) radix sort) and multi-tile radix
 passes; and TC on the device-relabelled graph must give the reference's
 count (its Hybrid path)."""
 
@@ -88,3 +88,18 @@ def test_relabel_sort_tiles(n):
     u = np.concatenate([i - 1, np.zeros(len(hubs), np.int32), [0] * (n == 1)]).astype(np.int32)
     v = np.concatenate([i, hubs, [0] * (n == 1)]).astype(np.int32)
     check(Graph.from_edges(u, v))
+
+
+@pytest.mark.parametrize("mids", [120, 140])
+def test_dense_graph_lists(mids):
+    # 2000 vertices of about 126 and 146 entries on average, below and above
+    # the density from which lists of 256 entries are spread over the grid.
+    print(f"[relabel] dense, {mids}", flush=True)
+    rng = np.random.default_rng(mids)
+    n = 2000
+    deg = np.full(n, mids // 2)
+    deg[:7] = [255, 256, 257, 511, 1023, 1024, 1500]
+    u = np.repeat(np.arange(n), deg)
+    v = np.concatenate([rng.choice(np.delete(np.arange(n), i), d, replace=False) for i, d in enumerate(deg)])
+    g = Graph.from_edges(u, v)
+    check(g)
