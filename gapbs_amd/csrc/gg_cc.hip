@@ -118,10 +118,12 @@ __global__ __launch_bounds__(kBS) void CcHook(const int64_t* __restrict__ off, c
 // second the others.  The trees that most vertices belong to are then merged
 // by few threads, and the rest find their labels joined instead of queueing
 // compare-and-swaps on the same roots (Kronecker 22: 325 us in one launch,
-// 156 us in two).  Graphs of less than kSampleVertices vertices, whose rounds
-// are launches rather than work, are linked in one (`part` kLinkAll).
+// 156 us in two; the whole call on 32 k vertices of 600 neighbours: 270 us and
+// 143).  Graphs of less than kSampleVertices vertices, whose rounds are launches
+// rather than work, are linked in one (`part` kLinkAll; 1024 vertices: 87 us, 115
+// in two).
 constexpr int kLinkSample = 64;
-constexpr int64_t kSampleVertices = 1 << 16;
+constexpr int64_t kSampleVertices = 1 << 13;
 enum LinkPart { kLinkSampled, kLinkOthers, kLinkAll };
 __global__ __launch_bounds__(kBS) void CcLinkRound(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
                                                    int32_t* comp, int64_t n, int r, bool first, LinkPart part) {
