@@ -237,16 +237,20 @@ __device__ __forceinline__ void NoteChange(bool hooked, int* change) {
   if (__ballot(hooked) && LaneId() == 0) *change = 1;
 }
 
+// Up to this many vertices (32 tiles) dense graphs' lists are spread over the
+// grid: 4096 vertices of 2000 entries 1.53 ms without, 0.22
+// with.
+constexpr int64_t kFewVertices = 8192;
 __global__ __launch_bounds__(kBS) void SvHook(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
                                               int32_t* comp, int64_t n, EdgeChunk* chunks, int32_t* nchunks,
-                                              int* change) {
+                                              int chunk_min, int* change) {
   __shared__ ExpandShared sh;
   bool hooked = false;
   HookVisit visit{dst, comp, &hooked};
   for (int64_t tile = int64_t(blockIdx.x) * kBS; tile < n; tile += int64_t(gridDim.x) * kBS) {
     const int64_t u = tile + threadIdx.x;
     const int64_t beg = u < n ? off[u] : 0, end = u < n ? off[u + 1] : 0;
-    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, WholeCut::kMin);
+    ExpandTile<WholeCut>(sh, static_cast<int32_t>(u), 0, beg, end, visit, chunks, nchunks, chunk_min);
   }
   NoteChange(hooked, change);
 }
@@ -520,8 +524,9 @@ extern "C" int gg_cc_sv(gg_graph* g, int32_t* comp_out, gg_stats* stats) {
     int32_t* comp = g->Scratch<int32_t>("cc.comp", n);
     int32_t* nchunks = g->Scratch<int32_t>("cc.nchunks", 2);
     int* change = g->Scratch<int>("sv.change", 1);
-    const bool use_chunks = g->max_degree >= WholeCut::kMin;
-    EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("cc.chunks", WholeCut::Bound(n, g->out_entries)) : nullptr;
+    const int chunk_min = n <= kFewVertices ? WholeCut::MinFor(n, g->out_entries) : WholeCut::kMin;
+    const bool use_chunks = g->max_degree >= chunk_min;
+    EdgeChunk* chunks = use_chunks ? g->Scratch<EdgeChunk>("cc.chunks", WholeCut::BoundFor(n, g->out_entries)) : nullptr;
     int* h_change = g->Pinned<int>(1);
     int64_t iterations = 0, launches = 0;
     BeginTiming(g);
@@ -533,7 +538,7 @@ extern "C" int gg_cc_sv(gg_graph* g, int32_t* comp_out, gg_stats* stats) {
       Run(g, "sv_clear", 0, SvClear, dim3(1), dim3(64), change, nchunks);
       Run(g, "sv_hook", 16 * N + 4.0 * g->out_entries, SvHook, dim3(GridFor(n, kBS, g->cu_count * 8)), blk,
           static_cast<const int64_t*>(g->out_off), static_cast<const int32_t*>(g->out_dst), comp, n,
-          use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), nchunks, change);
+          use_chunks ? chunks : static_cast<EdgeChunk*>(nullptr), nchunks, chunk_min, change);
       if (use_chunks)
         Run(g, "sv_hook_chunks", 0, SvHookChunks, dim3(g->cu_count * 4), blk,
             static_cast<const int32_t*>(g->out_dst), comp, static_cast<const EdgeChunk*>(chunks),

@@ -93,7 +93,8 @@ def test_relabel_sort_tiles(n):
 @pytest.mark.parametrize("mids", [120, 140])
 def test_dense_graph_lists(mids):
     # 2000 vertices of about 126 and 146 entries on average, below and above
-    # the density from which lists of 256 entries are spread over the grid.
+    # the density from which lists of 256 entries are spread over the grid in
+    # relabelling and Shiloach-Vishkin (the sampled components leave them whole).
     print(f"[relabel] dense, {mids}", flush=True)
     rng = np.random.default_rng(mids)
     n = 2000
@@ -103,3 +104,6 @@ def test_dense_graph_lists(mids):
     v = np.concatenate([rng.choice(np.delete(np.arange(n), i), d, replace=False) for i, d in enumerate(deg)])
     g = Graph.from_edges(u, v)
     check(g)
+    for rounds in (0, 2):
+        assert np.array_equal(gpu.cc(gpu.DeviceGraph(g), rounds).comp, np.zeros(n, np.int32))
+    assert np.array_equal(gpu.cc_sv(gpu.DeviceGraph(g)).comp, np.zeros(n, np.int32))
