@@ -120,8 +120,8 @@ __global__ __launch_bounds__(kBS) void CcHook(const int64_t* __restrict__ off, c
 // compare-and-swaps on the same roots (Kronecker 22: 325 us in one launch,
 // 156 us in two; the whole call on 32 k vertices of 600 neighbours: 270 us and
 // 143).  Graphs of less than kSampleVertices vertices, whose rounds are launches
-// rather than work, are linked in one (`part` kLinkAll; 1024 vertices: 87 us, 115
-// in two).
+// rather than work, are linked in one (`part` kLinkAll): Kronecker 10, two
+// rounds, 97 to 103 us, 98 to 107 in two.
 constexpr int kLinkSample = 64;
 constexpr int64_t kSampleVertices = 1 << 13;
 enum LinkPart { kLinkSampled, kLinkOthers, kLinkAll };
@@ -238,8 +238,7 @@ __device__ __forceinline__ void NoteChange(bool hooked, int* change) {
 }
 
 // Up to this many vertices (32 tiles) dense graphs' lists are spread over the
-// grid: 4096 vertices of 2000 entries 1.53 ms without, 0.22
-// with.
+// grid: 4096 vertices of 2000 entries 1.53 ms without, 0.20 with.
 constexpr int64_t kFewVertices = 8192;
 __global__ __launch_bounds__(kBS) void SvHook(const int64_t* __restrict__ off, const int32_t* __restrict__ dst,
                                               int32_t* comp, int64_t n, EdgeChunk* chunks, int32_t* nchunks,
